@@ -84,10 +84,10 @@ int nmi_linear_fp8_w8a16(const void* x_bf16, int64_t ldx, const void* w_e4m3, in
                          void* stream);
 
 /*
- * As nmi_linear_fp8_w8a16, with a caller-owned device workspace that lets the short-prompt
- * GEMM (17 <= M < 512) split K between workgroups.  For M >= 512 the prefill GEMM needs none:
- * where its 256 x 256 tiles would cover at most half of the CUs (e.g. N = 3136 at M = 2048) it
- * takes 128 x 256 tiles instead.  Its stream-K form (the k tiles of a few large tiles split
+ * As nmi_linear_fp8_w8a16, with a caller-owned device workspace that lets the GEMM (M >= 17)
+ * split K between workgroups where its tiles alone would leave CUs idle: float32 partials in the
+ * workspace, added in a fixed order by a second kernel (from M = 512 for one matrix of K >= 4096,
+ * e.g. N = 3136, K = 12544 at M = 777).  The stream-K form (the k tiles of a few large tiles split
  * between all CUs: fp32 partial tiles and per-workgroup flags in the workspace) runs only under
  * the tuning knob gemm.sk = 1 (or gemm.bm = 256), and nmi_linear_workspace_bytes sizes the
  * workspace for it only then.
@@ -197,10 +197,14 @@ int nmi_gemv_chain_destroy(nmi_gemv_chain* chain);
  * split (s4.kg > 1): 64 KiB of arrival counters and the fp32 partials, s4.kg x M x total_n x 4
  * bytes (fewer K groups when K has fewer windows).  For 17 <= M < 512 (the short-prompt GEMM) a
  * 64 KiB region it leaves alone, then the fp32 partials of its K split (0 when the schedule does
- * not split K).  For M >= 512 about 64 MiB: a 64 KiB flag region and one 256 x 256 fp32 partial
- * tile per CU.  Every kernel leaves the first 64 KiB as it found it (zero at rest), so one
- * zero-filled workspace serves every M in turn. */
+ * not split K).  For M >= 512 likewise a 64 KiB flag region and the fp32 partial tiles of one
+ * matrix's K split (at most one 256 x 256 tile per CU, 64 MiB; 0 when it is not split).  Every
+ * kernel leaves the first 64 KiB as it found it (zero at rest), so one zero-filled workspace
+ * serves every M in turn. */
 size_t nmi_linear_workspace_bytes(int M, int64_t total_n, int K);
+/* 0 where a workspace for M rows may hold anything (the K split of M >= 512 writes its partials
+ * before it reads them), 1 where it must start zero-filled. */
+int nmi_linear_workspace_needs_zero(int M);
 
 /*
  * Prefill GEMM y[M,N] = bf16_rne((x[M,K] . e4m3(W[N,K])^T) * s[n]) on bf16 MFMA, any M >= 1.
@@ -437,8 +441,8 @@ int nmi_mamba_forward_fp8(const void* input_bf16, const float* norm_w, const voi
  * the M = 1 stream kernel, "gemv.wgs": its workgroups per CU (1, 2), "gemv.grid": its exact
  * workgroup count, "gemv.balance": 2 keeps the plain grid instead of one whose waves get equal
  * row counts, "sdpa.chunk": cache positions per workgroup of the attention decode, "gemm.tile"
- * (1, 2: short-prompt kernel, 20, 21, 24), "gemm.sk", "gemm.splits": workgroups splitting K in
- * the short-prompt GEMM (1: none), "gemm.short": f + 1 forces its tile form f (0..7),
+ * (1, 2: short-prompt kernel, 20, 21, 24), "gemm.sk", "gemm.splits": workgroups splitting K
+ * (1: none), "gemm.bm": tile rows from M = 512 (128, 192, 256), "gemm.short": f + 1 forces its tile form f (0..7),
  * "gemm.sk_cap": workgroups per tile of the stream-K form at most (0: 2, -1: one workgroup per
  * CU), "skinny.path" (2: the skinny kernels take M = 2 too, 3: the GEMV kernel takes M <= 4),
  * "m1.path" (3: M = 1 on the 4x4x4 skinny kernel), "s4.ks", "s4.t", "s4.u",

@@ -70,27 +70,28 @@ AttnLayout attn_layout(int hidden, int n_heads, int n_kv, int S_cache) {
     return L;
 }
 
-// Prefill block workspace: the GEMMs' stream-K region (S >= 512), normed [S, hidden], q
-// [S, H*128], k and v [S, H_KV*128], o [S, H*128].
+// Prefill block workspace: the GEMMs' region, normed [S, hidden], q [S, H*128], k and v
+// [S, H_KV*128], o [S, H*128].
 struct FwdLayout {
     size_t gemm, normed, q, k, v, o, total;
 };
 
-// The GEMMs' region (the short-prompt kernel's K-split partials below M = 512; from 512 the
-// stream-K flags and partials where that form is forced by tuning knob, else nothing):
-// the largest of the q, k, v (launched one by one on the GEMM path) and o needs.
-size_t gemm_region(int M, int hidden, int QD, int KD) {
+// The GEMMs' region (the K splits' partials, or the stream-K flags and partials where that form
+// is forced by tuning knob): the largest of the q, k, v (launched one by one below M = 512) and o
+// needs.  split = false: without the K split of M >= 512.
+size_t gemm_region(int M, int hidden, int QD, int KD, bool split) {
     if (choose_path(M) != Path::Gemm) return 0;
-    const size_t qkv = std::max(linear_workspace_bytes(M, (int64_t)QD + 2 * (int64_t)KD, hidden),
-                                std::max(linear_workspace_bytes(M, QD, hidden), linear_workspace_bytes(M, KD, hidden)));
-    return round256(std::max(qkv, linear_workspace_bytes(M, hidden, QD)));
+    const auto need = split ? linear_workspace_bytes : linear_workspace_bytes_unsplit;
+    const size_t qkv = std::max(need(M, (int64_t)QD + 2 * (int64_t)KD, hidden),
+                                std::max(need(M, QD, hidden), need(M, KD, hidden)));
+    return round256(std::max(qkv, need(M, hidden, QD)));
 }
 
-FwdLayout fwd_layout(int S, int hidden, int n_heads, int n_kv) {
+FwdLayout fwd_layout(int S, int hidden, int n_heads, int n_kv, bool split = true) {
     FwdLayout L{};
     const size_t QD = (size_t)n_heads * kSdpaHead, KD = (size_t)n_kv * kSdpaHead;
     L.gemm = 0;
-    L.normed = L.gemm + gemm_region(S, hidden, (int)QD, (int)KD);
+    L.normed = L.gemm + gemm_region(S, hidden, (int)QD, (int)KD, split);
     L.q = L.normed + round256((size_t)S * hidden * 2);
     L.k = L.q + round256((size_t)S * QD * 2);
     L.v = L.k + round256((size_t)S * KD * 2);
@@ -174,10 +175,11 @@ int nmi_attn_forward_fp8(const void* input_bf16, const float* norm_w, const void
     if (!aligned(q_scale, 4) || !aligned(k_scale, 4) || !aligned(v_scale, 4) || !aligned(o_scale, 4) ||
         !aligned(out_bf16, 2))
         return fail(NMI_ERR_ALIGNMENT, "nmi_attn_forward_fp8: misaligned scale or output");
-    const FwdLayout lay = fwd_layout(S, hidden, n_heads, n_kv_heads);
+    FwdLayout lay = fwd_layout(S, hidden, n_heads, n_kv_heads);
     if (workspace) {
         if (!aligned(workspace, 256))
             return fail(NMI_ERR_ALIGNMENT, "nmi_attn_forward_fp8: workspace must be 256-byte aligned");
+        if (workspace_bytes < lay.total) lay = fwd_layout(S, hidden, n_heads, n_kv_heads, false);
         if (workspace_bytes < lay.total) {
             set_last_error("%s: workspace of %zu bytes, %zu needed", fn, workspace_bytes, lay.total);
             return NMI_ERR_WORKSPACE;

@@ -45,16 +45,16 @@ bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) %
 
 size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// Workspace layout: the prefill GEMM's stream-K region (M >= 512: flags, then partial tiles),
-// act [M, inter] bf16, then normed [M, hidden] bf16 when the RMSNorm is not fused into the up
+// Workspace layout: the GEMMs' region (M >= 17: flags, then the K split's partials), act [M, inter] bf16, then normed [M, hidden] bf16 when the RMSNorm is not fused into the up
 // projection.
 bool norm_fused(int M, int hidden) { return gemv_fuses_norm(M, hidden); }
 
-// split = false leaves the short-prompt GEMMs unsplit (no partial region): the allocation-free
-// form, whose buffers must fit a fixed array
+// split = false leaves the GEMMs unsplit (no partial region): the allocation-free form, whose
+// buffers must fit a fixed array, and from M = 512 a caller's workspace without room for it
 size_t gemm_region(int M, int hidden, int inter, bool split) {
     if (choose_path(M) != Path::Gemm || (!split && !gemm_workspace_has_flags(M))) return 0;
-    return round256(std::max(linear_workspace_bytes(M, inter, hidden), linear_workspace_bytes(M, hidden, inter)));
+    const auto need = split ? linear_workspace_bytes : linear_workspace_bytes_unsplit;
+    return round256(std::max(need(M, inter, hidden), need(M, hidden, inter)));
 }
 
 size_t mlp_bytes(int M, int hidden, int inter, bool split) {
@@ -121,8 +121,10 @@ int mlp_forward_fp8(const void* input_bf16, const float* norm_w, const void* up_
     if (workspace) {
         if (!aligned(workspace, 16))
             return fail2(NMI_ERR_ALIGNMENT, fn, "workspace must be 16-byte aligned");
-        if (workspace_bytes < need) {
-            set_last_error("%s: workspace of %zu bytes, %zu needed", fn, workspace_bytes, need);
+        if (workspace_bytes < need && M >= 512) split = false;      // room enough without the K split?
+        const size_t least = split ? need : mlp_bytes(M, hidden, inter, false);
+        if (workspace_bytes < least) {
+            set_last_error("%s: workspace of %zu bytes, %zu needed", fn, workspace_bytes, least);
             return NMI_ERR_WORKSPACE;
         }
     } else {

@@ -143,8 +143,13 @@ size_t linear_workspace_bytes(int M, int64_t total_n, int K) {
     const int t = tuning().gemm_tile;
     if (M > 16 && M < 512)                            // the short-prompt kernel's K-split partials
         return (t == 0 || t == 2) ? gemm_short_workspace_bytes(M, (int)std::min<int64_t>(total_n, 1 << 30), K) : 0;
-    if (M > 16) return gemm_workspace_bytes(M);       // stream-K flags and partials of the GEMM
+    if (M > 16)                                       // the GEMM's stream-K flags and partials, or its K split's
+        return std::max(gemm_workspace_bytes(M), (t == 0 || t == 24) ? gemm_split_workspace_bytes(M, total_n, K) : 0);
     return 0;                                         // the GEMV and skinny kernels use none
+}
+
+size_t linear_workspace_bytes_unsplit(int M, int64_t total_n, int K) {
+    return M < 512 ? linear_workspace_bytes(M, total_n, K) : gemm_workspace_bytes(M);
 }
 
 bool gemm_workspace_has_flags(int M) { return M >= 512 && choose_path(M) == Path::Gemm && gemm_workspace_bytes(M) > 0; }
@@ -446,6 +451,8 @@ int nmi_gemv_chain_destroy(nmi_gemv_chain* chain) {
     delete chain;
     return hip_status(e, "nmi_gemv_chain_destroy");
 }
+
+int nmi_linear_workspace_needs_zero(int M) { return M < 512 || gemm_workspace_has_flags(M) ? 1 : 0; }
 
 size_t nmi_linear_workspace_bytes(int M, int64_t total_n, int K) { return linear_workspace_bytes(M, total_n, K); }
 

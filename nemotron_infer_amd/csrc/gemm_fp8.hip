@@ -217,6 +217,10 @@ struct GemmArgs {
     };
     int ngroups;
     Group grp[kMaxGroups];
+    // DMA-fed kernel with K split (SPLIT): every tile as `splits` runs of k tiles, whose float32
+    // partial tiles go to `part` (split sp of tile t at slot t * splits + sp).
+    int splits;
+    float* part;
 };
 
 // ---------------------------------------------------------------------------------------
@@ -499,13 +503,21 @@ __device__ __forceinline__ void tile_coords(int seq, int tiles_m, int tiles_n, i
     tm = r0 + (loc - tn * h);
 }
 
-template <bool SK, bool GROUPED, int BM = 256>
+// The wait for this wave's DMAs of all but the latest N, with the workgroup barrier.
+template <int N>
+__device__ __forceinline__ void dma_wait_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+template <bool SK, bool GROUPED, int BM = 256, bool SPLIT = false>
 __global__ __launch_bounds__(256, 1) void gemm_fp8_w8a16_dma_kernel(const GemmArgs a) {
-    // BM = 256: 256 x 256 tiles, each wave 128 x 128 (TM = 4 blocks of 32 x rows); BM = 128:
-    // 128 x 256 tiles, each wave 64 x 128 (TM = 2), data-parallel only
-    static_assert(BM == 256 || (BM == 128 && !SK), "tile rows");
+    // BM = 256: 256 x 256 tiles, each wave 128 x 128 (TM = 4 blocks of 32 x rows); BM = 192 and
+    // 128: 192 x 256 and 128 x 256 tiles, each wave 96 or 64 x 128 (TM = 3, 2), not stream-K
+    static_assert(BM == 256 || ((BM == 192 || BM == 128) && !SK), "tile rows");
+    static_assert(!SPLIT || (!SK && !GROUPED), "K split: one matrix, data-parallel form");
     constexpr int NT = 256, BK = kBK, W_STAGE = 256 * 64, TN = 4, TM = BM / 64;
     constexpr int XI = BM / 32;                     // x DMA instructions per wave and k tile
+    constexpr int ND = 4 + XI;                      // DMA instructions per wave and k tile
     constexpr int STAGE = W_STAGE + BM * 128;       // bytes per LDS stage
     __shared__ int sk_up;                           // stream-K: the flag the finisher waited for came
     typedef __attribute__((address_space(3))) void lds_void;
@@ -630,20 +642,16 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_w8a16_dma_kernel(const GemmAr
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, cf[i]), xf[j], acc[i][j], 0, 0, 0);
         };
 
-        constexpr int NP = 1 + BM / 128;            // DMA parts per k tile (4 instructions each)
+        // DMA instruction d (0 .. ND - 1) of a k tile: the W tile (part 0), then the x tile
+        auto dma_nth = [&](uint32_t base, int kt, int d) { dma_to(base, kt, d >> 2, d & 3); };
 #pragma unroll
-        for (int p = 0; p < NP; ++p)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) dma_to(s_cur, kb, p, k);
+        for (int d = 0; d < ND; ++d) dma_nth(s_cur, kb, d);
         if (kb + 1 < ke) {
 #pragma unroll
-            for (int p = 0; p < NP; ++p)
-#pragma unroll
-                for (int k = 0; k < 4; ++k) dma_to(s_nxt, kb + 1, p, k);
-            if constexpr (BM == 256) asm volatile("s_waitcnt vmcnt(12)\n\ts_barrier" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
+            for (int d = 0; d < ND; ++d) dma_nth(s_nxt, kb + 1, d);
+            dma_wait_barrier<ND>();
         } else {
-            asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+            dma_wait_barrier<0>();
         }
         uint4 wr0[4], wr1[4];
         bf16x8 xa[TM], xb[TM];
@@ -702,15 +710,66 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_w8a16_dma_kernel(const GemmAr
                 for (int q = 0; q < 8; ++q) {
                     mf(cB, xb, q);
                     if (more) {
-                        if (q == 1) {
-                            if (pf) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                        }
+                        if (q == 1) dma_wait_barrier<pf ? ND : 0>();
                         if (q >= 2 && q < 6) wr0[q - 2] = rd_w(nst, 0, q - 2);
                         else if (q >= 6) xa[q - 6] = rd_x(nst, 0, q - 6);
                         if (q >= 6) {
                             cvt1(wr0, 0, 2 * (q - 6), cA);
                             cvt1(wr0, 0, 2 * (q - 6) + 1, cA);
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else if constexpr (BM == 192) {
+                // 192 x 256 tiles: 12 MFMAs per k step (q: W block q / 3, x block q % 3), one or
+                // two conversions per MFMA; the W DMAs go in step 0, the six x DMAs in steps 1 and
+                // 2.  Step 3 reads the next tile's step-0 operands after its barrier and converts
+                // them in its second half.
+                auto cvt12 = [&](const uint4 (&wr)[4], int t, int q, u32x4 (&cf)[4]) {
+                    if (q < 4) {
+                        cvt1(wr, t, 2 * q, cf);
+                        cvt1(wr, t, 2 * q + 1, cf);
+                    } else {
+                        cvt1(wr, t, q + 4, cf);
+                    }
+                };
+#pragma unroll
+                for (int q = 0; q < 12; ++q) {
+                    mf(cA, xa, q);
+                    if (q < 3) xb[q] = rd_x(st, 1, q);
+                    else if (q < 7) wr1[q - 3] = rd_w(st, 1, q - 3);
+                    if (pf && q % 3 == 2) dma_nth(s_dma, kt + 2, q / 3);
+                    cvt12(wr0, 1, q, cB);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int q = 0; q < 12; ++q) {
+                    mf(cB, xb, q);
+                    if (q < 3) xa[q] = rd_x(st, 2, q);
+                    if (pf && (q & 3) == 3) dma_nth(s_dma, kt + 2, 4 + (q >> 2));
+                    cvt12(wr1, 0, q, cA);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int q = 0; q < 12; ++q) {
+                    mf(cA, xa, q);
+                    if (q < 3) xb[q] = rd_x(st, 3, q);
+                    if (pf && (q & 3) == 3) dma_nth(s_dma, kt + 2, 7 + (q >> 2));
+                    cvt12(wr1, 1, q, cB);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int q = 0; q < 12; ++q) {
+                    mf(cB, xb, q);
+                    if (more) {
+                        if (q == 1) dma_wait_barrier<pf ? ND : 0>();
+                        if (q >= 2 && q < 6) wr0[q - 2] = rd_w(nst, 0, q - 2);
+                        else if (q >= 6 && q < 9) xa[q - 6] = rd_x(nst, 0, q - 6);
+                        // the fragments' first MFMAs are at least three slots away: W block
+                        // (c / 4) is converted in the order it was read
+                        if (q >= 6) {
+#pragma unroll
+                            for (int c = (16 * (q - 6)) / 6; c < (16 * (q - 5)) / 6; ++c) cvt1(wr0, 0, c, cA);
                         }
                     }
                     __builtin_amdgcn_sched_barrier(0);
@@ -753,10 +812,7 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_w8a16_dma_kernel(const GemmAr
             for (int q = 0; q < 16; ++q) {
                 mf(cB, xb, q);
                 if (more) {
-                    if (q == 1) {
-                        if (pf) asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                    }
+                    if (q == 1) dma_wait_barrier<pf ? ND : 0>();
                     if (q >= 2 && q < 6) wr0[q - 2] = rd_w(nst, 0, q - 2);
                     else if (q >= 6 && q < 10) xa[q - 6] = rd_x(nst, 0, q - 6);
                     if (q >= 8) {
@@ -899,15 +955,37 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_w8a16_dma_kernel(const GemmAr
         // against n-fastest order).
         const int g = (int)blockIdx.x;
         const int local = g >> 3;
-        const int tile = (g & 7) * a.per_xcd + local;
-        if (local >= a.per_xcd || tile >= a.tiles_m * a.tiles_n) return;   // uniform
+        const int unit = (g & 7) * a.per_xcd + local;
+        const int T = a.tiles_m * a.tiles_n;
+        const int sp = SPLIT ? unit / T : 0;        // K split: units (split, tile), tiles fastest
+        if (local >= a.per_xcd || unit >= (SPLIT ? T * a.splits : T)) return;  // uniform
+        const int tile = unit - sp * T;
         int tm, tn;
         tile_coords(tile, a.tiles_m, a.tiles_n, a.gh, tm, tn);
         m0 = tm * BM;
         select(tn);
         zero_acc();
-        run(0, KT);
-        store();
+        if constexpr (!SPLIT) {
+            run(0, KT);
+            store();
+        } else {
+            run((int)((int64_t)sp * KT / a.splits), (int)((int64_t)(sp + 1) * KT / a.splits));
+            // the accumulators as they lie: 16-byte piece p of thread t at (p * 256 + t) * 16 of the
+            // slot, whole 4 KiB runs per workgroup and piece
+            const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(
+                a.part + ((size_t)tile * a.splits + sp) * (BM * 256), 0, BM * 256 * (int)sizeof(float), 0x00020000);
+#pragma unroll
+            for (int i = 0; i < TN; ++i)
+#pragma unroll
+                for (int j = 0; j < TM; ++j)
+#pragma unroll
+                    for (int gq = 0; gq < 4; ++gq) {
+                        const f32x4 v{acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2],
+                                      acc[i][j][4 * gq + 3]};
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), out, tid * 16,
+                                                               ((i * TM + j) * 4 + gq) * NT * 16, 0);
+                    }
+        }
     } else {
         // Stream-K as in the 8-wave kernel: per-XCD problems, each workgroup a contiguous range
         // of (tile, k tile) steps walked backwards; the workgroup holding a tile's last k tile
@@ -1073,6 +1151,98 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_w8a16_dma_kernel(const GemmAr
 #undef gv16
 #undef gv16r
 
+// Sum of a split tile's float32 partials in split order, the scale, one rounding, the epilogue.
+// One workgroup per 32-row strip of a tile; a thread holds the partials' 16-byte pieces
+// of one lane of the main kernel's waves (so the loads are whole 1 KiB runs), rounds v into a
+// bf16 copy of the strip in LDS, and stores 16-byte row pieces as the main kernel's epilogue does.
+template <int BM>
+__global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const GemmArgs a) {
+    constexpr int TM = BM / 64, STRIPS = BM / 32, PITCH = 520;
+    __shared__ __attribute__((aligned(16))) uint8_t sm[32 * PITCH];
+    const GemmArgs::Group& G = a.grp[0];
+    const int r = (int)blockIdx.x / STRIPS, strip = (int)blockIdx.x % STRIPS;
+    int tm, tn;
+    tile_coords(r, a.tiles_m, a.tiles_n, a.gh, tm, tn);
+    const int m0 = tm * BM + 32 * strip, n0 = tn * 256;
+    if (m0 >= a.M) return;                          // uniform: a strip past the last row
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int h = lane >> 5, l32 = lane & 31;
+    const int wm = strip / TM, j = strip % TM;      // the strip's wave row and row block
+    const int wn = wave >> 1, i0 = 2 * (wave & 1);  // this wave's column half and first column block
+    const int src = (wm * 2 + wn) * 64 + lane;      // the main kernel's thread
+    const float4* part = reinterpret_cast<const float4*>(a.part + (size_t)r * a.splits * (BM * 256)) + src;
+    float4 v[2][4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int gq = 0; gq < 4; ++gq) v[i][gq] = part[(((i0 + i) * TM + j) * 4 + gq) * 256];
+#pragma unroll 3
+    for (int sp = 1; sp < a.splits; ++sp) {
+        const float4* ps = part + (size_t)sp * (BM * 64);
+        float4 f[2][4];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int gq = 0; gq < 4; ++gq) f[i][gq] = ps[(((i0 + i) * TM + j) * 4 + gq) * 256];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int gq = 0; gq < 4; ++gq) {
+                v[i][gq].x += f[i][gq].x; v[i][gq].y += f[i][gq].y;
+                v[i][gq].z += f[i][gq].z; v[i][gq].w += f[i][gq].w;
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int gq = 0; gq < 4; ++gq) {
+            const int nl = wn * 128 + (i0 + i) * 32 + 8 * gq + 4 * h;
+            float sc[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sc[e] = G.s[min(n0 + nl + e, G.N - 1)];
+            *reinterpret_cast<uint2*>(sm + l32 * PITCH + nl * 2) =
+                uint2{pack_bf16(v[i][gq].x * sc[0], v[i][gq].y * sc[1]), pack_bf16(v[i][gq].z * sc[2], v[i][gq].w * sc[3])};
+        }
+    __syncthreads();
+    const int c8 = (tid & 31) * 8, n = n0 + c8;
+    const bool full = G.vec16 && n + 7 < G.N;
+    const bool res16 = full && G.vec16_res;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        const int row = (tid >> 5) + 8 * p;
+        if (m0 + row >= a.M) continue;
+        const uint2* sp = reinterpret_cast<const uint2*>(sm + row * PITCH + c8 * 2);
+        const uint2 v0 = sp[0], v1 = sp[1];
+        uint32_t w[4] = {v0.x, v0.y, v1.x, v1.y};
+        if (G.epi == kEpiResidual) {
+            const uint16_t* rp = G.res + (int64_t)(m0 + row) * G.ldres + n;
+            uint32_t rv[4];
+            if (res16) {
+                const uint4 r4 = *reinterpret_cast<const uint4*>(rp);
+                rv[0] = r4.x; rv[1] = r4.y; rv[2] = r4.z; rv[3] = r4.w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    rv[e] = (n + 2 * e < G.N ? (uint32_t)rp[2 * e] : 0u) |
+                            ((n + 2 * e + 1 < G.N ? (uint32_t)rp[2 * e + 1] : 0u) << 16);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = add_bf16x2(w[e], rv[e]);
+        } else if (G.epi == kEpiRelu2) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = relu2_bf16x2(w[e]);
+        }
+        uint16_t* yp = G.y + (int64_t)(m0 + row) * G.ldy + n;
+        if (full) {
+            *reinterpret_cast<uint4*>(yp) = uint4{w[0], w[1], w[2], w[3]};
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (n + e < G.N) yp[e] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+        }
+    }
+}
+
 // Stream-K workspace: the flag slots share the 64 KiB counter region of the skinny kernel's
 // workspace layout (zero at rest in both; the last 4 bytes are the error word, NMI_WS_ERROR_OFFSET),
 // then one fp32 partial tile per workgroup.
@@ -1110,36 +1280,107 @@ bool dma_supported(const uint16_t* x, int64_t ldx, const uint8_t* W, int64_t ldw
            (int64_t)N * ldw < ((int64_t)1 << 31);
 }
 
-// The DMA-fed kernel: one tile per workgroup, or stream-K over all CUs when the tiles cover at
-// most half of them and the workspace holds the flags and one partial tile per workgroup
-// (tuning knob gemm.sk: 1 forces stream-K where the workspace allows, 2 forbids it).
-// Measured on MI355X (config 3, steady state): stream-K 950 vs 792 TFLOP/s on down_proj (104
-// tiles), but 955 vs 1002 on up_proj (392 tiles) and 879 vs 1050 on qkv (224 tiles): with every
-// CU busy the clock drops (~1.85 vs ~2.3 GHz with 104 busy) and the partial tiles cost traffic,
-// so filling a partly idle last round does not pay.
+constexpr int dma_lds_bytes(int bm) { return kDmaStages * (256 * 64 + bm * 128); }
+
+// The kernel without stream-K for `bm` tile rows, one matrix or several, K whole or split (one
+// matrix only).
+using DmaKernel = void (*)(GemmArgs);
+DmaKernel dma_kernel(int bm, bool grouped, bool split) {
+    switch (bm) {
+        case 128:
+            return split     ? &gemm_fp8_w8a16_dma_kernel<false, false, 128, true>
+                   : grouped ? &gemm_fp8_w8a16_dma_kernel<false, true, 128>
+                             : &gemm_fp8_w8a16_dma_kernel<false, false, 128>;
+        case 192:
+            return split     ? &gemm_fp8_w8a16_dma_kernel<false, false, 192, true>
+                   : grouped ? &gemm_fp8_w8a16_dma_kernel<false, true, 192>
+                             : &gemm_fp8_w8a16_dma_kernel<false, false, 192>;
+        default:
+            return split     ? &gemm_fp8_w8a16_dma_kernel<false, false, 256, true>
+                   : grouped ? &gemm_fp8_w8a16_dma_kernel<false, true, 256>
+                             : &gemm_fp8_w8a16_dma_kernel<false, false, 256>;
+    }
+}
+
+// How a launch of the DMA-fed kernel covers T = tiles_m x tiles_n tiles: the tile rows and, with
+// splits > 1, K cut into that many runs per tile.
+struct DmaPlan {
+    int bm, tiles, splits;
+    size_t part_bytes() const { return splits > 1 ? (size_t)tiles * splits * bm * 256 * sizeof(float) : 0; }
+};
+
+// The plan with the least modelled time.  One workgroup per CU, so U workgroups take
+// ceil(U / CUs) rounds; a k tile costs its workgroup a fixed time plus a share that grows with the
+// CUs in use (they share the power budget: the clock falls), fitted to a sweep of M = 512 .. 4096
+// on the model's projections (us, MI355X; the fit is within 5% of most of them):
+//   rounds * (start + KT * fixed) + KT * U / CUs * shared,   KT = k tiles of one workgroup,
+// and a split adds its second kernel.  K is split only from 4096 up and into one round of
+// workgroups (below, no split of any projection was faster than its best unsplit tiles) and only
+// for a modelled gain of 8%: with most CUs busy either way the power budget decides (2048 x 3136 x
+// 12544, 256-row tiles split in two against whole 128-row tiles: 143 against 148 us on one box, the
+// MLP block 329 against 318 us on another).
+// Examples (us): 777 x 12544 x 3136 256 / 192 / 128-row tiles 67.5 / 59.6 / 75.9; 2048 x 17504 x
+// 3136 209 / 180 / 209; 512 x 3136 x 12544 in 128-row tiles, splits of 1 / 2 / 3 / 4: 113 / 70 /
+// 55 / 50; 1000 x 3136 x 7680 1 / 2: 74 / 57.  Tuning knobs: gemm.bm forces the tile rows, gemm.splits the split (1: none).
+DmaPlan dma_plan(int M, int tiles_n, int K, bool may_split) {
+    struct Cost { int bm; double start, fixed, shared; };
+    constexpr Cost kCost[] = {{256, 12.0, 0.857, 0.408}, {192, 10.0, 0.61, 0.41}, {128, 8.6, 0.395, 0.337}};
+    constexpr double kReduce = 5.0, kReducePerByte = 0.09e-6;
+    constexpr double kSplitMargin = 1.08;
+    constexpr int kMinSplitK = 4096, kMaxSplits = 16;
+    const Tuning& t = tuning();
+    const int G = device_info().num_cu, KT = K / kBK;
+    DmaPlan best{};
+    double best_us = 0;
+    for (const Cost& c : kCost) {
+        if ((t.gemm_bm == 128 || t.gemm_bm == 192 || t.gemm_bm == 256) && t.gemm_bm != c.bm) continue;
+        const int64_t T = (int64_t)((M + c.bm - 1) / c.bm) * tiles_n;
+        for (int sp = 1; sp <= kMaxSplits; ++sp) {
+            const bool forced = t.gemm_splits > 0 && sp == t.gemm_splits;
+            if (sp > 1) {
+                if (!may_split || sp > KT || T * sp > (int64_t)4 * G) break;
+                if (t.gemm_splits > 0 ? !forced : (K < kMinSplitK || T * sp > G)) continue;
+            }
+            const DmaPlan p{c.bm, (int)T, sp};
+            const int64_t rounds = (T * sp + G - 1) / G;
+            const double kt = (double)((KT + sp - 1) / sp);
+            double us = rounds * (c.start + kt * c.fixed) + kt * c.shared * (double)(T * sp) / G;
+            if (sp > 1) us = (us + kReduce + (double)p.part_bytes() * kReducePerByte) * kSplitMargin;
+            if (forced && sp > 1) us -= 1e9;        // a forced split wins over its unsplit forms
+            if (best.bm == 0 || us < best_us) best = p, best_us = us;
+        }
+    }
+    return best;
+}
+
+// The DMA-fed kernel as dma_plan says, or under the knobs gemm.sk = 1 / gemm.bm = 256 in 256-row
+// tiles, one per workgroup or stream-K (gemm.sk = 1 where the workspace allows; with gemm.bm = 256
+// where the tiles cover at most half of the CUs; gemm.sk = 2: never).
 // ng > 1: matrices sharing x in one launch (their column bands follow one another in the
 // launch's tile numbering, each tile looks up its matrix).  Measured on MI355X: the attention
 // block's q | k | v at S = 2048 (160 + 32 + 32 tiles) as one launch took the block 496 -> 380 us.
 hipError_t launch_dma_groups(const uint16_t* x, int64_t ldx, const GemvGroup* g, int ng, int M, int K,
                              hipStream_t stream, void* ws, size_t ws_bytes) {
     constexpr int lds = kDmaStages * kDmaStage;
-    constexpr int lds128 = kDmaStages * (256 * 64 + 128 * 128);
     static const hipError_t attr = [] {
         hipError_t e = hipSuccess;
-        for (const void* k : {reinterpret_cast<const void*>(&gemm_fp8_w8a16_dma_kernel<false, false>),
-                              reinterpret_cast<const void*>(&gemm_fp8_w8a16_dma_kernel<true, false>),
-                              reinterpret_cast<const void*>(&gemm_fp8_w8a16_dma_kernel<false, true>),
-                              reinterpret_cast<const void*>(&gemm_fp8_w8a16_dma_kernel<true, true>)})
-            if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        for (const void* k : {reinterpret_cast<const void*>(&gemm_fp8_w8a16_dma_kernel<false, false, 128>),
-                              reinterpret_cast<const void*>(&gemm_fp8_w8a16_dma_kernel<false, true, 128>)})
-            if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds128);
+        const auto set = [&e](DmaKernel k, int bytes) {
+            if (e == hipSuccess)
+                e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+        };
+        set(&gemm_fp8_w8a16_dma_kernel<true, false>, lds);
+        set(&gemm_fp8_w8a16_dma_kernel<true, true>, lds);
+        for (const int bm : {128, 192, 256}) {
+            set(dma_kernel(bm, false, false), dma_lds_bytes(bm));
+            set(dma_kernel(bm, true, false), dma_lds_bytes(bm));
+            set(dma_kernel(bm, false, true), dma_lds_bytes(bm));
+        }
         return e;
     }();
     if (attr != hipSuccess) return attr;
     if (ng < 1 || ng > kMaxGroups) return hipErrorInvalidValue;
     const bool grouped = ng > 1;
-    const auto dp_kernel = grouped ? &gemm_fp8_w8a16_dma_kernel<false, true> : &gemm_fp8_w8a16_dma_kernel<false, false>;
+    const auto dp_kernel = dma_kernel(256, grouped, false);
     const auto sk_kernel = grouped ? &gemm_fp8_w8a16_dma_kernel<true, true> : &gemm_fp8_w8a16_dma_kernel<true, false>;
     GemmArgs a{};
     a.x = x; a.ldx = ldx;
@@ -1162,27 +1403,23 @@ hipError_t launch_dma_groups(const uint16_t* x, int64_t ldx, const GemvGroup* g,
     a.per_xcd = (T + 7) / 8;
     const int G = device_info().num_cu;             // one 144 KiB workgroup per CU
     const int gh_knob = tuning().gemm_gh;
-    // 128 x 256 tiles where they finish sooner: with one workgroup per CU a grid of t tiles takes
-    // ceil(t / CUs) rounds, and a 128-row tile costs 0.525 of a 256-row one (its MFMA rate measured
-    // 4-5% lower: down_proj at M = 2048 1152 against 1208 TFLOP/s).  That takes them where the
-    // 256-row tiles cover at most half the CUs -- each workgroup then has a whole tile with the
-    // same MFMA work as half a tile of the stream-K form, without its partial-tile exchange:
-    // down_proj at M = 2048 (208 tiles) 146.3 against 168.8 us in stream-K form, attention block at
-    // S = 2048 250 against 296 us, Mamba block at S = 512 336 against 376 us -- and where the
-    // 256-row tiles leave a short last round: the Mamba in_proj at M = 2048 (552 tiles, 3 rounds,
-    // against 1104 in 5) took the block 531 -> 524 us.  Tuning knob gemm.bm: 128 forces them, 256
-    // forbids them; gemm.sk = 1 keeps stream-K.
-    const int bm_knob = tuning().gemm_bm;
-    const int64_t T128 = (int64_t)((M + 127) / 128) * a.tiles_n;
-    const bool short_tiles = 21 * ((T128 + G - 1) / G) < 40 * (((int64_t)T + G - 1) / G);
-    if (bm_knob != 256 && tuning().gemm_sk != 1 && (bm_knob == 128 || short_tiles)) {
-        const auto kernel128 =
-            grouped ? &gemm_fp8_w8a16_dma_kernel<false, true, 128> : &gemm_fp8_w8a16_dma_kernel<false, false, 128>;
-        a.tiles_m = (M + 127) / 128;
-        const int T128 = a.tiles_m * a.tiles_n;
-        a.per_xcd = (T128 + 7) / 8;
+    // gemm.sk = 1 and gemm.bm = 256 keep the 256-row tiles below (stream-K where it is wanted)
+    if (tuning().gemm_sk != 1 && (tuning().gemm_bm != 256 || tuning().gemm_splits > 1)) {
+        DmaPlan p = dma_plan(M, tn, K, ng == 1 && ws != nullptr);
+        if (p.splits > 1 && ws_bytes < kSkFlagBytes + p.part_bytes()) p = dma_plan(M, tn, K, false);
+        a.tiles_m = (M + p.bm - 1) / p.bm;
         a.gh = gh_knob > 0 ? std::min(gh_knob, a.tiles_m) : a.tiles_m;
-        hipLaunchKernelGGL(kernel128, dim3(8 * a.per_xcd), dim3(256), lds128, stream, a);
+        a.splits = p.splits;
+        if (p.splits > 1) a.part = reinterpret_cast<float*>(static_cast<char*>(ws) + kSkFlagBytes);
+        a.per_xcd = (int)(((int64_t)p.tiles * p.splits + 7) / 8);
+        const auto kernel = dma_kernel(p.bm, grouped, p.splits > 1);
+        hipLaunchKernelGGL(kernel, dim3(8 * a.per_xcd), dim3(256), dma_lds_bytes(p.bm), stream, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess || p.splits == 1) return e;
+        const auto reduce = p.bm == 256   ? &gemm_split_reduce_kernel<256>
+                            : p.bm == 192 ? &gemm_split_reduce_kernel<192>
+                                          : &gemm_split_reduce_kernel<128>;
+        hipLaunchKernelGGL(reduce, dim3((unsigned)(p.tiles * (p.bm / 32))), dim3(256), 0, stream, a);
         return hipGetLastError();
     }
     const bool fits = ws && ws_bytes >= kSkFlagBytes + (size_t)G * kDmaPartialBytes && G % 8 == 0 &&
@@ -1235,13 +1472,20 @@ hipError_t launch_sk_flags_clear(void* ws, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// Only the stream-K form uses a workspace, and it runs only under gemm.sk = 1 (or with the
-// 128-row tiles forbidden, gemm.bm = 256): otherwise none, so that the blocks neither reserve
-// its 64 MiB nor clear its flags.
+// The stream-K form's workspace: it runs only under gemm.sk = 1 (or with the other tile rows
+// forbidden, gemm.bm = 256), so the blocks otherwise neither reserve its 64 MiB nor clear its flags.
 size_t gemm_workspace_bytes(int M) {
     const Tuning& t = tuning();
     if (M < 512 || t.gemm_sk == 2 || (t.gemm_sk != 1 && t.gemm_bm != 256)) return 0;
     return kSkFlagBytes + (size_t)device_info().num_cu * kDmaPartialBytes;
+}
+
+// The K split's partial tiles for one matrix of N rows (after the 64 KiB flag region, which it
+// leaves alone); 0 where dma_plan does not split.
+size_t gemm_split_workspace_bytes(int M, int64_t N, int K) {
+    if (M < 512 || K % kBK != 0 || N > (1 << 30) || tuning().gemm_sk == 1) return 0;
+    const DmaPlan p = dma_plan(M, (int)((N + 255) / 256), K, true);
+    return p.splits > 1 ? kSkFlagBytes + p.part_bytes() : 0;
 }
 
 // A grouped GEMM (matrices sharing x) as one launch of the DMA-fed kernel where it takes every

@@ -63,26 +63,27 @@ MambaLayout mamba_layout(int batch, int hidden, const MambaDims& d) {
     return L;
 }
 
-// Prefill workspace: the GEMMs' stream-K region (M = batch * S >= 512), normed [M, hidden],
+// Prefill workspace (M = batch * S): the GEMMs' region, normed [M, hidden],
 // proj [M, proj_ld], xc [M, conv_dim rounded to 8], y [M, INTER], g [M, INTER].
 struct FwdLayout {
     size_t gemm, normed, proj, xc, y, g, total;
     int64_t xc_ld;
 };
 
-// The GEMMs' region (the short-prompt kernel's K-split partials below M = 512; from 512 the
-// stream-K flags and partials where that form is forced by tuning knob, else nothing):
-// the larger of the in_proj and out_proj needs.
-size_t gemm_region(int M, int hidden, const MambaDims& d) {
+// The GEMMs' region (the K splits' partials, or the stream-K flags and partials where that form
+// is forced by tuning knob): the larger of the in_proj and out_proj needs.  split = false: without
+// the K split of M >= 512.
+size_t gemm_region(int M, int hidden, const MambaDims& d, bool split) {
     if (choose_path(M) != Path::Gemm) return 0;
-    return round256(std::max(linear_workspace_bytes(M, d.proj, hidden), linear_workspace_bytes(M, hidden, d.inter)));
+    const auto need = split ? linear_workspace_bytes : linear_workspace_bytes_unsplit;
+    return round256(std::max(need(M, d.proj, hidden), need(M, hidden, d.inter)));
 }
 
-FwdLayout fwd_layout(int M, int hidden, const MambaDims& d) {
+FwdLayout fwd_layout(int M, int hidden, const MambaDims& d, bool split = true) {
     FwdLayout L{};
     L.xc_ld = (d.conv_dim + 7) & ~7;
     L.gemm = 0;
-    L.normed = L.gemm + gemm_region(M, hidden, d);
+    L.normed = L.gemm + gemm_region(M, hidden, d, split);
     L.proj = L.normed + round256((size_t)M * hidden * 2);
     L.xc = L.proj + round256((size_t)M * d.proj_ld * 2);
     L.y = L.xc + round256((size_t)M * L.xc_ld * 2);
@@ -140,10 +141,11 @@ int nmi_mamba_forward_fp8(const void* input_bf16, const float* norm_w, const voi
         !aligned(out_bf16, 2))
         return fail(NMI_ERR_ALIGNMENT, "nmi_mamba_forward_fp8: misaligned scale, parameter, state or output");
     const int M = batch * S;
-    const FwdLayout lay = fwd_layout(M, hidden, d);
+    FwdLayout lay = fwd_layout(M, hidden, d);
     if (workspace) {
         if (!aligned(workspace, 256))
             return fail(NMI_ERR_ALIGNMENT, "nmi_mamba_forward_fp8: workspace must be 256-byte aligned");
+        if (workspace_bytes < lay.total) lay = fwd_layout(M, hidden, d, false);
         if (workspace_bytes < lay.total) {
             set_last_error("%s: workspace of %zu bytes, %zu needed", fn, workspace_bytes, lay.total);
             return NMI_ERR_WORKSPACE;

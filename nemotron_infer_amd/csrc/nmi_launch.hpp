@@ -54,9 +54,9 @@ struct Tuning {
     int sdpa_chunk = 0;    // attention decode: positions per split (0: kSdpaMinChunk, capped by the grid size)
     int gemv_grid = 0;     // M = 1 stream GEMV (single launches): explicit workgroup count
     int gemv_balance = 0;  // M = 1 stream GEMV (single launches): 2 turns off the grid sizing that makes row groups divide evenly
-    int gemm_splits = 0;   // short-prompt GEMM (17 <= M < 512): workgroups splitting K (0: automatic)
+    int gemm_splits = 0;   // GEMM: workgroups splitting K (0: automatic, 1: none)
     int gemm_short = 0;    // short-prompt GEMM: f + 1 forces kernel form f (0..7, gemm_short.hip)
-    int gemm_bm = 0;       // DMA-fed GEMM tile rows: 0 automatic (128 where 256-row tiles cover at most half the CUs), 128, 256
+    int gemm_bm = 0;       // DMA-fed GEMM tile rows: 0 automatic (dma_plan), 128, 192, 256
     int gemm_sk_cap = 0;   // GEMM stream-K: at most this many workgroups per tile (0: 2; -1: one per CU)
     int gemm_gh = 0;       // DMA-fed GEMM: row bands per group of the tile order (0: all of them, stream-K: 1)
     int s16 = 0;           // 16x16x32 skinny kernel: 0 automatic (M >= 3), 1 for 2 <= M <= 16, 2 never
@@ -202,6 +202,9 @@ hipError_t launch_gemv_stream_chain(const StreamPhase* tab, const int* wave_step
 // one tile per workgroup.  launch_sk_flags_clear zeroes the flag region (one small kernel, safe
 // under graph capture).
 size_t gemm_workspace_bytes(int M);
+// Workspace of the DMA-fed kernel's K split (M >= 512, one matrix of N rows; 0: not split): float32
+// partial tiles after the flag region, no initialisation needed.
+size_t gemm_split_workspace_bytes(int M, int64_t N, int K);
 // Short prompts (17 <= M < 512; gemm_short.hip): the pipelined 128-row-tile kernel, with K split
 // between workgroups when a workspace of gemm_short_workspace_bytes(M, N, K) bytes is given
 // (float32 partials, no initialisation needed; 0: the schedule does not split).
@@ -213,6 +216,8 @@ size_t gemm_short_workspace_bytes(int M, int N, int K);
 // (launch_sk_flags_clear) -- the short-prompt kernel's partials need no initialisation.
 size_t linear_workspace_bytes(int M, int64_t total_n, int K);
 bool gemm_workspace_has_flags(int M);
+// The same without the K split of M >= 512, whose region a caller may leave out.
+size_t linear_workspace_bytes_unsplit(int M, int64_t total_n, int K);
 // The fp8 MLP block (block.cpp) behind nmi_mlp_forward_fp8 (split = true) and its allocation-free
 // form (split = false: the short-prompt GEMMs run unsplit, so the workspace has no partial
 // region); fn names the entry point in error messages.

@@ -68,7 +68,7 @@ _WORKSPACE: dict[int, torch.Tensor] = {}
 
 
 def workspace(device: torch.device, nbytes: int) -> torch.Tensor | None:
-    """Per-device workspace of the skinny kernel's K split: zero-filled when (re)allocated,
+    """Per-device workspace of the short-prompt GEMM's K split: zero-filled when (re)allocated,
     kept for the process; every launch leaves it ready for the next.  Calls on one device
     share it, so they must be ordered on one stream (as torch's current stream orders them).
     Grows on demand -- make one eager call of the largest shape before capturing a graph."""
@@ -80,6 +80,16 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor | None:
         ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _WORKSPACE[idx] = ws
     return ws
+
+
+def _linear_ws(L, device: torch.device, M: int, N: int, K: int) -> torch.Tensor | None:
+    """The workspace of one linear call.  From M = 512 the K split's partials (up to 64 MiB) come
+    from torch's allocator for this call, ordered on the current stream like any temporary, so
+    calls on several streams share nothing; below, the per-device tensor of workspace()."""
+    need = L.nmi_linear_workspace_bytes(M, N, K)
+    if need and M >= 512 and not L.nmi_linear_workspace_needs_zero(M):
+        return torch.empty(need, dtype=torch.uint8, device=device)
+    return workspace(device, need)
 
 
 def _as_2d(x: torch.Tensor):
@@ -105,7 +115,7 @@ def linear_fp8_w8a16(x: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
     y2 = _check_out(out, M, N)
     _check_device(x2, w, w_scale, y2)
     L = _lib.lib()
-    ws = workspace(x.device, L.nmi_linear_workspace_bytes(M, N, K)) if use_workspace else None
+    ws = _linear_ws(L, x.device, M, N, K) if use_workspace else None
     rc = L.nmi_linear_fp8_w8a16_ws(
         x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0), w_scale.data_ptr(),
         y2.data_ptr(), y2.stride(0), M, N, K,
@@ -136,7 +146,7 @@ def linear_fp8_w8a16_grouped(x: torch.Tensor, weights, outs=None, use_workspace:
                                   w.shape[0])
     L = _lib.lib()
     total = sum(w.shape[0] for w, _ in weights)
-    ws = workspace(x.device, L.nmi_linear_workspace_bytes(M, total, K)) if use_workspace else None
+    ws = _linear_ws(L, x.device, M, total, K) if use_workspace else None
     rc = L.nmi_linear_fp8_w8a16_grouped(x2.data_ptr(), x2.stride(0), M, K, arr, n,
                                         None if ws is None else ws.data_ptr(),
                                         0 if ws is None else ws.numel(), _stream())
@@ -195,8 +205,8 @@ def gemv_fp8(x: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
 
 def gemm_fp8_w8a16(x: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
                    out: torch.Tensor | None = None, use_workspace: bool = True) -> torch.Tensor:
-    """Prefill GEMM on bf16 MFMA for any M (ops/gemm.cuh:325-403 replacement).  With the
-    per-device workspace the large-tile kernels may split K between workgroups (stream-K)."""
+    """Prefill GEMM on bf16 MFMA for any M (ops/gemm.cuh:325-403 replacement).  With a workspace
+    the kernels may split K between workgroups."""
     if x.dim() != 2:
         raise ValueError("x must be a 2-D [M, K] bf16 matrix")
     x2 = _as_2d(x)
@@ -209,7 +219,7 @@ def gemm_fp8_w8a16(x: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
     y2 = _check_out(out, M, N)
     _check_device(x2, w, w_scale, y2)
     L = _lib.lib()
-    ws = workspace(x.device, L.nmi_linear_workspace_bytes(M, N, K)) if use_workspace else None
+    ws = _linear_ws(L, x.device, M, N, K) if use_workspace else None
     rc = L.nmi_gemm_fp8_w8a16(x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0),
                               w_scale.data_ptr(), y2.data_ptr(), y2.stride(0), M, N, K,
                               None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),

@@ -1,0 +1,119 @@
+"""The DMA-fed GEMM's tile rows (128, 192, 256) and its K split (float32 partial tiles in the
+workspace, added by a second kernel) against the oracle, at the edges of the tiles."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import DEV, announce, assert_parity, bits, oracle_bits, s_to_dev, w_to_dev, x_to_dev
+from nemotron_infer_amd import _lib, ops, synth
+
+pytestmark = pytest.mark.gpu
+
+KNOBS = ("gemm.bm", "gemm.splits", "gemm.tile", "gemm.sk")
+
+
+@pytest.fixture(autouse=True)
+def _reset():
+    yield
+    for k in KNOBS:
+        _lib.tuning_set(k, 0)
+
+
+def _case(M, N, K, seed, scales="log_uniform"):
+    w, s = synth.make_weight(N, K, seed, "cpu", scales=scales)
+    x = synth.make_act(M, K, seed + 1, "cpu")
+    return x.view(torch.int16).numpy().view(np.uint16), w.numpy(), s.numpy()
+
+
+def _call(xd, wd, sd, y, ldy, M, N, K, ws, nbytes):
+    _lib.check(_lib.lib().nmi_gemm_fp8_w8a16(xd.data_ptr(), K, wd.data_ptr(), K, sd.data_ptr(), y.data_ptr(), ldy, M,
+                                             N, K, None if ws is None else ws.data_ptr(), nbytes,
+                                             torch.cuda.current_stream().cuda_stream), "gemm")
+
+
+# M around the tile rows and the 32-row strips of the second kernel, ragged N (one and two column
+# bands), one k tile per split and uneven splits.
+@pytest.mark.parametrize("M,N,K", [(512, 256, 320), (513, 300, 640), (576, 257, 704), (767, 40, 320), (1, 264, 320),
+                                   (97, 513, 1024)])
+@pytest.mark.parametrize("bm", [128, 192, 256])
+def test_tile_rows_and_splits(bm, M, N, K):
+    x, w, s = _case(M, N, K, bm + M + N + K)
+    xd, wd, sd = x_to_dev(x), w_to_dev(w), s_to_dev(s)
+    ref = oracle_bits(x, w, s)
+    L = _lib.lib()
+    _lib.tuning_set("gemm.tile", 24)
+    _lib.tuning_set("gemm.bm", bm)
+    _lib.tuning_set("gemm.sk", 2)                  # not the stream-K form, whose flags must be zero
+    unsplit = None
+    for sp in (1, 2, 5):
+        _lib.tuning_set("gemm.splits", sp)
+        need = L.nmi_linear_workspace_bytes(max(M, 512), N, K)
+        announce("gemm_split", bm, M, N, K, sp, need)
+        ws = torch.full((max(need, 256),), 255, dtype=torch.uint8, device=DEV)   # NaN where not written
+        ys = []
+        # contiguous y, y with an odd row stride and 2-byte offset, and a workspace of the
+        # flag region only
+        for ldy, off, nbytes in ((N, 0, need), (N + 3, 1, need), (N, 0, min(need, 65536))):
+            buf = torch.full((M, ldy), 5.0, dtype=torch.bfloat16, device=DEV)
+            _call(xd, wd, sd, buf[:, off:], ldy, M, N, K, ws, nbytes)
+            torch.cuda.synchronize()
+            ys.append(bits(buf[:, off:off + N]))
+            assert torch.all(buf[:, :off] == 5.0) and torch.all(buf[:, off + N:] == 5.0)
+        assert torch.all(ws[:min(need, 65536)] == 255), "flag region written"
+        assert_parity(ys[0], ref, f"bm={bm} splits={sp}", per_row_scales=True)
+        assert np.array_equal(ys[0], ys[1])
+        unsplit = ys[0] if unsplit is None else unsplit
+        assert np.array_equal(ys[2], unsplit), "without room for the partials: the unsplit sums"
+
+
+def test_automatic_split_in_the_mlp_block_and_a_graph():
+    """M = 520 at the model's sizes: down_proj (K = 12544) is split.  relu^2, the residual (in place
+    too) and graph replays give the composition's bytes; a workspace without room for the
+    partials is accepted and stays within the parity of another summation order."""
+    M, hidden, inter = 520, 3136, 12544
+    announce("gemm_split_mlp", M, hidden, inter)
+    L = _lib.lib()
+    assert L.nmi_linear_workspace_bytes(M, hidden, inter) > 65536
+    assert L.nmi_linear_workspace_needs_zero(M) == 0 and L.nmi_linear_workspace_needs_zero(511) == 1
+    up, ups = synth.make_weight(inter, hidden, 31, DEV)
+    dn, dns = synth.make_weight(hidden, inter, 32, DEV)
+    nw = torch.ones(hidden, device=DEV)
+    x = synth.make_act(M, hidden, 33, DEV)
+    h = ops.rmsnorm_bf16(x, nw)
+    u = ops.linear_fp8_w8a16(h, up, ups)
+    r = torch.relu(u)
+    want = x + ops.linear_fp8_w8a16(r * r, dn, dns)
+    got = ops.mlp_forward_fp8(x, nw, up, ups, dn, dns)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    xi = x.clone()
+    ops.mlp_forward_fp8(xi, nw, up, ups, dn, dns, out=xi)
+    assert torch.equal(xi.view(torch.int16), want.view(torch.int16)), "in place"
+    out = torch.empty_like(x)
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=stream):
+        ops.mlp_forward_fp8(x, nw, up, ups, dn, dns, out=out)
+        lin = ops.linear_fp8_w8a16(r * r, dn, dns)
+    for _ in range(3):
+        out.zero_()
+        lin.zero_()
+        ops.mlp_forward_fp8(x, nw, up, ups, dn, dns)          # eager work between replays
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+        assert torch.equal((x + lin).view(torch.int16), want.view(torch.int16))
+    need = L.nmi_mlp_workspace_bytes(M, hidden, inter)
+    least = need - (L.nmi_linear_workspace_bytes(M, hidden, inter) + 255) // 256 * 256
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    for nbytes, ok in ((need - 1, True), (least, True), (least - 1, False)):
+        rc = L.nmi_mlp_forward_fp8(x.data_ptr(), nw.data_ptr(), up.data_ptr(), ups.data_ptr(), dn.data_ptr(),
+                                   dns.data_ptr(), out.data_ptr(), M, hidden, inter, 1e-5, ws.data_ptr(), nbytes, None)
+        assert (rc == _lib.NMI_OK) == ok, (nbytes, rc)
+        torch.cuda.synchronize()
+        if ok:
+            d = (out.double() - want.double()).norm() / want.double().norm()
+            assert d < 2e-3, d                               # rounding flips of another float32 order

@@ -195,14 +195,13 @@ int nmi_gemv_chain_destroy(nmi_gemv_chain* chain);
  * and K on the current device; 0 when the selected kernel needs none (the GEMV, the skinny
  * kernels by default, which split K inside the workgroup only).  With the 4x4x4 kernel's K
  * split (s4.kg > 1): 64 KiB of arrival counters and the fp32 partials, s4.kg x M x total_n x 4
- * bytes (fewer K groups when K has fewer windows).  For 17 <= M < 512 (the short-prompt GEMM) a
- * 64 KiB region it leaves alone, then the fp32 partials of its K split (0 when the schedule does
- * not split K).  For M >= 512 likewise a 64 KiB flag region and the fp32 partial tiles of one
- * matrix's K split (at most one 256 x 256 tile per CU, 64 MiB; 0 when it is not split).  Every
+ * bytes (fewer K groups when K has fewer windows).  For M >= 17 (the GEMMs) a 64 KiB region they
+ * leave alone, then the fp32 partials of the K split (at most about one 256 x 256 tile per CU,
+ * 64 MiB; 0 when no kernel the call may take splits K).  Every
  * kernel leaves the first 64 KiB as it found it (zero at rest), so one zero-filled workspace
  * serves every M in turn. */
 size_t nmi_linear_workspace_bytes(int M, int64_t total_n, int K);
-/* 0 where a workspace for M rows may hold anything (the K split of M >= 512 writes its partials
+/* 0 where a workspace for M rows may hold anything (the K split from M = 512 writes its partials
  * before it reads them), 1 where it must start zero-filled. */
 int nmi_linear_workspace_needs_zero(int M);
 

@@ -78,10 +78,10 @@ struct FwdLayout {
 
 // The GEMMs' region (the K splits' partials, or the stream-K flags and partials where that form
 // is forced by tuning knob): the largest of the q, k, v (launched one by one below M = 512) and o
-// needs.  split = false: without the K split of M >= 512.
+// needs.  split = false: without the DMA-fed kernel's K split.
 size_t gemm_region(int M, int hidden, int QD, int KD, bool split) {
     if (choose_path(M) != Path::Gemm) return 0;
-    const auto need = split ? linear_workspace_bytes : linear_workspace_bytes_unsplit;
+    const auto need = split ? linear_workspace_bytes : linear_workspace_bytes_least;
     const size_t qkv = std::max(need(M, (int64_t)QD + 2 * (int64_t)KD, hidden),
                                 std::max(need(M, QD, hidden), need(M, KD, hidden)));
     return round256(std::max(qkv, need(M, hidden, QD)));

@@ -49,15 +49,17 @@ size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 // projection.
 bool norm_fused(int M, int hidden) { return gemv_fuses_norm(M, hidden); }
 
-// split = false leaves the GEMMs unsplit (no partial region): the allocation-free form, whose
-// buffers must fit a fixed array, and from M = 512 a caller's workspace without room for it
-size_t gemm_region(int M, int hidden, int inter, bool split) {
-    if (choose_path(M) != Path::Gemm || (!split && !gemm_workspace_has_flags(M))) return 0;
-    const auto need = split ? linear_workspace_bytes : linear_workspace_bytes_unsplit;
+// The GEMMs' region: kFull, kLeast without the DMA-fed kernel's K split (a caller's workspace
+// without room for it), kNone without any split (the allocation-free form, whose buffers must fit
+// a fixed array)
+enum class Region { kNone, kLeast, kFull };
+size_t gemm_region(int M, int hidden, int inter, Region split) {
+    if (choose_path(M) != Path::Gemm || (split == Region::kNone && !gemm_workspace_has_flags(M))) return 0;
+    const auto need = split == Region::kFull ? linear_workspace_bytes : linear_workspace_bytes_least;
     return round256(std::max(need(M, inter, hidden), need(M, hidden, inter)));
 }
 
-size_t mlp_bytes(int M, int hidden, int inter, bool split) {
+size_t mlp_bytes(int M, int hidden, int inter, Region split) {
     size_t b = gemm_region(M, hidden, inter, split) + round256((size_t)M * inter * 2);
     if (!norm_fused(M, hidden)) b += round256((size_t)M * hidden * 2);
     return b;
@@ -83,7 +85,7 @@ int nmi_rmsnorm_bf16(const void* x_bf16, const float* w, void* y_bf16, int M, in
 
 size_t nmi_mlp_workspace_bytes(int M, int hidden, int inter) {
     if (M < 1 || hidden < 16 || inter < 16) return 0;
-    return mlp_bytes(M, hidden, inter, true);
+    return mlp_bytes(M, hidden, inter, Region::kFull);
 }
 
 int nmi_mlp_forward_fp8(const void* input_bf16, const float* norm_w, const void* up_w_e4m3, const float* up_scale,
@@ -99,7 +101,7 @@ namespace nmi {
 
 size_t mlp_workspace_bytes(int M, int hidden, int inter, bool split) {
     if (M < 1 || hidden < 16 || inter < 16) return 0;
-    return mlp_bytes(M, hidden, inter, split);
+    return mlp_bytes(M, hidden, inter, split ? Region::kFull : Region::kNone);
 }
 
 int mlp_forward_fp8(const void* input_bf16, const float* norm_w, const void* up_w_e4m3, const float* up_scale,
@@ -117,14 +119,17 @@ int mlp_forward_fp8(const void* input_bf16, const float* norm_w, const void* up_
         return fail2(NMI_ERR_ALIGNMENT, fn, "input, norm_w and the weights must be 16-byte aligned");
     if (!aligned(up_scale, 4) || !aligned(down_scale, 4) || !aligned(out_bf16, 2))
         return fail2(NMI_ERR_ALIGNMENT, fn, "misaligned scale or output");
-    const size_t need = mlp_bytes(M, hidden, inter, split);
+    Region region = split ? Region::kFull : Region::kNone;
+    size_t need = mlp_bytes(M, hidden, inter, region);
     if (workspace) {
         if (!aligned(workspace, 16))
             return fail2(NMI_ERR_ALIGNMENT, fn, "workspace must be 16-byte aligned");
-        if (workspace_bytes < need && M >= 512) split = false;      // room enough without the K split?
-        const size_t least = split ? need : mlp_bytes(M, hidden, inter, false);
-        if (workspace_bytes < least) {
-            set_last_error("%s: workspace of %zu bytes, %zu needed", fn, workspace_bytes, least);
+        if (split && workspace_bytes < need) {
+            region = Region::kLeast;
+            need = mlp_bytes(M, hidden, inter, region);
+        }
+        if (workspace_bytes < need) {
+            set_last_error("%s: workspace of %zu bytes, %zu needed", fn, workspace_bytes, need);
             return NMI_ERR_WORKSPACE;
         }
     } else {
@@ -135,7 +140,7 @@ int mlp_forward_fp8(const void* input_bf16, const float* norm_w, const void* up_
     const uint16_t* in = static_cast<const uint16_t*>(input_bf16);
     uint16_t* out = static_cast<uint16_t*>(out_bf16);
     char* base = static_cast<char*>(workspace);
-    const size_t gws = gemm_region(M, hidden, inter, split);
+    const size_t gws = gemm_region(M, hidden, inter, region);
     void* gemm_ws = gws ? base : nullptr;        // the GEMMs' stream-K region or K-split partials
     uint16_t* act = reinterpret_cast<uint16_t*>(base + gws);
     const Norm norm{norm_w, eps};

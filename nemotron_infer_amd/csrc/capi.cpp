@@ -141,15 +141,16 @@ namespace nmi {
 size_t linear_workspace_bytes(int M, int64_t total_n, int K) {
     if (M < 1 || K < 16 || K % 16 != 0 || total_n < 1) return 0;
     const int t = tuning().gemm_tile;
-    if (M > 16 && M < 512)                            // the short-prompt kernel's K-split partials
-        return (t == 0 || t == 2) ? gemm_short_workspace_bytes(M, (int)std::min<int64_t>(total_n, 1 << 30), K) : 0;
-    if (M > 16)                                       // the GEMM's stream-K flags and partials, or its K split's
-        return std::max(gemm_workspace_bytes(M), (t == 0 || t == 24) ? gemm_split_workspace_bytes(M, total_n, K) : 0);
-    return 0;                                         // the GEMV and skinny kernels use none
+    if (M <= 16) return 0;                            // the GEMV and skinny kernels use none
+    return std::max(linear_workspace_bytes_least(M, total_n, K),
+                    (t == 0 || t == 24) ? gemm_split_workspace_bytes(M, total_n, K) : 0);
 }
 
-size_t linear_workspace_bytes_unsplit(int M, int64_t total_n, int K) {
-    return M < 512 ? linear_workspace_bytes(M, total_n, K) : gemm_workspace_bytes(M);
+size_t linear_workspace_bytes_least(int M, int64_t total_n, int K) {
+    if (M <= 16 || K < 16 || K % 16 != 0 || total_n < 1) return 0;
+    if (M >= 512) return gemm_workspace_bytes(M);     // stream-K flags and partials
+    const int t = tuning().gemm_tile;                 // the short-prompt kernel's K-split partials
+    return (t == 0 || t == 2) ? gemm_short_workspace_bytes(M, (int)std::min<int64_t>(total_n, 1 << 30), K) : 0;
 }
 
 bool gemm_workspace_has_flags(int M) { return M >= 512 && choose_path(M) == Path::Gemm && gemm_workspace_bytes(M) > 0; }

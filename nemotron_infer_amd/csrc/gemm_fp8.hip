@@ -514,7 +514,7 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_w8a16_dma_kernel(const GemmAr
     // BM = 256: 256 x 256 tiles, each wave 128 x 128 (TM = 4 blocks of 32 x rows); BM = 192 and
     // 128: 192 x 256 and 128 x 256 tiles, each wave 96 or 64 x 128 (TM = 3, 2), not stream-K
     static_assert(BM == 256 || ((BM == 192 || BM == 128) && !SK), "tile rows");
-    static_assert(!SPLIT || (!SK && !GROUPED), "K split: one matrix, data-parallel form");
+    static_assert(!SPLIT || !SK, "K split of the data-parallel form");
     constexpr int NT = 256, BK = kBK, W_STAGE = 256 * 64, TN = 4, TM = BM / 64;
     constexpr int XI = BM / 32;                     // x DMA instructions per wave and k tile
     constexpr int ND = 4 + XI;                      // DMA instructions per wave and k tile
@@ -1155,15 +1155,21 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_w8a16_dma_kernel(const GemmAr
 // One workgroup per 32-row strip of a tile; a thread holds the partials' 16-byte pieces
 // of one lane of the main kernel's waves (so the loads are whole 1 KiB runs), rounds v into a
 // bf16 copy of the strip in LDS, and stores 16-byte row pieces as the main kernel's epilogue does.
-template <int BM>
+template <int BM, bool GROUPED>
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const GemmArgs a) {
     constexpr int TM = BM / 64, STRIPS = BM / 32, PITCH = 520;
     __shared__ __attribute__((aligned(16))) uint8_t sm[32 * PITCH];
-    const GemmArgs::Group& G = a.grp[0];
     const int r = (int)blockIdx.x / STRIPS, strip = (int)blockIdx.x % STRIPS;
-    int tm, tn;
+    int tm, tn, gi = 0;
     tile_coords(r, a.tiles_m, a.tiles_n, a.gh, tm, tn);
-    const int m0 = tm * BM + 32 * strip, n0 = tn * 256;
+    if constexpr (GROUPED) {
+#pragma unroll
+        for (int i = 1; i < kMaxGroups; ++i)
+            if (i < a.ngroups && tn >= a.grp[i].tn_begin) gi = i;
+        gi = __builtin_amdgcn_readfirstlane(gi);
+    }
+    const GemmArgs::Group& G = a.grp[gi];
+    const int m0 = tm * BM + 32 * strip, n0 = (tn - G.tn_begin) * 256;
     if (m0 >= a.M) return;                          // uniform: a strip past the last row
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int h = lane >> 5, l32 = lane & 31;
@@ -1282,23 +1288,33 @@ bool dma_supported(const uint16_t* x, int64_t ldx, const uint8_t* W, int64_t ldw
 
 constexpr int dma_lds_bytes(int bm) { return kDmaStages * (256 * 64 + bm * 128); }
 
-// The kernel without stream-K for `bm` tile rows, one matrix or several, K whole or split (one
-// matrix only).
+// The kernel without stream-K for `bm` tile rows, one matrix or several, K whole or split.
 using DmaKernel = void (*)(GemmArgs);
 DmaKernel dma_kernel(int bm, bool grouped, bool split) {
     switch (bm) {
         case 128:
-            return split     ? &gemm_fp8_w8a16_dma_kernel<false, false, 128, true>
-                   : grouped ? &gemm_fp8_w8a16_dma_kernel<false, true, 128>
-                             : &gemm_fp8_w8a16_dma_kernel<false, false, 128>;
+            if (split)
+                return grouped ? &gemm_fp8_w8a16_dma_kernel<false, true, 128, true>
+                               : &gemm_fp8_w8a16_dma_kernel<false, false, 128, true>;
+            return grouped ? &gemm_fp8_w8a16_dma_kernel<false, true, 128> : &gemm_fp8_w8a16_dma_kernel<false, false, 128>;
         case 192:
-            return split     ? &gemm_fp8_w8a16_dma_kernel<false, false, 192, true>
-                   : grouped ? &gemm_fp8_w8a16_dma_kernel<false, true, 192>
-                             : &gemm_fp8_w8a16_dma_kernel<false, false, 192>;
+            if (split)
+                return grouped ? &gemm_fp8_w8a16_dma_kernel<false, true, 192, true>
+                               : &gemm_fp8_w8a16_dma_kernel<false, false, 192, true>;
+            return grouped ? &gemm_fp8_w8a16_dma_kernel<false, true, 192> : &gemm_fp8_w8a16_dma_kernel<false, false, 192>;
         default:
-            return split     ? &gemm_fp8_w8a16_dma_kernel<false, false, 256, true>
-                   : grouped ? &gemm_fp8_w8a16_dma_kernel<false, true, 256>
-                             : &gemm_fp8_w8a16_dma_kernel<false, false, 256>;
+            if (split)
+                return grouped ? &gemm_fp8_w8a16_dma_kernel<false, true, 256, true>
+                               : &gemm_fp8_w8a16_dma_kernel<false, false, 256, true>;
+            return grouped ? &gemm_fp8_w8a16_dma_kernel<false, true, 256> : &gemm_fp8_w8a16_dma_kernel<false, false, 256>;
+    }
+}
+// The second kernel of a split.
+DmaKernel dma_reduce_kernel(int bm, bool grouped) {
+    switch (bm) {
+        case 128: return grouped ? &gemm_split_reduce_kernel<128, true> : &gemm_split_reduce_kernel<128, false>;
+        case 192: return grouped ? &gemm_split_reduce_kernel<192, true> : &gemm_split_reduce_kernel<192, false>;
+        default: return grouped ? &gemm_split_reduce_kernel<256, true> : &gemm_split_reduce_kernel<256, false>;
     }
 }
 
@@ -1306,6 +1322,7 @@ DmaKernel dma_kernel(int bm, bool grouped, bool split) {
 // splits > 1, K cut into that many runs per tile.
 struct DmaPlan {
     int bm, tiles, splits;
+    double us;                                      // the modelled time
     size_t part_bytes() const { return splits > 1 ? (size_t)tiles * splits * bm * 256 * sizeof(float) : 0; }
 };
 
@@ -1314,15 +1331,16 @@ struct DmaPlan {
 // CUs in use (they share the power budget: the clock falls), fitted to a sweep of M = 512 .. 4096
 // on the model's projections (us, MI355X; the fit is within 5% of most of them):
 //   rounds * (start + KT * fixed) + KT * U / CUs * shared,   KT = k tiles of one workgroup,
-// and a split adds its second kernel.  K is split only from 4096 up and into one round of
-// workgroups (below, no split of any projection was faster than its best unsplit tiles) and only
-// for a modelled gain of 8%: with most CUs busy either way the power budget decides (2048 x 3136 x
+// and a split adds its second kernel.  K is split into one round of workgroups: one matrix where
+// K >= 4096 (below, from M = 512, no split of any projection was faster than its best unsplit
+// tiles, and a row's sums stay the same in a larger batch or a group), matrices sharing x where
+// M < 512 (dma_plan_ws); and only for a modelled gain of 8%: with most CUs busy either way the power budget decides (2048 x 3136 x
 // 12544, 256-row tiles split in two against whole 128-row tiles: 143 against 148 us on one box, the
 // MLP block 329 against 318 us on another).
 // Examples (us): 777 x 12544 x 3136 256 / 192 / 128-row tiles 67.5 / 59.6 / 75.9; 2048 x 17504 x
 // 3136 209 / 180 / 209; 512 x 3136 x 12544 in 128-row tiles, splits of 1 / 2 / 3 / 4: 113 / 70 /
 // 55 / 50; 1000 x 3136 x 7680 1 / 2: 74 / 57.  Tuning knobs: gemm.bm forces the tile rows, gemm.splits the split (1: none).
-DmaPlan dma_plan(int M, int tiles_n, int K, bool may_split) {
+DmaPlan dma_plan(int M, int tiles_n, int K, int ng, bool may_split) {
     struct Cost { int bm; double start, fixed, shared; };
     constexpr Cost kCost[] = {{256, 12.0, 0.857, 0.408}, {192, 10.0, 0.61, 0.41}, {128, 8.6, 0.395, 0.337}};
     constexpr double kReduce = 5.0, kReducePerByte = 0.09e-6;
@@ -1339,18 +1357,27 @@ DmaPlan dma_plan(int M, int tiles_n, int K, bool may_split) {
             const bool forced = t.gemm_splits > 0 && sp == t.gemm_splits;
             if (sp > 1) {
                 if (!may_split || sp > KT || T * sp > (int64_t)4 * G) break;
-                if (t.gemm_splits > 0 ? !forced : (K < kMinSplitK || T * sp > G)) continue;
+                if (t.gemm_splits > 0 ? !forced : ((ng == 1 && K < kMinSplitK) || T * sp > G)) continue;
             }
-            const DmaPlan p{c.bm, (int)T, sp};
+            DmaPlan p{c.bm, (int)T, sp, 0.0};
             const int64_t rounds = (T * sp + G - 1) / G;
             const double kt = (double)((KT + sp - 1) / sp);
             double us = rounds * (c.start + kt * c.fixed) + kt * c.shared * (double)(T * sp) / G;
             if (sp > 1) us = (us + kReduce + (double)p.part_bytes() * kReducePerByte) * kSplitMargin;
+            p.us = us;
             if (forced && sp > 1) us -= 1e9;        // a forced split wins over its unsplit forms
             if (best.bm == 0 || us < best_us) best = p, best_us = us;
         }
     }
     return best;
+}
+
+// dma_plan for ng matrices sharing x and a workspace of ws_bytes: unsplit where the partials do not
+// fit, and for groups from M = 512.
+DmaPlan dma_plan_ws(int M, int tiles_n, int K, int ng, size_t ws_bytes) {
+    DmaPlan p = dma_plan(M, tiles_n, K, ng, ws_bytes > 0 && (ng == 1 || M < 512));
+    if (p.splits > 1 && ws_bytes < kSkFlagBytes + p.part_bytes()) p = dma_plan(M, tiles_n, K, ng, false);
+    return p;
 }
 
 // The DMA-fed kernel as dma_plan says, or under the knobs gemm.sk = 1 / gemm.bm = 256 in 256-row
@@ -1374,6 +1401,7 @@ hipError_t launch_dma_groups(const uint16_t* x, int64_t ldx, const GemvGroup* g,
             set(dma_kernel(bm, false, false), dma_lds_bytes(bm));
             set(dma_kernel(bm, true, false), dma_lds_bytes(bm));
             set(dma_kernel(bm, false, true), dma_lds_bytes(bm));
+            set(dma_kernel(bm, true, true), dma_lds_bytes(bm));
         }
         return e;
     }();
@@ -1405,8 +1433,7 @@ hipError_t launch_dma_groups(const uint16_t* x, int64_t ldx, const GemvGroup* g,
     const int gh_knob = tuning().gemm_gh;
     // gemm.sk = 1 and gemm.bm = 256 keep the 256-row tiles below (stream-K where it is wanted)
     if (tuning().gemm_sk != 1 && (tuning().gemm_bm != 256 || tuning().gemm_splits > 1)) {
-        DmaPlan p = dma_plan(M, tn, K, ng == 1 && ws != nullptr);
-        if (p.splits > 1 && ws_bytes < kSkFlagBytes + p.part_bytes()) p = dma_plan(M, tn, K, false);
+        const DmaPlan p = dma_plan_ws(M, tn, K, ng, ws ? ws_bytes : 0);
         a.tiles_m = (M + p.bm - 1) / p.bm;
         a.gh = gh_knob > 0 ? std::min(gh_knob, a.tiles_m) : a.tiles_m;
         a.splits = p.splits;
@@ -1416,10 +1443,7 @@ hipError_t launch_dma_groups(const uint16_t* x, int64_t ldx, const GemvGroup* g,
         hipLaunchKernelGGL(kernel, dim3(8 * a.per_xcd), dim3(256), dma_lds_bytes(p.bm), stream, a);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess || p.splits == 1) return e;
-        const auto reduce = p.bm == 256   ? &gemm_split_reduce_kernel<256>
-                            : p.bm == 192 ? &gemm_split_reduce_kernel<192>
-                                          : &gemm_split_reduce_kernel<128>;
-        hipLaunchKernelGGL(reduce, dim3((unsigned)(p.tiles * (p.bm / 32))), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL(dma_reduce_kernel(p.bm, grouped), dim3((unsigned)(p.tiles * (p.bm / 32))), dim3(256), 0, stream, a);
         return hipGetLastError();
     }
     const bool fits = ws && ws_bytes >= kSkFlagBytes + (size_t)G * kDmaPartialBytes && G % 8 == 0 &&
@@ -1480,20 +1504,59 @@ size_t gemm_workspace_bytes(int M) {
     return kSkFlagBytes + (size_t)device_info().num_cu * kDmaPartialBytes;
 }
 
-// The K split's partial tiles for one matrix of N rows (after the 64 KiB flag region, which it
-// leaves alone); 0 where dma_plan does not split.
+// The K split's partial tiles for N rows of one matrix, or of up to kMaxGroups below M = 512
+// (after the 64 KiB flag region, which it leaves alone); 0 where dma_plan does not split.  Groups
+// have up to kMaxGroups - 1 more column bands than one matrix of their rows.
 size_t gemm_split_workspace_bytes(int M, int64_t N, int K) {
-    if (M < 512 || K % kBK != 0 || N > (1 << 30) || tuning().gemm_sk == 1) return 0;
-    const DmaPlan p = dma_plan(M, (int)((N + 255) / 256), K, true);
-    return p.splits > 1 ? kSkFlagBytes + p.part_bytes() : 0;
+    if (M < 1 || K % kBK != 0 || N > (1 << 30) || tuning().gemm_sk == 1) return 0;
+    size_t bytes = 0;
+    for (int more = 0; more < (M < 512 ? kMaxGroups : 1); ++more) {
+        for (int ng = 1; ng <= (M < 512 ? 2 : 1); ++ng) {
+            const DmaPlan p = dma_plan(M, (int)((N + 255) / 256) + more, K, ng, true);
+            if (p.splits > 1) bytes = std::max(bytes, kSkFlagBytes + p.part_bytes());
+        }
+    }
+    return bytes;
 }
 
+namespace {
+// The DMA-fed kernel for one matrix at M < 512, by its modelled time against the short-prompt
+// kernel's: their crossing lies between M = 100 (N = 17504) and about 300 (N = 3136).  Measured
+// (us, short-prompt / DMA-fed): 100 x 17504 x 3136 35.6 / 34.6, 200 x 17504 x 3136 66.8 / 36.1, 300
+// x 12544 x 3136 68.5 / 35.5, 300 x 3136 x 12544 44.2 / 40.0, 500 x 3136 x 7680 39.8 / 36.5; but 200 x
+// 3136 x 12544 33.7 / 34.4, 256 x 7168 x 3136 24.8 / 24.9.  The short kernel's own knobs keep it.
+double dma_short_m_us(int M, int N, int K, size_t ws_bytes) {
+    return dma_plan_ws(M, (N + 255) / 256, K, 1, ws_bytes).us;
+}
+bool dma_beats_short(int M, int N, int K, size_t ws_bytes) {
+    const Tuning& t = tuning();
+    if (M <= kShortOnlyM || t.gemm_short != 0 || t.gemm_splits > 1 || t.gemm_sk == 1 || t.gemm_bm == 256) return false;
+    return dma_short_m_us(M, N, K, ws_bytes) < gemm_short_us(M, N, K, ws_bytes);
+}
+}  // namespace
+
 // A grouped GEMM (matrices sharing x) as one launch of the DMA-fed kernel where it takes every
-// matrix (M >= 512, automatic tile choice); otherwise one launch per matrix.
+// matrix (automatic tile choice, M >= 512 or where that is the least modelled time); otherwise one
+// launch per matrix.  Measured (q | k | v, 5120 + 1024 + 1024 rows of K = 3136): see the attention
+// block's figures in attention.cpp.
 hipError_t launch_gemm_grouped(const uint16_t* x, int64_t ldx, int M, int K, const GemvGroup* g, int ng,
                                hipStream_t stream, void* ws, size_t ws_bytes) {
-    bool one = ng > 1 && M >= 512 && tuning().gemm_tile == 0;
+    const Tuning& t = tuning();
+    bool one = ng > 1 && t.gemm_tile == 0;
     for (int i = 0; one && i < ng; ++i) one = dma_supported(x, ldx, g[i].W, g[i].ldw, M, g[i].N, K);
+    const bool forced = t.gemm_bm != 0 && t.gemm_splits > 1;
+    if (one && M < 512 && !forced) {
+        one = t.gemm_short == 0 && t.gemm_splits <= 1 && t.gemm_sk != 1 && t.gemm_bm != 256;
+        const size_t wsb = ws ? ws_bytes : 0;
+        int tn = 0;
+        double separate = 0;
+        for (int i = 0; one && i < ng; ++i) {
+            tn += (g[i].N + 255) / 256;
+            const double us = gemm_short_us(M, g[i].N, K, wsb);
+            separate += M <= kShortOnlyM ? us : std::min(us, dma_short_m_us(M, g[i].N, K, wsb));
+        }
+        one = one && dma_plan_ws(M, tn, K, ng, wsb).us < separate;
+    }
     if (one) return launch_dma_groups(x, ldx, g, ng, M, K, stream, ws, ws_bytes);
     hipError_t e = hipSuccess;
     for (int i = 0; i < ng && e == hipSuccess; ++i)
@@ -1507,15 +1570,17 @@ hipError_t launch_gemm(const uint16_t* x, int64_t ldx, const uint8_t* W, int64_t
                        hipStream_t stream, const Epi& epi, void* ws, size_t ws_bytes) {
     int tile = tuning().gemm_tile;
     if (tile != 1 && tile != 2 && tile != 20 && tile != 21 && tile != 24) {
-        // M < 512: the short-prompt kernel (gemm_short.hip) where it can take the operands, else
-        // the 128 x 128 16 x 16 x 32 kernel; otherwise the DMA-fed 256 x 256 kernel where it can
+        // M < 512: the short-prompt kernel (gemm_short.hip) where it can take the operands and is
+        // the faster one (dma_beats_short), else
+        // the 128 x 128 16 x 16 x 32 kernel; otherwise the DMA-fed kernel where it can
         // take the operands, else the 8-wave 32 x 32 kernel with 256 x 256 tiles where they fill
         // at least 3/4 of the CUs, 256 x 128 below that.  (Measured on MI355X, config 3; the other
         // tile shapes and schedules tried -- 16 x 16 x 32 MFMA at 256-wide tiles, 64-bit LDS reads,
         // 4-wave forms, raised issue priority -- were slower.)
         const DeviceInfo& dev = device_info();
         const int64_t big = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
-        if (M < 512) tile = gemm_short_supported(x, ldx, W, ldw, M, N, K) ? 2 : 1;
+        if (M < 512 && !(dma_supported(x, ldx, W, ldw, M, N, K) && dma_beats_short(M, N, K, ws ? ws_bytes : 0)))
+            tile = gemm_short_supported(x, ldx, W, ldw, M, N, K) ? 2 : 1;
         else if (dma_supported(x, ldx, W, ldw, M, N, K)) tile = 24;
         else tile = (4 * big >= 3 * (int64_t)dev.num_cu) ? 20 : 21;
     }

@@ -381,6 +381,21 @@ int gemm_short_splits(int M, int N, int K) {
     return std::max(1, std::min(want, std::min(by_k, by_bytes)));
 }
 
+// Fitted to a sweep of M = 100 .. 500 on the model's projections above M = 64 (within 10% of most):
+// rounds of one workgroup per CU, a k tile 0.66 us, 0.58 where K is split, 4 us to start and end
+// one, 6 us for the second kernel.  M <= 64: two launches of about 7 us whatever the shape.
+double gemm_short_us(int M, int N, int K, size_t ws_bytes) {
+    if (M <= 64) return 14.0;
+    const ShortCfg& c = kForms[short_form(M, N)];
+    const int KT = std::max(1, K / kBK), cu = device_info().num_cu;
+    int splits = gemm_short_splits(M, N, K);
+    if (splits > 1 && ws_bytes < kFlagRegion + (size_t)splits * M * N * sizeof(float)) splits = 1;
+    const int64_t units = (int64_t)((N + c.bn() - 1) / c.bn()) * ((M + c.bm() - 1) / c.bm()) * splits;
+    const double kt = (double)((KT + splits - 1) / splits);
+    const double rounds = (double)((units + cu - 1) / cu);
+    return splits > 1 ? rounds * (kt * 0.58 + 4.0) + 6.0 : rounds * (kt * 0.66 + 4.0);
+}
+
 // Enough for any N' <= N (grouped launches share one workspace): splits x N' is at most
 // min(splits by k and bytes) x N, and the one-round limit keeps it below the rows one round of
 // workgroups covers.

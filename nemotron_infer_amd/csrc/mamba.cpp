@@ -72,10 +72,10 @@ struct FwdLayout {
 
 // The GEMMs' region (the K splits' partials, or the stream-K flags and partials where that form
 // is forced by tuning knob): the larger of the in_proj and out_proj needs.  split = false: without
-// the K split of M >= 512.
+// the DMA-fed kernel's K split.
 size_t gemm_region(int M, int hidden, const MambaDims& d, bool split) {
     if (choose_path(M) != Path::Gemm) return 0;
-    const auto need = split ? linear_workspace_bytes : linear_workspace_bytes_unsplit;
+    const auto need = split ? linear_workspace_bytes : linear_workspace_bytes_least;
     return round256(std::max(need(M, d.proj, hidden), need(M, hidden, d.inter)));
 }
 

@@ -202,22 +202,25 @@ hipError_t launch_gemv_stream_chain(const StreamPhase* tab, const int* wave_step
 // one tile per workgroup.  launch_sk_flags_clear zeroes the flag region (one small kernel, safe
 // under graph capture).
 size_t gemm_workspace_bytes(int M);
-// Workspace of the DMA-fed kernel's K split (M >= 512, one matrix of N rows; 0: not split): float32
-// partial tiles after the flag region, no initialisation needed.
+// Workspace of the DMA-fed kernel's K split (N rows in all; 0: not split): float32 partial tiles
+// after the flag region, no initialisation needed.
 size_t gemm_split_workspace_bytes(int M, int64_t N, int K);
 // Short prompts (17 <= M < 512; gemm_short.hip): the pipelined 128-row-tile kernel, with K split
 // between workgroups when a workspace of gemm_short_workspace_bytes(M, N, K) bytes is given
 // (float32 partials, no initialisation needed; 0: the schedule does not split).
 bool gemm_short_supported(const uint16_t* x, int64_t ldx, const uint8_t* W, int64_t ldw, int M, int N, int K);
 int gemm_short_splits(int M, int N, int K);
+// Its modelled time (us) with a workspace of ws_bytes (0: none).
+double gemm_short_us(int M, int N, int K, size_t ws_bytes);
+constexpr int kShortOnlyM = 64;   // up to this M one matrix always takes the short-prompt kernel
 size_t gemm_short_workspace_bytes(int M, int N, int K);
 // Workspace bytes a linear of M rows over matrices of total_n rows and K columns can use
 // (nmi_linear_workspace_bytes); whether that region holds stream-K flags that must start at zero
 // (launch_sk_flags_clear) -- the short-prompt kernel's partials need no initialisation.
 size_t linear_workspace_bytes(int M, int64_t total_n, int K);
 bool gemm_workspace_has_flags(int M);
-// The same without the K split of M >= 512, whose region a caller may leave out.
-size_t linear_workspace_bytes_unsplit(int M, int64_t total_n, int K);
+// The same without the DMA-fed kernel's K split, whose region a caller may leave out.
+size_t linear_workspace_bytes_least(int M, int64_t total_n, int K);
 // The fp8 MLP block (block.cpp) behind nmi_mlp_forward_fp8 (split = true) and its allocation-free
 // form (split = false: the short-prompt GEMMs run unsplit, so the workspace has no partial
 // region); fn names the entry point in error messages.

@@ -117,3 +117,63 @@ def test_automatic_split_in_the_mlp_block_and_a_graph():
         if ok:
             d = (out.double() - want.double()).norm() / want.double().norm()
             assert d < 2e-3, d                               # rounding flips of another float32 order
+
+
+# The choice between the short-prompt and the DMA-fed kernel at M < 512 (one matrix, and matrices
+# sharing x), on both sides of it: with a workspace, without one, and with one too small.
+@pytest.mark.parametrize("M", [17, 64, 65, 130, 300, 511])
+@pytest.mark.parametrize("Ns,K", [((17500,), 320), ((1000, 260, 130), 1024), ((300,), 5120)])
+def test_below_512_rows(M, Ns, K):
+    announce("gemm_below_512", M, Ns, K)
+    cases = [_case(M, N, K, 13 * i + M + N + K) for i, N in enumerate(Ns)]
+    x = cases[0][0]
+    xd = x_to_dev(x)
+    wd = [(w_to_dev(w), s_to_dev(s)) for _, w, s in cases]
+    L = _lib.lib()
+    need = L.nmi_linear_workspace_bytes(M, sum(Ns), K)
+    ws = torch.full((max(need, 256),), 255, dtype=torch.uint8, device=DEV)
+    refs = [oracle_bits(x, w, s) for _, w, s in cases]
+    arr = (_lib.LinearGroup * len(Ns))()
+    for nbytes in (need, min(need, 65536), 0):
+        ys = [torch.full((M, N), 5.0, dtype=torch.bfloat16, device=DEV) for N in Ns]
+        for i, ((w, s), y) in enumerate(zip(wd, ys)):
+            arr[i] = _lib.LinearGroup(w.data_ptr(), w.stride(0), s.data_ptr(), y.data_ptr(), y.stride(0), w.shape[0])
+        _lib.check(L.nmi_linear_fp8_w8a16_grouped(xd.data_ptr(), K, M, K, arr, len(Ns),
+                                                  ws.data_ptr() if nbytes else None, nbytes, None), "grouped")
+        torch.cuda.synchronize()
+        assert torch.all(ws[:min(need, 65536)] == 255), "flag region written"
+        for i, (y, ref) in enumerate(zip(ys, refs)):
+            assert_parity(bits(y), ref, f"M={M} group {i} ws={nbytes}", per_row_scales=True)
+
+
+# Groups of ragged column bands with K split in every tile height.
+@pytest.mark.parametrize("bm", [128, 192, 256])
+def test_grouped_split_tile_rows(bm):
+    M, Ns, K = 200, (300, 40, 257), 640
+    announce("gemm_grouped_split", bm, M, Ns, K)
+    cases = [_case(M, N, K, 17 * i + bm + N) for i, N in enumerate(Ns)]
+    xd = x_to_dev(cases[0][0])
+    wd = [(w_to_dev(w), s_to_dev(s)) for _, w, s in cases]
+    refs = [oracle_bits(cases[0][0], w, s) for _, w, s in cases]
+    _lib.tuning_set("gemm.sk", 2)
+    _lib.tuning_set("gemm.bm", bm)
+    _lib.tuning_set("gemm.splits", 3)
+    L = _lib.lib()
+    total = sum(Ns)
+    need = L.nmi_linear_workspace_bytes(M, total, K)
+    assert need > 0
+    ws = torch.full((need,), 255, dtype=torch.uint8, device=DEV)
+    ybig = torch.full((M, total + 3), 5.0, dtype=torch.bfloat16, device=DEV)
+    offs = np.cumsum((0,) + Ns)
+    arr = (_lib.LinearGroup * len(Ns))()
+    for i, (w, s) in enumerate(wd):
+        y = ybig[:, offs[i]:offs[i + 1]]
+        arr[i] = _lib.LinearGroup(w.data_ptr(), w.stride(0), s.data_ptr(), y.data_ptr(), y.stride(0), w.shape[0])
+    for split in (3, 0):
+        _lib.tuning_set("gemm.splits", split)
+        ybig[:, :total] = 5.0
+        _lib.check(L.nmi_linear_fp8_w8a16_grouped(xd.data_ptr(), K, M, K, arr, len(Ns), ws.data_ptr(), need, None), "g")
+        torch.cuda.synchronize()
+        for i, ref in enumerate(refs):
+            assert_parity(bits(ybig[:, offs[i]:offs[i + 1]]), ref, f"bm={bm} group {i}", per_row_scales=True)
+        assert torch.all(ybig[:, total:] == 5.0)

@@ -386,6 +386,8 @@ int nmi_attn_forward_fp8(const void* input_bf16, const float* norm_w, const void
  * row 0 only; this entry computes every row (the linears dispatch on M = batch).
  * workspace: nmi_mamba_decode_workspace_bytes(batch, hidden, n_heads, head_dim, n_groups,
  * d_state) bytes, 16-byte aligned, no initialisation; NULL takes it from the bump allocator.
+ * From batch 17 the size includes the projections' K-split partials, in its last part: a workspace
+ * without room for them is accepted and the projections run unsplit.
  */
 /*
  * The mixer of the Mamba-2 block at decode, between its projections (replaces the op calls

@@ -177,3 +177,49 @@ def test_grouped_split_tile_rows(bm):
         for i, ref in enumerate(refs):
             assert_parity(bits(ybig[:, offs[i]:offs[i + 1]]), ref, f"bm={bm} group {i}", per_row_scales=True)
         assert torch.all(ybig[:, total:] == 5.0)
+
+
+@pytest.mark.parametrize("batch", [16, 17, 33])
+def test_mamba_decode_batch_workspace(batch):
+    """The Mamba-2 decode block where its projections turn into GEMMs (batch 17): with the whole
+    workspace and without the part for the K split (the older size) it stays within the flips of
+    another float32 order of the composition of the library's calls; states the same bytes."""
+    H, P, G, hidden = 96, 80, 8, 3136
+    inter, conv_dim = H * P, H * P + 2 * G * 128
+    announce("mamba_decode_batch_ws", batch)
+    g = torch.Generator(device=DEV).manual_seed(50 + batch)
+    f = {"device": DEV, "generator": g}
+    iw, isc = synth.make_weight(inter + conv_dim + H, hidden, 61, DEV)
+    ow, osc = synth.make_weight(hidden, inter, 62, DEV)
+    prm = [0.3 * torch.randn((conv_dim, 4), **f), 0.1 * torch.randn(conv_dim, **f), torch.rand(H, **f),
+           torch.randn(H, **f), 0.5 * torch.randn(H, **f), 1.0 + 0.1 * torch.randn(inter, **f)]
+    nw = torch.ones(hidden, device=DEV)
+    x = synth.make_act(batch, hidden, 63, DEV)
+    cs = torch.randn((batch, conv_dim, 3), **f)
+    ss = 0.1 * torch.randn((batch, H, P, 128), **f)
+    h = ops.rmsnorm_bf16(x, nw)
+    c0, s0 = cs.clone(), ss.clone()
+    proj = ops.linear_fp8_w8a16(h, iw, isc)
+    _, gg = ops.mamba_mixer_decode(proj, *prm, c0, s0, H, P, G)
+    want = x + ops.linear_fp8_w8a16(gg, ow, osc)
+    L = _lib.lib()
+    need = L.nmi_mamba_decode_workspace_bytes(batch, hidden, H, P, G, 128)
+    r256 = lambda b: (b + 255) // 256 * 256  # noqa: E731
+    least = r256(batch * 17504 * 2) + 2 * r256(batch * inter * 2) + r256(batch * hidden * 2)
+    assert need >= least and (need > least) == (batch > 16)
+    ws = torch.full((need,), 255, dtype=torch.uint8, device=DEV)
+    for nbytes in (need, least, least - 1):
+        c1, s1, out = cs.clone(), ss.clone(), torch.empty_like(x)
+        rc = L.nmi_mamba_decode_fp8(x.data_ptr(), nw.data_ptr(), iw.data_ptr(), isc.data_ptr(),
+                                    *[t.data_ptr() for t in prm], ow.data_ptr(), osc.data_ptr(), c1.data_ptr(),
+                                    s1.data_ptr(), out.data_ptr(), batch, hidden, H, P, G, 128, 4, 1e-5, ws.data_ptr(),
+                                    nbytes, None)
+        assert (rc == _lib.NMI_OK) == (nbytes >= least), (nbytes, rc)
+        torch.cuda.synchronize()
+        if nbytes == need:
+            assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+            assert torch.equal(c1, c0) and torch.equal(s1, s0)
+        elif nbytes == least:
+            # a few flipped roundings (2^-9 relative each) among the block's values
+            assert (out.double() - want.double()).norm() / want.double().norm() < 2e-3
+            assert (s1 - s0).norm() / s0.norm() < 1e-3

@@ -136,7 +136,8 @@ int nmi_sdpa_prefill_bf16(const void* q_bf16, int64_t ldq, const void* k_bf16, i
     const hipError_t e = launch_sdpa_prefill(static_cast<const uint16_t*>(q_bf16), ldq,
                                              static_cast<const uint16_t*>(k_bf16), ldk,
                                              static_cast<const uint16_t*>(v_bf16), ldv, static_cast<uint16_t*>(o_bf16),
-                                             ldo, S, n_heads, n_kv_heads, static_cast<hipStream_t>(stream));
+                                             ldo, S, n_heads, n_kv_heads, nullptr, nullptr, 0,
+                                             static_cast<hipStream_t>(stream));
     return hip_status(e, fn);
 }
 
@@ -216,11 +217,10 @@ int nmi_attn_forward_fp8(const void* input_bf16, const float* norm_w, const void
         if (e == hipSuccess) e = dispatch_linear(normed, hidden, S, hidden, qkv, 3, gemm_ws, gws, st);
     }
     if (e != hipSuccess) return hip_status(e, fn);
-    // the caches, causal attention
-    if (caches)
-        e = launch_kv_cache(k, KD, v, KD, S, n_kv_heads, static_cast<uint16_t*>(k_cache_bf16),
-                            static_cast<uint16_t*>(v_cache_bf16), cap, st);
-    if (e == hipSuccess) e = launch_sdpa_prefill(q, QD, k, KD, v, KD, o, QD, S, n_heads, n_kv_heads, st);
+    // causal attention, which fills the caches too
+    e = launch_sdpa_prefill(q, QD, k, KD, v, KD, o, QD, S, n_heads, n_kv_heads,
+                            caches ? static_cast<uint16_t*>(k_cache_bf16) : nullptr,
+                            caches ? static_cast<uint16_t*>(v_cache_bf16) : nullptr, cap, st);
     if (e != hipSuccess) return hip_status(e, fn);
     // out = bf16(input + bf16(o_proj(o)))
     GemvGroup og{static_cast<const uint8_t*>(o_w_e4m3), QD, o_scale, static_cast<uint16_t*>(out_bf16), hidden, hidden,

@@ -16,9 +16,8 @@
 // (v_mfma_f32_32x32x16_bf16):
 // * S^T = K . Q^T (32 keys x 32 queries): the wave's query rows are the B operand, held in
 //   registers for the whole kernel; the scores of one query then sit in one lane (16 registers,
-//   the two lane halves holding alternate 4-key groups), so the row max and sum are in-lane plus
-//   one exchange between the halves.  The next block's scores are computed while this block's
-//   softmax runs, their MFMAs interleaved with its vector work.
+//   the two lane halves holding alternate 4-key groups), so the row max and sum are in-lane, with
+//   one exchange between the halves per block for the max and one at the end for the sum.
 // * online softmax in base 2 (weights exp2((s - m) log2(e) / sqrt(128)) with one fma per score),
 //   the running max m raised lazily (only when a score exceeds it by 2^8 in weight, so the
 //   accumulators are rescaled rarely); keys after the query masked on the diagonal blocks only.
@@ -27,6 +26,18 @@
 //   bf16(p - hi)), so the weights carry about 16 significant bits and the float32 row sums stay
 //   consistent with them.  The V^T operand, in the same key order, comes from two transposing
 //   LDS reads (ds_read_b64_tr_b16) of the token-major V tile.
+// The three run as a pipeline over blocks: while the matrix cores do the products with V of block g
+// and the scores of block g + 2, the same wave's vector unit turns the scores of block g + 1 into
+// weights.  A 32-cycle MFMA hides up to six vector instructions or two exponentials of its own
+// wave (measured), so the 24 MFMAs of a block are laid out in 24 slots with the block's 106 vector
+// instructions and 24 LDS reads spread over them; the compiler's own order ran the vector work
+// between the MFMAs' blocks.  Same-box times against that form (scores one block ahead, weights in
+// the block that uses them), 40 / 8 heads, S = 512 / 1000 / 2048 / 4096 / 8192: 17.5 / 31.4 / 69.8
+// / 235.9 / 877.5 -> 16.2 / 27.9 / 65.5 / 223.6 / 826.9 us; 16 / 4 heads, S = 2048: 52.4 -> 43.7.
+// At S = 4096 the cycles fell by 16% and the clock with them (2.1 -> 1.76 GHz): with the matrix
+// cores busy 62% of the time at 1.5 times the plain flops (P in two parts) the power budget is the
+// next bound.
+// The KV caches of the attention block are filled by the same launch (it was one of its own, 5-7 us).
 // Query tiles are scheduled longest first over all heads (the last tiles see the most keys).
 #include "nmi_device.hpp"
 #include "nmi_launch.hpp"
@@ -55,6 +66,10 @@ struct PrefillArgs {
     int S, H, H_KV, qtiles;
     int nslot;              // workgroups per pass of the dispatcher (one per CU)
     float scale2;           // log2(e) / sqrt(128)
+    float lazy;             // kLazy / scale2
+    uint16_t* k_cache;      // [H_KV, cap, 128] caches to fill from k and v (positions [0, S)), or nullptr
+    uint16_t* v_cache;
+    int cap;
 };
 
 __device__ __forceinline__ float fexp2(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -166,15 +181,14 @@ __global__ __launch_bounds__(256, 2) void sdpa_prefill_kernel(const PrefillArgs 
     for (int b = 0; b < 4; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) oacc[b][r] = 0.f;
-    float m = -INFINITY, l = 0.f;                               // raw score units
+    float m = -INFINITY, l = 0.f;       // raw score units; l is this lane half's share of the row sum
+    float corr = 1.f;                   // oacc's pending rescale
+    bool pending = false;               // (wave-uniform)
 
-    // causal mask of a block of 32 keys at kvb (only where it reaches past the wave's first query:
+    // causal mask of a block of 32 keys at kvb (only where it reaches past the wave's first query):
     // register r is key kvb + 8 (r / 4) + 4 h + r % 4, kept where it is <= qrow, then also < S for
-    // every stored query), the block's row max, and the lazy raise of the running max m: only when a
-    // score exceeds it by more than 8 / scale2 (then the weights exp2((s - m) scale2) stay below 2^8);
-    // the rescale of the accumulators runs when any lane of the wave raises its max.  O / l does not
-    // depend on m.  The first block holds key 0, so every query's max is finite from there on.
-    auto front = [&](f32x16& sc, int kvb) {
+    // every stored query
+    auto mask = [&](f32x16& sc, int kvb) {
         if (kvb + 31 > qw) {
             // a branch the compiler keeps: the blocks below the diagonal skip the mask entirely
             asm volatile("" ::: "memory");
@@ -183,135 +197,241 @@ __global__ __launch_bounds__(256, 2) void sdpa_prefill_kernel(const PrefillArgs 
             for (int r = 0; r < 16; ++r)
                 if (8 * (r >> 2) + (r & 3) > dq) sc[r] = -INFINITY;
         }
-        float tmax = -INFINITY;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, sc[r]);
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-        const bool raise = tmax > m + kLazy / a.scale2;
+    };
+    // The running max m raised lazily by a block's in-lane max: only when a score exceeds it by more
+    // than 8 / scale2 (the weights exp2((s - m) scale2) stay below 2^8).  O / l does not depend on
+    // m.  The first block holds key 0, so every query's max is finite from there on.  l holds the
+    // earlier blocks and is rescaled at once; oacc still misses the block before, whose weights are
+    // under the old max, and is rescaled after that block's products (settle).
+    auto raise_max = [&](float tmax) {
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(tmax), __float_as_uint(tmax), false, false);
+        tmax = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));       // both lane halves
+        const bool raise = tmax > m + a.lazy;
         if (__builtin_amdgcn_ballot_w64(raise)) {
             const float mn = raise ? tmax : m;
-            const float corr = raise ? fexp2((m - mn) * a.scale2) : 1.f;
+            corr = raise ? fexp2((m - mn) * a.scale2) : 1.f;
             l *= corr;
+            m = mn;
+            pending = true;
+        }
+    };
+    auto settle = [&]() {
+        if (pending) {
 #pragma unroll
             for (int b = 0; b < 4; ++b)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) oacc[b][r] *= corr;
-            m = mn;
+            pending = false;
         }
     };
-    // One block of 32 keys = key steps j0, j0 + 1 of the V tile at vst.  Key step j (16 keys): the
-    // weights as the P^T B fragment (registers 8 (j - j0) .. + 7 of sc), each in two bf16 parts
-    // (hi = bf16(p), lo = bf16(p - hi)), then O^T += V^T . P^T (the V^T operand of lane half h: keys
-    // 16 j + 4 h + {0..3} and 16 j + 8 + 4 h + {0..3}, two transposing reads of the V tile).  With NEXT, the next block's scores S^T = K . Q^T (the K slot at kst, four MFMAs
-    // per key step) go between them: independent work for the matrix cores under the softmax.
-    auto block = [&](auto next, const f32x16& sc, int j0, const uint8_t* vst, f32x16& nxt, const uint8_t* kst) {
-        constexpr bool NEXT = decltype(next)::value;
+    auto row_max = [&](const f32x16& sc) {
+        float t = sc[0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) t = fmaxf(t, sc[r]);
+        return t;
+    };
+    // The weights of 16 scores as the P^T B fragments of key steps 0 and 1 (registers 8 j .. + 7), each
+    // in two bf16 parts: hi = bf16(p), lo = bf16(p - hi).  Three stages per pair of scores e = 2 i,
+    // 2 i + 1, so that a pair can be spread over three MFMAs.
+    struct Weights {
+        uint32_t hi[8], lo[8];
+    };
+    float p0 = 0.f, p1 = 0.f;
+    // pin: keeps the computation of x in the slot it is written in (the compiler otherwise sinks it
+    // to the block that uses it, past all the MFMAs meant to hide it)
+    auto pin = [](auto& x) __attribute__((always_inline)) { asm volatile("" : "+v"(x)); };
+    auto weigh = [&](const f32x16& sc, float mc, int i, int stage, Weights& w) __attribute__((always_inline)) {
+        if (stage == 0) {
+            p0 = fexp2(__builtin_fmaf(sc[2 * i], a.scale2, -mc));
+            p1 = fexp2(__builtin_fmaf(sc[2 * i + 1], a.scale2, -mc));
+            pin(p0);
+            pin(p1);
+        } else if (stage == 1) {
+            w.hi[i] = pack_bf16(p0, p1);
+            l += p0;
+            l += p1;
+            pin(w.hi[i]);
+            pin(l);
+        } else {
+            // (v_dot2 would save the unpacking of hi, but beside MFMAs each costs 16 cycles and more)
+            w.lo[i] = pack_bf16(p0 - bf16lo_to_f32(w.hi[i]), p1 - bf16hi_to_f32(w.hi[i]));
+            pin(w.lo[i]);
+        }
+    };
+    auto frag = [&](const uint32_t (&w)[8], int j) {
+        return __builtin_bit_cast(bf16x8, uint4{w[4 * j], w[4 * j + 1], w[4 * j + 2], w[4 * j + 3]});
+    };
+    auto read_k = [&](const uint8_t* kst, int s) {
+        return *reinterpret_cast<const bf16x8*>(kst + k_off(l32, 2 * s + h));
+    };
+    auto read_v = [&](const uint8_t* vst, int j, int b) {
+        const v4i16 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vst + vtr[b] + 4096 * j));
+        const v4i16 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vst + vtr[b] + 4096 * j + 2048));
+        return __builtin_bit_cast(bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    // Block g (32 keys: key steps j0, j0 + 1 of the V tile at vst) of a three-deep pipeline: the 16
+    // products O^T += V^T . P^T of block g (weights wc), the 8 products S^T = K . Q^T of block g + 2
+    // (K slot at kst, into nxt), and the weights of block g + 1 (scores sc, into wn).  None of the
+    // three depends on another within the block, so the matrix cores run under the vector work of the
+    // same wave: 24 slots of one MFMA, at most two LDS reads (three slots ahead of their use) and
+    // three or four vector instructions, fenced so that the compiler keeps them apart.  Then block
+    // g + 2's mask and max.  kvb2: its first key.
+    auto block = [&](auto masked, const f32x16& sc, f32x16& nxt, const Weights& wc, Weights& wn, const uint8_t* kst,
+                     const uint8_t* vst, int j0, int kvb2) __attribute__((always_inline)) {
         const float mc = m * a.scale2;
-        float psum = 0.f;
-        if constexpr (NEXT) {
+        bf16x8 kf[4], vf[3];
+        kf[0] = read_k(kst, 0);
+        kf[1] = read_k(kst, 1);
+        vf[0] = read_v(vst, j0, 0);
+        weigh(sc, mc, 0, 0, wn);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) nxt[r] = 0.f;
+        for (int r = 0; r < 16; ++r) nxt[r] = 0.f;
+        float tmax = 0.f;
+#pragma unroll
+        for (int q = 0; q < 24; ++q) {
+            // MFMA: S in slots 0, 1, 3, 4, 6, 7, 9, 10; P.V (hi, lo of each V fragment u) in the others
+            const bool is_k = q < 11 && q % 3 != 2;
+            if (is_k) {
+                const int st = 2 * (q / 3) + q % 3;
+                nxt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[st & 3], qf[st], nxt, 0, 0, 0);
+                if (st + 2 < 8) kf[(st + 2) & 3] = read_k(kst, st + 2);
+            } else {
+                const int p = q < 12 ? q / 3 : q - 8, u = p >> 1, b = u & 3;
+                const bf16x8 w = frag((p & 1) ? wc.lo : wc.hi, u >> 2);
+                oacc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[u % 3], w, oacc[b], 0, 0, 0);
+            }
+            // V fragment u + 1: at slot 4 (u = 0), then three or four slots ahead of its use
+            if (q == 4) vf[1] = read_v(vst, j0, 1);
+            if (q >= 9 && q <= 19 && (q & 1)) {
+                const int u = (q - 9) / 2 + 2;
+                vf[u % 3] = read_v(vst, j0 + (u >> 2), u & 3);
+            }
+            // vector work: pair q / 3's stages (pair 0's first is above), one stage ahead of the slot
+            if (q < 23) weigh(sc, mc, (q + 1) / 3, (q + 1) % 3, wn);
+            if constexpr (!decltype(masked)::value) {
+                if (q == 14) tmax = fmaxf(fmaxf(nxt[0], nxt[1]), nxt[2]);
+                if (q >= 15 && q <= 20) tmax = fmaxf(fmaxf(tmax, nxt[2 * q - 27]), nxt[2 * q - 26]);
+                if (q == 21) tmax = fmaxf(tmax, nxt[15]);
+                if (q >= 14 && q <= 21) pin(tmax);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-            uint32_t hw[4], lw[4];
-#pragma unroll
-            for (int e = 0; e < 8; e += 2) {
-                const float p0 = fexp2(__builtin_fmaf(sc[8 * jj + e], a.scale2, -mc));
-                const float p1 = fexp2(__builtin_fmaf(sc[8 * jj + e + 1], a.scale2, -mc));
-                psum += p0;
-                psum += p1;
-                const uint32_t w = pack_bf16(p0, p1);
-                hw[e >> 1] = w;
-                lw[e >> 1] = pack_bf16(p0 - __uint_as_float(w << 16), p1 - __uint_as_float(w & 0xffff0000u));
-            }
-            const bf16x8 phi = __builtin_bit_cast(bf16x8, uint4{hw[0], hw[1], hw[2], hw[3]});
-            const bf16x8 plo = __builtin_bit_cast(bf16x8, uint4{lw[0], lw[1], lw[2], lw[3]});
-            if constexpr (NEXT) {
-#pragma unroll
-                for (int s = 4 * jj; s < 4 * jj + 4; ++s) {
-                    const bf16x8 kf = *reinterpret_cast<const bf16x8*>(kst + k_off(l32, 2 * s + h));
-                    nxt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[s], nxt, 0, 0, 0);
-                }
-            }
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const int j = j0 + jj;
-                const v4i16 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vst + vtr[b] + 4096 * j));
-                const v4i16 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vst + vtr[b] + 4096 * j + 2048));
-                const bf16x8 vf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
-                oacc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, phi, oacc[b], 0, 0, 0);
-                oacc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, plo, oacc[b], 0, 0, 0);
-            }
+        if constexpr (decltype(masked)::value) {
+            mask(nxt, kvb2);
+            tmax = row_max(nxt);
         }
-        psum += __shfl_xor(psum, 32);
-        l += psum;
+        settle();
+        raise_max(tmax);
     };
     auto kslot = [&](int g) { return lds + (g & 3) * kKBlk; };
     auto vstage = [&](int t) { return lds + 4 * kKBlk + (t & 1) * kVBytes; };
-    // Tile t (blocks 2 t, 2 t + 1) with a tile after it: every wave has keys <= its queries in all
-    // tiles but the last.  On entry sa holds block 2 t's scores, K slots hold blocks 2 t + 1 and
-    // 2 t + 2, V stage t & 1 tile t.  The DMAs refill the slots and the stage read in step t - 1
-    // (published by its closing barrier).  P, the parity of t, makes the LDS offsets constants.
+    // Tile t = blocks 2 t, 2 t + 1.  On entry wa holds block 2 t's weights, sb block 2 t + 1's scores;
+    // K slots hold blocks 2 t + 2 and 2 t + 3, V stage t & 1 tile t.  The DMAs refill the slots and
+    // the stage read in tile t - 1 (published by its closing barrier).  P, the parity of t, makes the
+    // LDS offsets constants.
     f32x16 sa, sb;
-    auto step = [&](auto P, int t) {
-        constexpr int par = decltype(P)::value;
+    Weights wa, wb;
+    auto issue = [&](int t) {
         issue_v(t + 1);
-        issue_k(2 * t + 3);
-        if (2 * t + 4 < nblk) issue_k(2 * t + 4);
-        front(sa, t * kBK);
-        block(std::true_type{}, sa, 0, vstage(par), sb, kslot(2 * par + 1));
-        front(sb, t * kBK + 32);
-        block(std::true_type{}, sb, 2, vstage(par), sa, kslot(2 * par + 2));
-        // this wave's DMAs done and its LDS reads returned (the compiler may place the MFMAs that
-        // consume the last reads after this statement; the stages they read are refilled right
-        // after the barrier), then the barrier
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    };
-    // the last tile: only the waves with a key <= some query of theirs (a second block past the
-    // wave's queries is all masked: weights 0)
-    auto last = [&](auto P, int t) {
-        constexpr int par = decltype(P)::value;
-        if (t * kBK <= qw + 31) {
-            front(sa, t * kBK);
-            block(std::true_type{}, sa, 0, vstage(par), sb, kslot(2 * par + 1));
-            front(sb, t * kBK + 32);
-            block(std::false_type{}, sb, 2, vstage(par), sb, lds);
+        if (2 * t + 4 < nblk) {
+            issue_k(2 * t + 4);
+            issue_k(2 * t + 5);
         }
+    };
+    // this wave's DMAs done and its LDS reads returned (the compiler may place the MFMAs that consume
+    // the last reads after this statement; the stages they read are refilled right after the
+    // barrier), then the barrier
+    auto publish = []() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    // below the diagonal: P, the parity of t, makes the LDS offsets constants
+    auto step = [&](auto P, int t) __attribute__((always_inline)) {
+        constexpr int par = decltype(P)::value;
+        constexpr std::false_type masked{};
+        issue(t);
+        block(masked, sb, sa, wa, wb, kslot(2 * par + 2), vstage(par), 0, t * kBK + 64);
+        block(masked, sa, sb, wb, wa, kslot(2 * par + 3), vstage(par), 2, t * kBK + 96);
+        publish();
     };
 
     issue_k(0);
-    issue_v(0);
     issue_k(1);
-    if (nblk > 2) issue_k(2);
-    // every load complete (the query's too, so the compiler has no load of its own outstanding in
-    // the loop and places no wait there), then the barrier that publishes the first blocks
+    issue_v(0);
+    if (nblk > 2) {
+        issue_k(2);
+        issue_k(3);
+    }
+    // K blocks 0 and 1 landed (the query's loads too, so the compiler has no load of its own
+    // outstanding), then the barrier that publishes them; V tile 0 and K blocks 2, 3 may still be
+    // on their way
 #pragma unroll
     for (int s = 0; s < 8; ++s) asm volatile("" ::"v"(qf[s]));
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    if (nblk > 2) asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(4)\n\ts_barrier" ::: "memory");
+    // this workgroup's share of the KV cache fill: its own rows, by one query head of the group
+    const bool fill = a.k_cache && head % (a.H / a.H_KV) == qt % (a.H / a.H_KV);
+    uint4 kr[8], vr[8];
+    if (fill) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) sa[r] = 0.f;
+        for (int u = 0; u < 8; ++u) {
+            const int p = min(q0 + (tid >> 4) + 16 * u, S - 1);
+            kr[u] = load16(a.k + (int64_t)p * a.ldk + kvh * kD + 8 * (tid & 15));
+            vr[u] = load16(a.v + (int64_t)p * a.ldv + kvh * kD + 8 * (tid & 15));
+        }
+    }
+    // fill the pipeline: scores of blocks 0 and 1, weights of block 0
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sa[r] = sb[r] = 0.f;
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
-        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(lds + k_off(l32, 2 * s + h));
-        sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[s], sa, 0, 0, 0);
+        sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(read_k(kslot(0), s), qf[s], sa, 0, 0, 0);
+        sb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(read_k(kslot(1), s), qf[s], sb, 0, 0, 0);
     }
-    // slot 0 is refilled in step 0: every wave's block-0 reads first
-    __syncthreads();
-    using even = std::integral_constant<int, 0>;
-    using odd = std::integral_constant<int, 1>;
-    // pairs of tiles, then the tail (one exit: the register allocation of the loop stays simple)
+    if (fill) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int p = q0 + (tid >> 4) + 16 * u;
+            if (p < S) {
+                const int64_t off = ((int64_t)kvh * a.cap + p) * kD + 8 * (tid & 15);
+                *reinterpret_cast<uint4*>(a.k_cache + off) = kr[u];
+                *reinterpret_cast<uint4*>(a.v_cache + off) = vr[u];
+            }
+        }
+    }
+    mask(sa, 0);
+    mask(sb, 32);
+    raise_max(row_max(sa));
+    settle();
+    {
+        const float mc = m * a.scale2;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int st = 0; st < 3; ++st) weigh(sa, mc, i, st, wa);
+    }
+    raise_max(row_max(sb));
+    // the rest landed; and slots 0 and 1 are refilled in tile 0: every wave's reads of them first
+    publish();
     int t = 0;
-    for (; t + 2 < ntiles; t += 2) {
-        step(even{}, t);
-        step(odd{}, t + 1);
+    // tiles t, t + 1 compute the scores of keys up to 64 t + 255: below the diagonal while that is
+    // before the workgroup's first query
+    for (; t * kBK + 4 * kBK <= q0; t += 2) {
+        step(std::integral_constant<int, 0>{}, t);
+        step(std::integral_constant<int, 1>{}, t + 1);
     }
-    if (t + 1 < ntiles) {
-        step(even{}, t);
-        last(odd{}, t + 1);
-    } else {
-        last(even{}, t);
+    // the last tiles (up to four), one body for all: a short prompt runs no other.  Each wave takes
+    // the blocks with a key <= some query of its own.  The scores past those come from slots that
+    // may hold other blocks; they are masked (their keys lie past every query).
+    for (; t < ntiles; ++t) {
+        const bool more = t + 1 < ntiles;
+        if (more) issue(t);
+        if (qw < S && t * kBK <= qw + 31) {
+            constexpr std::true_type masked{};
+            block(masked, sb, sa, wa, wb, kslot(2 * t + 2), vstage(t), 0, t * kBK + 64);
+            if (t * kBK + 32 <= qw + 31) block(masked, sa, sb, wb, wa, kslot(2 * t + 3), vstage(t), 2, t * kBK + 96);
+        }
+        if (more) publish();
     }
+    l += __shfl_xor(l, 32);
 
     // O = O^T / l: register r of block b is dim 32 b + 8 (r / 4) + 4 h + r % 4 of query qrow
     if (qrow < S) {
@@ -328,43 +448,11 @@ __global__ __launch_bounds__(256, 2) void sdpa_prefill_kernel(const PrefillArgs 
     }
 }
 
-// KV cache fill: k_cache / v_cache [H_KV, cap, 128] positions [0, S) from k and v (the
-// reference's cudaMemcpy2DAsync of its head-major K/V, attention_block.cuh:355-364).  One workgroup
-// per (64 positions, KV head); thread t copies chunk t % 16 of rows t / 16 + 16 u.
-__global__ __launch_bounds__(256) void kv_cache_kernel(const uint16_t* __restrict__ k, int64_t ldk,
-                                                       const uint16_t* __restrict__ v, int64_t ldv,
-                                                       uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, int cap,
-                                                       int S) {
-    const int p0 = blockIdx.x * 64, kvh = blockIdx.y, tid = threadIdx.x;
-    const int c = tid & 15;
-    uint4 kr[4], vr[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int p = min(p0 + (tid >> 4) + 16 * u, S - 1);
-        kr[u] = load16(k + (int64_t)p * ldk + kvh * kD + 8 * c);
-        vr[u] = load16(v + (int64_t)p * ldv + kvh * kD + 8 * c);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int p = p0 + (tid >> 4) + 16 * u;
-        if (p < S) {
-            *reinterpret_cast<uint4*>(kc + ((int64_t)kvh * cap + p) * kD + 8 * c) = kr[u];
-            *reinterpret_cast<uint4*>(vc + ((int64_t)kvh * cap + p) * kD + 8 * c) = vr[u];
-        }
-    }
-}
-
 }  // namespace
 
-hipError_t launch_kv_cache(const uint16_t* k, int64_t ldk, const uint16_t* v, int64_t ldv, int S, int H_KV,
-                           uint16_t* k_cache, uint16_t* v_cache, int cap, hipStream_t stream) {
-    hipLaunchKernelGGL(kv_cache_kernel, dim3((unsigned)((S + 63) / 64), H_KV), dim3(256), 0, stream, k, ldk, v, ldv,
-                       k_cache, v_cache, cap, S);
-    return hipGetLastError();
-}
-
 hipError_t launch_sdpa_prefill(const uint16_t* q, int64_t ldq, const uint16_t* k, int64_t ldk, const uint16_t* v,
-                               int64_t ldv, uint16_t* o, int64_t ldo, int S, int H, int H_KV, hipStream_t stream) {
+                               int64_t ldv, uint16_t* o, int64_t ldo, int S, int H, int H_KV, uint16_t* k_cache,
+                               uint16_t* v_cache, int cap, hipStream_t stream) {
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&sdpa_prefill_kernel),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     if (attr != hipSuccess) return attr;
@@ -383,6 +471,10 @@ hipError_t launch_sdpa_prefill(const uint16_t* q, int64_t ldq, const uint16_t* k
     a.qtiles = (S + kBQ - 1) / kBQ;
     a.nslot = device_info().num_cu;
     a.scale2 = 1.4426950408889634f / sqrtf((float)kD);
+    a.lazy = kLazy / a.scale2;
+    a.k_cache = k_cache;
+    a.v_cache = v_cache;
+    a.cap = cap;
     hipLaunchKernelGGL(sdpa_prefill_kernel, dim3(a.qtiles * H), dim3(256), kLds, stream, a);
     return hipGetLastError();
 }

@@ -1331,7 +1331,8 @@ struct DmaPlan {
 // CUs in use (they share the power budget: the clock falls), fitted to a sweep of M = 512 .. 4096
 // on the model's projections (us, MI355X; the fit is within 5% of most of them):
 //   rounds * (start + KT * fixed) + KT * U / CUs * shared,   KT = k tiles of one workgroup,
-// and a split adds its second kernel.  K is split into one round of workgroups: one matrix where
+// and a split adds its second kernel (a fixed time, the partials read one split after another, and
+// their bytes).  K is split into one round of workgroups: one matrix where
 // K >= 4096 (below, from M = 512, no split of any projection was faster than its best unsplit
 // tiles, and a row's sums stay the same in a larger batch or a group), matrices sharing x where
 // M < 512 (dma_plan_ws); and only for a modelled gain of 8%: with most CUs busy either way the power budget decides (2048 x 3136 x
@@ -1343,7 +1344,7 @@ struct DmaPlan {
 DmaPlan dma_plan(int M, int tiles_n, int K, int ng, bool may_split) {
     struct Cost { int bm; double start, fixed, shared; };
     constexpr Cost kCost[] = {{256, 12.0, 0.857, 0.408}, {192, 10.0, 0.61, 0.41}, {128, 8.6, 0.395, 0.337}};
-    constexpr double kReduce = 5.0, kReducePerByte = 0.09e-6;
+    constexpr double kReduce = 5.0, kReducePerSplit = 0.5, kReducePerByte = 0.09e-6;
     constexpr double kSplitMargin = 1.08;
     constexpr int kMinSplitK = 4096, kMaxSplits = 16;
     const Tuning& t = tuning();
@@ -1363,7 +1364,7 @@ DmaPlan dma_plan(int M, int tiles_n, int K, int ng, bool may_split) {
             const int64_t rounds = (T * sp + G - 1) / G;
             const double kt = (double)((KT + sp - 1) / sp);
             double us = rounds * (c.start + kt * c.fixed) + kt * c.shared * (double)(T * sp) / G;
-            if (sp > 1) us = (us + kReduce + (double)p.part_bytes() * kReducePerByte) * kSplitMargin;
+            if (sp > 1) us = (us + kReduce + sp * kReducePerSplit + (double)p.part_bytes() * kReducePerByte) * kSplitMargin;
             p.us = us;
             if (forced && sp > 1) us -= 1e9;        // a forced split wins over its unsplit forms
             if (best.bm == 0 || us < best_us) best = p, best_us = us;
@@ -1521,16 +1522,17 @@ size_t gemm_split_workspace_bytes(int M, int64_t N, int K) {
 
 namespace {
 // The DMA-fed kernel for one matrix at M < 512, by its modelled time against the short-prompt
-// kernel's: their crossing lies between M = 100 (N = 17504) and about 300 (N = 3136).  Measured
-// (us, short-prompt / DMA-fed): 100 x 17504 x 3136 35.6 / 34.6, 200 x 17504 x 3136 66.8 / 36.1, 300
-// x 12544 x 3136 68.5 / 35.5, 300 x 3136 x 12544 44.2 / 40.0, 500 x 3136 x 7680 39.8 / 36.5; but 200 x
-// 3136 x 12544 33.7 / 34.4, 256 x 7168 x 3136 24.8 / 24.9.  The short kernel's own knobs keep it.
+// kernel's: their crossing lies between M = 100 (N = 17504) and about 400 (N = 3136).  Measured
+// (us, short-prompt / DMA-fed): 100 x 17504 x 3136 35.6 / 34.6, 200 x 17504 x 3136 66.8 / 36.1, 300 x
+// 12544 x 3136 68.5 / 35.5, 400 x 3136 x 12544 57.0 / 46.7, 500 x 3136 x 7680 39.8 / 36.5; but 200 x 3136
+// x 12544 33.7 / 34.4, 256 x 7168 x 3136 24.8 / 24.9, 511 x 1024 x 12544 27.6 / 34.6; and fewer rows
+// than a column band stay with the short kernel (300 x 64 x 2048 23.6 / 26.0), as do its own knobs.
 double dma_short_m_us(int M, int N, int K, size_t ws_bytes) {
     return dma_plan_ws(M, (N + 255) / 256, K, 1, ws_bytes).us;
 }
 bool dma_beats_short(int M, int N, int K, size_t ws_bytes) {
     const Tuning& t = tuning();
-    if (M <= kShortOnlyM || t.gemm_short != 0 || t.gemm_splits > 1 || t.gemm_sk == 1 || t.gemm_bm == 256) return false;
+    if (M <= kShortOnlyM || N < 256 || t.gemm_short != 0 || t.gemm_splits > 1 || t.gemm_sk == 1 || t.gemm_bm == 256) return false;
     return dma_short_m_us(M, N, K, ws_bytes) < gemm_short_us(M, N, K, ws_bytes);
 }
 }  // namespace

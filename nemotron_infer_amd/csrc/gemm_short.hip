@@ -381,9 +381,10 @@ int gemm_short_splits(int M, int N, int K) {
     return std::max(1, std::min(want, std::min(by_k, by_bytes)));
 }
 
-// Fitted to a sweep of M = 100 .. 500 on the model's projections above M = 64 (within 10% of most):
-// rounds of one workgroup per CU, a k tile 0.66 us, 0.58 where K is split, 4 us to start and end
-// one, 6 us for the second kernel.  M <= 64: two launches of about 7 us whatever the shape.
+// Fitted to sweeps of M = 100 .. 511 on the model's projections and on N = 64 .. 2048 above M = 64
+// (within 10% of most): rounds of one workgroup per CU, 4 us to start and end one, a k tile 0.66 us,
+// or where K is split 0.40 us and up to 0.18 more with the CUs in use, and 6 us for the second
+// kernel.  M <= 64: two launches of about 7 us whatever the shape.
 double gemm_short_us(int M, int N, int K, size_t ws_bytes) {
     if (M <= 64) return 14.0;
     const ShortCfg& c = kForms[short_form(M, N)];
@@ -393,7 +394,8 @@ double gemm_short_us(int M, int N, int K, size_t ws_bytes) {
     const int64_t units = (int64_t)((N + c.bn() - 1) / c.bn()) * ((M + c.bm() - 1) / c.bm()) * splits;
     const double kt = (double)((KT + splits - 1) / splits);
     const double rounds = (double)((units + cu - 1) / cu);
-    return splits > 1 ? rounds * (kt * 0.58 + 4.0) + 6.0 : rounds * (kt * 0.66 + 4.0);
+    const double busy = std::min(1.0, (double)units / cu);
+    return splits > 1 ? rounds * (kt * (0.40 + 0.18 * busy) + 4.0) + 6.0 : rounds * (kt * 0.66 + 4.0);
 }
 
 // Enough for any N' <= N (grouped launches share one workspace): splits x N' is at most

@@ -291,6 +291,12 @@ __global__ __launch_bounds__(256, 4) void mamba_scan_kernel(const MambaPrefillAr
 // state accumulates in float32 MFMA registers across chunks.  Each wave forms the G rows of its
 // own 16 tokens and uses them straight from the MFMA output registers, so per chunk only the
 // staging of B, C and x and the state's two-part copy go through a barrier.
+// Eight waves: four for y (16 tokens each), four for the state (32 of its 128 rows each), which read
+// the same staged chunk and the same S0, so the two run beside each other instead of one after the
+// other in four waves: a chunk is a chain of dependent LDS reads, MFMAs and vector work (at S =
+// 2048 the four-wave form had its vector units busy 43% of the cycles, its matrix cores 14%, and
+// waited 35%).  Same box, 96 heads of 80: one sequence of 2048 tokens 87.9 -> 82.7 us, two of 500 equal.  (Two,
+// three or five blocks of 16 rows of P per workgroup, sharing G: slower, the chain grows by each.)
 // Each SIMD issues a wave64 VALU instruction over 4 cycles, so the per-element work is kept on
 // MFMA: what remains on VALU per chunk is the decay weights, the G mask and the two-part splits.
 // Tokens past the end of the sequence get dt = 0 and x = 0: no weight, no decay.
@@ -330,7 +336,9 @@ __device__ __forceinline__ int bc_off(int row, int c) { return row * 256 + ((c ^
 __device__ __forceinline__ int t_off(int row, int c) { return row * 128 + ((c ^ ((row >> 1) & 7)) << 4); }
 __device__ __forceinline__ int s_off(int p, int c) { return p * 256 + ((c ^ (p & 15)) << 4); }
 
-__global__ __launch_bounds__(256, 2) void mamba_ssd_kernel(const MambaPrefillArgs a) {
+constexpr int kSsdWaves = 8, kSsdThreads = 64 * kSsdWaves;
+
+__global__ __launch_bounds__(kSsdThreads, 4) void mamba_ssd_kernel(const MambaPrefillArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int slices = (a.P + kPW - 1) / kPW;
     const int h = blockIdx.x / slices, p0 = (blockIdx.x % slices) * kPW;
@@ -350,13 +358,14 @@ __global__ __launch_bounds__(256, 2) void mamba_ssd_kernel(const MambaPrefillArg
     auto dec_arr = [&](int k, int i) __attribute__((always_inline)) { return reinterpret_cast<float*>(lds + kOffDec + k * kDecSet + i * 256); };
 
     // chunk staging in registers (the next chunk's loads are in flight during this one): B and C
-    // rows (1024 chunks of 16 B each: 4 per thread), x (threads < 128: token tid / 2, P columns
+    // rows (1024 chunks of 16 B each: 2 per thread), x (threads < 128: token tid / 2, P columns
     // 8 (tid % 2) .. + 7 of the slice)
-    uint4 rb[4], rc[4], rx = uint4{0u, 0u, 0u, 0u};
+    constexpr int BU = 1024 / kSsdThreads;
+    uint4 rb[BU], rc[BU], rx = uint4{0u, 0u, 0u, 0u};
     auto gload = [&](int t0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int q = tid + 256 * u;
+        for (int u = 0; u < BU; ++u) {
+            const int q = tid + kSsdThreads * u;
             const int t = min(t0 + (q >> 4), S - 1), c = q & 15;
             const uint16_t* row = a.xc + (xrow0 + t) * a.xc_ld + a.inter;
             rb[u] = load16(row + grp * kN + 8 * c);
@@ -376,11 +385,11 @@ __global__ __launch_bounds__(256, 2) void mamba_ssd_kernel(const MambaPrefillArg
             }
         }
     };
-    // dt of the chunk at t0 (wave 1 scans it one chunk ahead of its use)
+    // dt of the chunk at t0 (wave 4 scans it one chunk ahead of its use)
     auto load_dt = [&](int t0) __attribute__((always_inline)) {
         return a.proj[(xrow0 + min(t0 + lane, S - 1)) * a.proj_ld + a.inter + a.conv_dim + h];
     };
-    // Wave 1: softplus(dt + bias) (the reference's cut-offs) and the chunk's inclusive cumulative
+    // Wave 4: softplus(dt + bias) (the reference's cut-offs) and the chunk's inclusive cumulative
     // log2-decay (finite even where dt saturates: a decay that small is a reset either way), into
     // decay set k; tokens at or past nt get dt = 0.
     auto scan = [&](uint16_t dtb, int nt, int k) __attribute__((always_inline)) {
@@ -426,28 +435,28 @@ __global__ __launch_bounds__(256, 2) void mamba_ssd_kernel(const MambaPrefillArg
         lo = __builtin_bit_cast(bf16x8, uint4{lw[0], lw[1], lw[2], lw[3]});
     };
 
-    // the state, transposed, as two 16 x 16 MFMA accumulator blocks per wave: rows n = 16 (2 wave +
-    // nb) + 4 g4 + r, columns p = l16
+    // the state, transposed, as two 16 x 16 MFMA accumulator blocks in each of waves 4 .. 7: rows n =
+    // 16 (2 (wave - 4) + nb) + 4 g4 + r, columns p = l16
     f32x4 st[2];
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) st[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // S0 hi / lo of the first chunk (buffer 0): zero (thread t clears 16 bytes of each)
+    // S0 hi / lo of the first chunk (buffer 0): zero (thread t clears 16 bytes)
+    static_assert(16 * kSsdThreads == kSBuf, "one buffer");
     *reinterpret_cast<uint4*>(lds + kOffS + 16 * tid) = uint4{0u, 0u, 0u, 0u};
-    *reinterpret_cast<uint4*>(lds + kOffS + 4096 + 16 * tid) = uint4{0u, 0u, 0u, 0u};
 
     gload(0);
-    // dt two chunks ahead (wave 1): chunk 0 scanned here, chunk c + 1 during chunk c
+    // dt two chunks ahead (wave 4): chunk 0 scanned here, chunk c + 1 during chunk c
     uint16_t rdt1 = 0, rdt2 = 0;
-    if (wave == 1) {
+    if (wave == 4) {
         const uint16_t rdt0 = load_dt(0);
         rdt1 = load_dt(kQ);
         scan(rdt0, min(kQ, S), 0);
     }
     // One chunk: (a) the staged chunk into LDS (B, C row-major; x row-major, zero past the
-    // sequence), the next chunk's loads, barrier; then each wave on its own (no barrier): rows
-    // i = 16 wave + l16 of G and y, rows n = 32 wave .. + 31 of the state; the new state's two-part
-    // copy into the other S0 buffer; barrier.  rcur holds the next chunk's dt (wave 1), rnext
-    // receives the one after it (register roles alternate between calls: no copy waits on a load).
+    // sequence), the next chunk's loads, barrier; then each wave on its own (no barrier): waves 0 .. 3
+    // rows i = 16 wave + l16 of G and y; waves 4 .. 7 rows n = 32 (wave - 4) .. + 31 of the state and
+    // its two-part copy into the other S0 buffer; barrier.  rcur holds the next chunk's dt (wave 4),
+    // rnext receives the one after it (register roles alternate between calls: no copy waits on a load).
     auto chunk = [&](auto W, int t0, uint16_t& rcur, uint16_t& rnext) __attribute__((always_inline)) {
         constexpr int w = decltype(W)::value;                    // this wave (a constant per instantiation)
         const int par = (t0 / kQ) & 1;
@@ -457,8 +466,8 @@ __global__ __launch_bounds__(256, 2) void mamba_ssd_kernel(const MambaPrefillArg
         const float* dts = dec_arr(par, 3);
         const int nt = min(kQ, S - t0);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int q = tid + 256 * u;
+        for (int u = 0; u < BU; ++u) {
+            const int q = tid + kSsdThreads * u;
             const int j = q >> 4, cc = q & 15;
             *reinterpret_cast<uint4*>(lds + kOffB + bc_off(j, cc)) = rb[u];
             *reinterpret_cast<uint4*>(lds + kOffC + bc_off(j, cc)) = rc[u];
@@ -468,13 +477,10 @@ __global__ __launch_bounds__(256, 2) void mamba_ssd_kernel(const MambaPrefillArg
             *reinterpret_cast<uint4*>(lds + kOffX + j * 32 + 2 * pc) = j < nt ? rx : uint4{0u, 0u, 0u, 0u};
         }
         if (t0 + kQ < S) gload(t0 + kQ);
-        if (w == 1 && t0 + 2 * kQ < S) rnext = load_dt(t0 + 2 * kQ);
+        if (w == 4 && t0 + 2 * kQ < S) rnext = load_dt(t0 + 2 * kQ);
         __syncthreads();
 
-        // wave 1: the next chunk's decay into the other set (its last readers finished before the
-        // previous chunk's closing barrier)
-        if (w == 1 && t0 + kQ < S) scan(rcur, min(kQ, S - t0 - kQ), par ^ 1);
-
+        if constexpr (w < 4) {
         const int i = 16 * w + l16;                              // this lane's token row of G and y
         // C rows i as the B operand (k = n): used by C B^T and by S0 C^T
         bf16x8 cf[4];
@@ -558,7 +564,8 @@ __global__ __launch_bounds__(256, 2) void mamba_ssd_kernel(const MambaPrefillArg
                 }
             }
         }
-        // S^T = exp(c_63) S0^T + B^T (w x): rows n = 16 (2 wave + nb) + 4 g4 + r, columns p = l16; A =
+        } else {
+        // S^T = exp(c_63) S0^T + B^T (w x): rows n = 16 (2 (w - 4) + nb) + 4 g4 + r, columns p = l16; A =
         // B^T (transposing reads of B), B = (w x) in two parts (k = 8 g4 + 4 q + e <-> token
         // 32 ks + 8 g4 + 4 q + e, x^T by transposing reads)
         {
@@ -583,7 +590,7 @@ __global__ __launch_bounds__(256, 2) void mamba_ssd_kernel(const MambaPrefillArg
                 split(wv, wh, wl);
 #pragma unroll
                 for (int nb = 0; nb < 2; ++nb) {
-                    const bf16x8 ab = bt_frag(16 * (2 * w + nb), ks);
+                    const bf16x8 ab = bt_frag(16 * (2 * (w - 4) + nb), ks);
                     st[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ab, wh, st[nb], 0, 0, 0);
                     st[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ab, wl, st[nb], 0, 0, 0);
                 }
@@ -594,7 +601,7 @@ __global__ __launch_bounds__(256, 2) void mamba_ssd_kernel(const MambaPrefillArg
             uint8_t* s1 = lds + kOffS + (par ^ 1) * kSBuf;
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb) {
-                const int n0 = 16 * (2 * w + nb) + 4 * g4;
+                const int n0 = 16 * (2 * (w - 4) + nb) + 4 * g4;
                 const f32x4 v = st[nb];
                 const uint32_t h01 = pack_bf16(v[0], v[1]), h23 = pack_bf16(v[2], v[3]);
                 const uint32_t l01 = pack_bf16(v[0] - __uint_as_float(h01 << 16), v[1] - __uint_as_float(h01 & 0xffff0000u));
@@ -603,6 +610,10 @@ __global__ __launch_bounds__(256, 2) void mamba_ssd_kernel(const MambaPrefillArg
                 *reinterpret_cast<uint2*>(s1 + off) = uint2{h01, h23};
                 *reinterpret_cast<uint2*>(s1 + 4096 + off) = uint2{l01, l23};
             }
+        }
+        // wave 4: the next chunk's decay into the other set (its last readers finished before the
+        // previous chunk's closing barrier)
+        if (w == 4 && t0 + kQ < S) scan(rcur, min(kQ, S - t0 - kQ), par ^ 1);
         }
         __syncthreads();
     };
@@ -617,12 +628,16 @@ __global__ __launch_bounds__(256, 2) void mamba_ssd_kernel(const MambaPrefillArg
         case 0: run(std::integral_constant<int, 0>{}); break;
         case 1: run(std::integral_constant<int, 1>{}); break;
         case 2: run(std::integral_constant<int, 2>{}); break;
-        default: run(std::integral_constant<int, 3>{}); break;
+        case 3: run(std::integral_constant<int, 3>{}); break;
+        case 4: run(std::integral_constant<int, 4>{}); break;
+        case 5: run(std::integral_constant<int, 5>{}); break;
+        case 6: run(std::integral_constant<int, 6>{}); break;
+        default: run(std::integral_constant<int, 7>{}); break;
     }
-    if (a.ssm_state && l16 < pw) {
+    if (a.ssm_state && l16 < pw && wave >= 4) {
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
-            const int n0 = 16 * (2 * wave + nb) + 4 * g4;
+            const int n0 = 16 * (2 * (wave - 4) + nb) + 4 * g4;
             *reinterpret_cast<float4*>(a.ssm_state + (((size_t)b * a.H + h) * a.P + p0 + l16) * kN + n0) =
                 float4{st[nb][0], st[nb][1], st[nb][2], st[nb][3]};
         }
@@ -652,7 +667,7 @@ hipError_t launch_mamba_prefill_mixer(const MambaPrefillArgs& a, int batch, hipS
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, kSsdLds);
     if (attr != hipSuccess) return attr;
     const int slices = (a.P + kPW - 1) / kPW;
-    hipLaunchKernelGGL(mamba_ssd_kernel, dim3(a.H * slices, batch), dim3(256), kSsdLds, stream, a);
+    hipLaunchKernelGGL(mamba_ssd_kernel, dim3(a.H * slices, batch), dim3(kSsdThreads), kSsdLds, stream, a);
     return hipGetLastError();
 }
 

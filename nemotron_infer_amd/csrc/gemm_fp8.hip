@@ -1155,6 +1155,10 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_w8a16_dma_kernel(const GemmAr
 // One workgroup per 32-row strip of a tile; a thread holds the partials' 16-byte pieces
 // of one lane of the main kernel's waves (so the loads are whole 1 KiB runs), rounds v into a
 // bf16 copy of the strip in LDS, and stores 16-byte row pieces as the main kernel's epilogue does.
+// Bound by memory latency more than by bytes (27 MB of partials at 2.4 TB/s): one round of workgroups,
+// each a chain of loads, so the loads are issued together -- residual, scales, then up to three
+// splits' pieces.  1000 x 3136 in four splits 12.4 -> 11.2 us, 777 x 3136 11.4 -> 10.6 us against the
+// splits one after the other with the residual loaded last.
 template <int BM, bool GROUPED>
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const GemmArgs a) {
     constexpr int TM = BM / 64, STRIPS = BM / 32, PITCH = 520;
@@ -1177,42 +1181,83 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const GemmArgs a
     const int wn = wave >> 1, i0 = 2 * (wave & 1);  // this wave's column half and first column block
     const int src = (wm * 2 + wn) * 64 + lane;      // the main kernel's thread
     const float4* part = reinterpret_cast<const float4*>(a.part + (size_t)r * a.splits * (BM * 256)) + src;
+    // everything but the partials first, so that one memory round trip covers all: the residual of
+    // this thread's row pieces (row p: 32-row strip row (tid / 32) + 8 p, 8 columns; y may be the
+    // residual) and the scales
+    const int c8 = (tid & 31) * 8, n = n0 + c8;
+    const bool full = G.vec16 && n + 7 < G.N;
+    uint4 rv[4];
+    if (G.epi == kEpiResidual) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const int row = min(m0 + (tid >> 5) + 8 * p, a.M - 1);
+            const uint16_t* rp = G.res + (int64_t)row * G.ldres + n;
+            if (full && G.vec16_res) {
+                rv[p] = *reinterpret_cast<const uint4*>(rp);
+            } else {
+                uint32_t w[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    w[e] = (n + 2 * e < G.N ? (uint32_t)rp[2 * e] : 0u) |
+                           ((n + 2 * e + 1 < G.N ? (uint32_t)rp[2 * e + 1] : 0u) << 16);
+                rv[p] = uint4{w[0], w[1], w[2], w[3]};
+            }
+        }
+    }
+    float4 sc[2][4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int gq = 0; gq < 4; ++gq) {
+            const int nl = n0 + wn * 128 + (i0 + i) * 32 + 8 * gq + 4 * h;
+            if (G.vec_scale && n0 + 256 <= G.N) {
+                sc[i][gq] = *reinterpret_cast<const float4*>(G.s + nl);
+            } else {
+                sc[i][gq] = float4{G.s[min(nl, G.N - 1)], G.s[min(nl + 1, G.N - 1)], G.s[min(nl + 2, G.N - 1)],
+                                   G.s[min(nl + 3, G.N - 1)]};
+            }
+        }
+    auto piece = [&](int sp, int i, int gq) {
+        return part[(size_t)sp * (BM * 64) + (((i0 + i) * TM + j) * 4 + gq) * 256];
+    };
     float4 v[2][4];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int gq = 0; gq < 4; ++gq) v[i][gq] = part[(((i0 + i) * TM + j) * 4 + gq) * 256];
-#pragma unroll 3
-    for (int sp = 1; sp < a.splits; ++sp) {
-        const float4* ps = part + (size_t)sp * (BM * 64);
-        float4 f[2][4];
+        for (int gq = 0; gq < 4; ++gq) v[i][gq] = piece(0, i, gq);
+    // the further splits two at a time: 16 pieces of each thread in flight (with the first split's,
+    // 24), added in split order
+    for (int sp = 1; sp < a.splits; sp += 2) {
+        const bool two = sp + 1 < a.splits;         // uniform
+        float4 f[2][2][4];
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int q = 0; q < 2; ++q)
 #pragma unroll
-            for (int gq = 0; gq < 4; ++gq) f[i][gq] = ps[(((i0 + i) * TM + j) * 4 + gq) * 256];
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+                for (int gq = 0; gq < 4; ++gq)
+                    if (q == 0 || two) f[q][i][gq] = piece(sp + q, i, gq);
 #pragma unroll
-            for (int gq = 0; gq < 4; ++gq) {
-                v[i][gq].x += f[i][gq].x; v[i][gq].y += f[i][gq].y;
-                v[i][gq].z += f[i][gq].z; v[i][gq].w += f[i][gq].w;
-            }
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int gq = 0; gq < 4; ++gq)
+                    if (q == 0 || two) {
+                        v[i][gq].x += f[q][i][gq].x; v[i][gq].y += f[q][i][gq].y;
+                        v[i][gq].z += f[q][i][gq].z; v[i][gq].w += f[q][i][gq].w;
+                    }
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int gq = 0; gq < 4; ++gq) {
             const int nl = wn * 128 + (i0 + i) * 32 + 8 * gq + 4 * h;
-            float sc[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) sc[e] = G.s[min(n0 + nl + e, G.N - 1)];
+            const float4 s4 = sc[i][gq];
             *reinterpret_cast<uint2*>(sm + l32 * PITCH + nl * 2) =
-                uint2{pack_bf16(v[i][gq].x * sc[0], v[i][gq].y * sc[1]), pack_bf16(v[i][gq].z * sc[2], v[i][gq].w * sc[3])};
+                uint2{pack_bf16(v[i][gq].x * s4.x, v[i][gq].y * s4.y), pack_bf16(v[i][gq].z * s4.z, v[i][gq].w * s4.w)};
         }
     __syncthreads();
-    const int c8 = (tid & 31) * 8, n = n0 + c8;
-    const bool full = G.vec16 && n + 7 < G.N;
-    const bool res16 = full && G.vec16_res;
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
         const int row = (tid >> 5) + 8 * p;
@@ -1221,19 +1266,9 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const GemmArgs a
         const uint2 v0 = sp[0], v1 = sp[1];
         uint32_t w[4] = {v0.x, v0.y, v1.x, v1.y};
         if (G.epi == kEpiResidual) {
-            const uint16_t* rp = G.res + (int64_t)(m0 + row) * G.ldres + n;
-            uint32_t rv[4];
-            if (res16) {
-                const uint4 r4 = *reinterpret_cast<const uint4*>(rp);
-                rv[0] = r4.x; rv[1] = r4.y; rv[2] = r4.z; rv[3] = r4.w;
-            } else {
+            const uint32_t r4[4] = {rv[p].x, rv[p].y, rv[p].z, rv[p].w};
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    rv[e] = (n + 2 * e < G.N ? (uint32_t)rp[2 * e] : 0u) |
-                            ((n + 2 * e + 1 < G.N ? (uint32_t)rp[2 * e + 1] : 0u) << 16);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) w[e] = add_bf16x2(w[e], rv[e]);
+            for (int e = 0; e < 4; ++e) w[e] = add_bf16x2(w[e], r4[e]);
         } else if (G.epi == kEpiRelu2) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) w[e] = relu2_bf16x2(w[e]);

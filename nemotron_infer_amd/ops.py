@@ -15,20 +15,23 @@ import torch
 from . import _lib
 
 
-def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+def _stream() -> int:
+    """torch's current stream as a hipStream_t, without building a torch.cuda.Stream (a call's
+    tensors are on a GPU, so torch's device state is set up)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _check_w(w: torch.Tensor, K: int | None = None) -> torch.Tensor:
-    """e4m3 weights [N, K] as uint8 codes; rows must be contiguous (stride(-1) == 1)."""
-    if w.dtype == torch.float8_e4m3fn:
-        w = w.view(torch.uint8)
-    elif w.dtype != torch.uint8:
+    """e4m3 weights [N, K], as float8_e4m3fn or uint8 codes (both read by address, shape and row
+    stride only); rows must be contiguous (stride(-1) == 1)."""
+    dtype = w.dtype
+    if dtype != torch.float8_e4m3fn and dtype != torch.uint8:
         raise TypeError(f"weights must be float8_e4m3fn or uint8 codes, got {w.dtype}")
-    if w.dim() != 2 or w.stride(-1) != 1:
+    shape = w.shape
+    if len(shape) != 2 or w.stride()[1] != 1:
         raise ValueError(f"weights must be a 2-D [N, K] matrix with contiguous rows (shape {tuple(w.shape)}, "
                          f"strides {w.stride()})")
-    if K is not None and w.shape[1] != K:
+    if K is not None and shape[1] != K:
         raise ValueError(f"weights have K = {w.shape[1]}, activations K = {K}")
     return w
 
@@ -37,25 +40,32 @@ def _check_s(s: torch.Tensor, N: int) -> torch.Tensor:
     """Per-row scales: contiguous float32 [N]."""
     if s.dtype != torch.float32:
         raise TypeError(f"w_scale must be float32, got {s.dtype}")
-    if s.dim() != 1 or s.numel() != N or not s.is_contiguous():
+    if s.shape != (N,) or not s.is_contiguous():
         raise ValueError(f"w_scale must be a contiguous float32 vector of N = {N} values (shape {tuple(s.shape)})")
     return s
 
 
 def _check_out(y: torch.Tensor, M: int, N: int, name: str = "out") -> torch.Tensor:
-    """An output buffer: contiguous bf16 holding exactly [M, N] (or [N] when M == 1), returned
-    as a 2-D view.  Anything else raises: a strided or copied view would silently receive
+    """An output buffer: contiguous bf16 holding exactly [M, N] (or [N] when M == 1), so its row
+    stride is N.  Anything else raises: a strided or copied view would silently receive
     the wrong elements or lose the results."""
     if y.dtype != torch.bfloat16:
         raise TypeError(f"{name} must be bfloat16, got {y.dtype}")
-    ok_shape = tuple(y.shape) == (M, N) or (M == 1 and tuple(y.shape) == (N,))
-    if not ok_shape or not y.is_contiguous():
+    shape = y.shape
+    if not (shape == (M, N) or (M == 1 and shape == (N,))) or not y.is_contiguous():
         raise ValueError(f"{name} must be a contiguous bf16 tensor of shape ({M}, {N}) "
                          f"(got shape {tuple(y.shape)}, strides {y.stride()})")
-    return y.view(M, N)
+    return y
 
 
 def _check_device(*ts: torch.Tensor) -> None:
+    if ts[0].is_cuda:
+        idx = ts[0].get_device()
+        for t in ts:
+            if t.get_device() != idx or not t.is_cuda:
+                break
+        else:
+            return
     dev = ts[0].device
     if dev.type != "cuda":
         raise ValueError(f"tensors must be on a GPU, got {dev}")
@@ -74,7 +84,7 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor | None:
     Grows on demand -- make one eager call of the largest shape before capturing a graph."""
     if nbytes <= 0:
         return None
-    idx = torch.device(device).index or 0
+    idx = (device if isinstance(device, torch.device) else torch.device(device)).index or 0
     ws = _WORKSPACE.get(idx)
     if ws is None or ws.numel() < nbytes:
         ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
@@ -96,7 +106,7 @@ def _as_2d(x: torch.Tensor):
     x2 = x.unsqueeze(0) if x.dim() == 1 else x
     if x2.dtype != torch.bfloat16:
         raise TypeError("x must be bfloat16")
-    if x2.stride(-1) != 1:
+    if x2.stride()[-1] != 1:
         raise ValueError("x must be contiguous in the last dimension")
     return x2
 
@@ -112,13 +122,13 @@ def linear_fp8_w8a16(x: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
     _check_s(w_scale, N)
     if out is None:
         out = torch.empty((N,) if squeeze else (M, N), dtype=torch.bfloat16, device=x.device)
-    y2 = _check_out(out, M, N)
-    _check_device(x2, w, w_scale, y2)
+    _check_out(out, M, N)
+    _check_device(x2, w, w_scale, out)
     L = _lib.lib()
     ws = _linear_ws(L, x.device, M, N, K) if use_workspace else None
     rc = L.nmi_linear_fp8_w8a16_ws(
         x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0), w_scale.data_ptr(),
-        y2.data_ptr(), y2.stride(0), M, N, K,
+        out.data_ptr(), N, M, N, K,
         None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _stream())
     _lib.check(rc, "nmi_linear_fp8_w8a16_ws")
     return out
@@ -140,10 +150,10 @@ def linear_fp8_w8a16_grouped(x: torch.Tensor, weights, outs=None, use_workspace:
     for i, ((w, s), y) in enumerate(zip(weights, outs)):
         w = _check_w(w, K)
         _check_s(s, w.shape[0])
-        y2 = _check_out(y, M, w.shape[0], f"outs[{i}]")
-        _check_device(x2, w, s, y2)
-        arr[i] = _lib.LinearGroup(w.data_ptr(), w.stride(0), s.data_ptr(), y2.data_ptr(), y2.stride(0),
-                                  w.shape[0])
+        N = w.shape[0]
+        _check_out(y, M, N, f"outs[{i}]")
+        _check_device(x2, w, s, y)
+        arr[i] = _lib.LinearGroup(w.data_ptr(), w.stride(0), s.data_ptr(), y.data_ptr(), N, N)
     L = _lib.lib()
     total = sum(w.shape[0] for w, _ in weights)
     ws = _linear_ws(L, x.device, M, total, K) if use_workspace else None
@@ -173,11 +183,11 @@ def linear_fp8_w8a16_batch(jobs, outs=None):
         K = x2.shape[1]
         w = _check_w(w, K)
         _check_s(s, w.shape[0])
-        y2 = _check_out(y, M, w.shape[0], f"outs[{i}]")
-        _check_device(x2, w, s, y2)
+        N = w.shape[0]
+        _check_out(y, M, N, f"outs[{i}]")
+        _check_device(x2, w, s, y)
         arr[i] = _lib.LinearJob(x2.data_ptr(), x2.stride(0), K,
-                                _lib.LinearGroup(w.data_ptr(), w.stride(0), s.data_ptr(), y2.data_ptr(),
-                                                 y2.stride(0), w.shape[0]))
+                                _lib.LinearGroup(w.data_ptr(), w.stride(0), s.data_ptr(), y.data_ptr(), N, N))
     _lib.check(_lib.lib().nmi_linear_fp8_w8a16_batch(arr, n, M, _stream()), "nmi_linear_fp8_w8a16_batch")
     return outs
 
@@ -216,12 +226,12 @@ def gemm_fp8_w8a16(x: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
     _check_s(w_scale, N)
     if out is None:
         out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-    y2 = _check_out(out, M, N)
-    _check_device(x2, w, w_scale, y2)
+    _check_out(out, M, N)
+    _check_device(x2, w, w_scale, out)
     L = _lib.lib()
     ws = _linear_ws(L, x.device, M, N, K) if use_workspace else None
     rc = L.nmi_gemm_fp8_w8a16(x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0),
-                              w_scale.data_ptr(), y2.data_ptr(), y2.stride(0), M, N, K,
+                              w_scale.data_ptr(), out.data_ptr(), N, M, N, K,
                               None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
                               _stream())
     _lib.check(rc, "nmi_gemm_fp8_w8a16")
@@ -267,7 +277,7 @@ def mlp_forward_fp8(x: torch.Tensor, norm_w: torch.Tensor, up_w: torch.Tensor, u
         raise ValueError(f"down_proj has {down_w.shape[0]} rows, hidden size is {hidden}")
     _check_s(up_s, inter)
     _check_s(down_s, hidden)
-    if norm_w.dtype != torch.float32 or tuple(norm_w.shape) != (hidden,) or not norm_w.is_contiguous():
+    if norm_w.dtype != torch.float32 or norm_w.shape != (hidden,) or not norm_w.is_contiguous():
         raise ValueError(f"norm_w must be a contiguous float32 vector of {hidden} values")
     if out is None:
         out = torch.empty_like(x)
@@ -293,7 +303,7 @@ def _block_ws(device: torch.device, need: int) -> torch.Tensor:
 
 
 def _check_bf16(t: torch.Tensor, shape, name: str) -> None:
-    if t.dtype != torch.bfloat16 or tuple(t.shape) != tuple(shape) or not t.is_contiguous():
+    if t.dtype != torch.bfloat16 or t.shape != shape or not t.is_contiguous():
         raise ValueError(f"{name} must be a contiguous bf16 tensor of shape {tuple(shape)}, "
                          f"got {t.dtype} {tuple(t.shape)}")
 
@@ -363,7 +373,7 @@ def attn_decode_fp8(x: torch.Tensor, norm_w: torch.Tensor, q_w, q_s, k_w, k_s, v
     _check_s(k_s, n_kv * 128)
     _check_s(v_s, n_kv * 128)
     _check_s(o_s, hidden)
-    if norm_w.dtype != torch.float32 or tuple(norm_w.shape) != (hidden,) or not norm_w.is_contiguous():
+    if norm_w.dtype != torch.float32 or norm_w.shape != (hidden,) or not norm_w.is_contiguous():
         raise ValueError(f"norm_w must be a contiguous float32 vector of {hidden} values")
     if out is None:
         out = torch.empty_like(x)
@@ -433,7 +443,7 @@ def attn_forward_fp8(x: torch.Tensor, norm_w: torch.Tensor, q_w, q_s, k_w, k_s, 
     _check_s(k_s, n_kv * 128)
     _check_s(v_s, n_kv * 128)
     _check_s(o_s, hidden)
-    if norm_w.dtype != torch.float32 or tuple(norm_w.shape) != (hidden,) or not norm_w.is_contiguous():
+    if norm_w.dtype != torch.float32 or norm_w.shape != (hidden,) or not norm_w.is_contiguous():
         raise ValueError(f"norm_w must be a contiguous float32 vector of {hidden} values")
     cap = 0
     if k_cache is not None or v_cache is not None:
@@ -460,7 +470,7 @@ def attn_forward_fp8(x: torch.Tensor, norm_w: torch.Tensor, q_w, q_s, k_w, k_s, 
 
 
 def _check_f32(t: torch.Tensor, shape, name: str) -> None:
-    if t.dtype != torch.float32 or tuple(t.shape) != tuple(shape) or not t.is_contiguous():
+    if t.dtype != torch.float32 or t.shape != shape or not t.is_contiguous():
         raise ValueError(f"{name} must be a contiguous float32 tensor of shape {tuple(shape)}, "
                          f"got {t.dtype} {tuple(t.shape)}")
 
@@ -522,7 +532,7 @@ def mamba_decode_fp8(x: torch.Tensor, norm_w: torch.Tensor, in_w, in_s, conv_w, 
         raise ValueError(f"out_proj has {out_w.shape[0]} rows, hidden size is {hidden}")
     _check_s(in_s, in_w.shape[0])
     _check_s(out_s, hidden)
-    if norm_w.dtype != torch.float32 or tuple(norm_w.shape) != (hidden,) or not norm_w.is_contiguous():
+    if norm_w.dtype != torch.float32 or norm_w.shape != (hidden,) or not norm_w.is_contiguous():
         raise ValueError(f"norm_w must be a contiguous float32 vector of {hidden} values")
     if out is None:
         out = torch.empty_like(x)
@@ -575,7 +585,7 @@ def mamba_forward_fp8(x: torch.Tensor, norm_w: torch.Tensor, in_w, in_s, conv_w,
         raise ValueError(f"out_proj has {out_w.shape[0]} rows, hidden size is {hidden}")
     _check_s(in_s, in_w.shape[0])
     _check_s(out_s, hidden)
-    if norm_w.dtype != torch.float32 or tuple(norm_w.shape) != (hidden,) or not norm_w.is_contiguous():
+    if norm_w.dtype != torch.float32 or norm_w.shape != (hidden,) or not norm_w.is_contiguous():
         raise ValueError(f"norm_w must be a contiguous float32 vector of {hidden} values")
     if out is None:
         out = torch.empty_like(x)

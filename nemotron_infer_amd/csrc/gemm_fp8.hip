@@ -1572,28 +1572,45 @@ bool dma_beats_short(int M, int N, int K, size_t ws_bytes) {
 }
 }  // namespace
 
-// A grouped GEMM (matrices sharing x) as one launch of the DMA-fed kernel where it takes every
-// matrix (automatic tile choice, M >= 512 or where that is the least modelled time); otherwise one
-// launch per matrix.  Measured (q | k | v, 5120 + 1024 + 1024 rows of K = 3136): see the attention
-// block's figures in attention.cpp.
+// A grouped GEMM (matrices sharing x) as one launch where a kernel takes every matrix (automatic
+// tile choice): from M = 512 the DMA-fed kernel; below, that or the short-prompt kernel by modelled
+// time, and always the latter up to kShortOnlyM rows; otherwise one launch per matrix.  Measured
+// (us; one launch DMA-fed / short-prompt), q | k | v of 5120 + 1024 + 1024 rows, K = 3136: M = 17 20.8 /
+// 12.8, 64 21.1 / 14.6, 100 22.1 / 19.5, 200 26.5 / 25.7, 300 30.9 / 37.7; of 2048 + 512 + 512 rows,
+// K = 2048: 17 15.0 / 7.4, 100 16.9 / 14.6, 256 25.0 / 19.2, 300 25.1 / 27.3; two of 8192, K = 2048: 17
+// 24.8 / 13.1, 128 25.6 / 23.3, 160 26.3 / 30.5.
 hipError_t launch_gemm_grouped(const uint16_t* x, int64_t ldx, int M, int K, const GemvGroup* g, int ng,
                                hipStream_t stream, void* ws, size_t ws_bytes) {
     const Tuning& t = tuning();
     bool one = ng > 1 && t.gemm_tile == 0;
     for (int i = 0; one && i < ng; ++i) one = dma_supported(x, ldx, g[i].W, g[i].ldw, M, g[i].N, K);
     const bool forced = t.gemm_bm != 0 && t.gemm_splits > 1;
-    if (one && M < 512 && !forced) {
-        one = t.gemm_short == 0 && t.gemm_splits <= 1 && t.gemm_sk != 1 && t.gemm_bm != 256;
-        const size_t wsb = ws ? ws_bytes : 0;
+    const size_t wsb = ws ? ws_bytes : 0;
+    // Below 512 rows all matrices as one launch of the short-prompt kernel where its K split fits the
+    // workspace, if the models say so (they are the single matrix's, over the rows of all).
+    bool shorts = ng > 1 && M < 512 && t.gemm_tile == 0 && t.gemm_short == 0 && t.gemm_splits == 0 && t.gemm_bm == 0 &&
+                  t.gemm_sk != 1;
+    int total_n = 0;
+    for (int i = 0; shorts && i < ng; ++i) {
+        shorts = gemm_short_supported(x, ldx, g[i].W, g[i].ldw, M, g[i].N, K) && g[i].N <= INT32_MAX - total_n;
+        if (shorts) total_n += g[i].N;
+    }
+    shorts = shorts && gemm_short_grouped_fits(M, g, ng, K, ws, wsb);
+    if (M < 512 && !forced && (one || shorts)) {
+        one = one && t.gemm_short == 0 && t.gemm_splits <= 1 && t.gemm_sk != 1 && t.gemm_bm != 256;
         int tn = 0;
         double separate = 0;
-        for (int i = 0; one && i < ng; ++i) {
+        for (int i = 0; i < ng; ++i) {
             tn += (g[i].N + 255) / 256;
             const double us = gemm_short_us(M, g[i].N, K, wsb);
-            separate += M <= kShortOnlyM ? us : std::min(us, dma_short_m_us(M, g[i].N, K, wsb));
+            separate += M <= kShortOnlyM || !one ? us : std::min(us, dma_short_m_us(M, g[i].N, K, wsb));
         }
-        one = one && dma_plan_ws(M, tn, K, ng, wsb).us < separate;
+        const double one_us = one ? dma_plan_ws(M, tn, K, ng, wsb).us : separate;
+        // 10%: its model is the less exact (two of 8192 x 2048 at M = 160: 25 modelled, 30.9 measured)
+        shorts = shorts && (M <= kShortOnlyM || 1.1 * gemm_short_us(M, total_n, K, wsb) < std::min(one_us, separate));
+        one = one && one_us < separate;
     }
+    if (shorts) return launch_gemm_short_grouped(x, ldx, M, K, g, ng, stream, ws);
     if (one) return launch_dma_groups(x, ldx, g, ng, M, K, stream, ws, ws_bytes);
     hipError_t e = hipSuccess;
     for (int i = 0; i < ng && e == hipSuccess; ++i)

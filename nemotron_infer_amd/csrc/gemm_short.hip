@@ -39,19 +39,26 @@ constexpr int kBK = 64;          // k per tile
 constexpr int kWaves = 4;
 constexpr size_t kFlagRegion = 64 * 1024;        // the workspace's counter / flag region, left alone
 
-struct ShortArgs {
-    const uint16_t* x;
-    int64_t ldx;
+// A weight matrix of a launch.  The groups of one launch share x and the K split.
+struct ShortGroup {
     const uint8_t* W;
     int64_t ldw;
     const float* s;
     uint16_t* y;
     int64_t ldy;
     float* part;             // [splits][M][N] float32 (splits > 1)
-    int M, N, K;
-    int tiles_n, splits, kt_per;
-    int part_vec;            // N % 4 == 0: 16-byte partial stores
+    int N;
+    int tile_begin;          // first tile of this matrix in the launch's numbering
+    int part_vec;            // partial rows 16-byte aligned: 16-byte stores
     Epi epi;
+};
+
+struct ShortArgs {
+    const uint16_t* x;
+    int64_t ldx;
+    int M, K;
+    int tiles_n, splits, kt_per, ngroups;
+    ShortGroup g[kMaxGroups];
 };
 
 // 16 bytes per lane from base + off to LDS [lds_addr + 16 lane] (LDS DMA).  Inline asm so that
@@ -86,7 +93,7 @@ __device__ __forceinline__ int wswz(int row, int q) { return q ^ ((row >> 2) & 3
 // The 4 waves form a WN x (4 / WN) grid; each wave computes TN 32-row blocks of W times TM
 // 32-row blocks of x, so a workgroup covers BN = 32 TN WN weight rows and BM = 32 TM (4 / WN) x
 // rows.  NS: LDS stages.
-template <int TN, int TM, int WN, int NS, int OCC>
+template <int TN, int TM, int WN, int NS, int OCC, bool GROUPED>
 __global__ __launch_bounds__(256, OCC) void gemm_short_kernel(const ShortArgs a) {
     constexpr int WM = kWaves / WN;
     constexpr int BN = 32 * TN * WN, BM = 32 * TM * WM;
@@ -106,7 +113,15 @@ __global__ __launch_bounds__(256, OCC) void gemm_short_kernel(const ShortArgs a)
     const int h = lane >> 5, l32 = lane & 31;
     const int wn = wave % WN, wm = wave / WN;
     const int tn = (int)blockIdx.x / a.splits, sp = (int)blockIdx.x % a.splits;
-    const int n0 = tn * BN, m0 = (int)blockIdx.y * BM;
+    int gi = 0;
+    if constexpr (GROUPED) {
+#pragma unroll
+        for (int i = 1; i < kMaxGroups; ++i)
+            if (i < a.ngroups && tn >= a.g[i].tile_begin) gi = i;
+        gi = __builtin_amdgcn_readfirstlane(gi);
+    }
+    const ShortGroup& G = a.g[gi];
+    const int n0 = (tn - G.tile_begin) * BN, m0 = (int)blockIdx.y * BM;
     const int KT = a.K / kBK;
     const int kt0 = sp * a.kt_per, kt1 = min(KT, kt0 + a.kt_per);
     const int nk = kt1 - kt0;
@@ -118,7 +133,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_short_kernel(const ShortArgs a)
 #pragma unroll
     for (int i = 0; i < WI; ++i) {
         const int r = (4 * i + wave) * 16 + (lane >> 2);
-        woff[i] = (uint32_t)(min(n0 + r, a.N - 1) * a.ldw + 16 * wswz(r, lane & 3));
+        woff[i] = (uint32_t)(min(n0 + r, G.N - 1) * G.ldw + 16 * wswz(r, lane & 3));
     }
 #pragma unroll
     for (int i = 0; i < XI; ++i) {
@@ -128,7 +143,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_short_kernel(const ShortArgs a)
     auto issue = [&](int j) {                      // k tile kt0 + j into stage j % NS
         const uint32_t sb = lds0 + (uint32_t)((j % NS) * STAGE);
         const int kt = kt0 + j;
-        const uint8_t* wb = a.W + (int64_t)kt * kBK;
+        const uint8_t* wb = G.W + (int64_t)kt * kBK;
         const uint8_t* xb = reinterpret_cast<const uint8_t*>(a.x) + (int64_t)kt * kBK * 2;
 #pragma unroll
         for (int i = 0; i < WI; ++i) dma16(wb, woff[i], sb + (4 * i + wave) * 1024);
@@ -190,24 +205,24 @@ __global__ __launch_bounds__(256, OCC) void gemm_short_kernel(const ShortArgs a)
     // m = m0 + 32 (TM wm + t) + l32.
     if (a.splits > 1) {
         // partial tile of this split, raw sums (the reduce kernel scales)
-        float* part = a.part + (size_t)sp * a.M * a.N;
+        float* part = G.part + (size_t)sp * a.M * G.N;
 #pragma unroll
         for (int t = 0; t < TM; ++t) {
             const int m = m0 + 32 * (TM * wm + t) + l32;
             if (m >= a.M) continue;
-            float* row = part + (size_t)m * a.N;
+            float* row = part + (size_t)m * G.N;
 #pragma unroll
             for (int u = 0; u < TN; ++u)
 #pragma unroll
                 for (int gq = 0; gq < 4; ++gq) {
                     const int n = n0 + 32 * (TN * wn + u) + 4 * h + 8 * gq;
-                    if (a.part_vec && n + 3 < a.N) {
+                    if (G.part_vec && n + 3 < G.N) {
                         *reinterpret_cast<float4*>(row + n) = float4{acc[u][t][4 * gq], acc[u][t][4 * gq + 1],
                                                                      acc[u][t][4 * gq + 2], acc[u][t][4 * gq + 3]};
                     } else {
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            if (n + e < a.N) row[n + e] = acc[u][t][4 * gq + e];
+                            if (n + e < G.N) row[n + e] = acc[u][t][4 * gq + e];
                     }
                 }
         }
@@ -220,10 +235,10 @@ __global__ __launch_bounds__(256, OCC) void gemm_short_kernel(const ShortArgs a)
 #pragma unroll
         for (int gq = 0; gq < 4; ++gq)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) sc[gq][e] = a.s[min(nb + 8 * gq + e, a.N - 1)];
+            for (int e = 0; e < 4; ++e) sc[gq][e] = G.s[min(nb + 8 * gq + e, G.N - 1)];
         // residuals first (y may be the residual), then the stores
         uint16_t res[TM][4][4];
-        if (a.epi.kind == kEpiResidual) {
+        if (G.epi.kind == kEpiResidual) {
 #pragma unroll
             for (int t = 0; t < TM; ++t) {
                 const int m = min(m0 + 32 * (TM * wm + t) + l32, a.M - 1);
@@ -231,22 +246,22 @@ __global__ __launch_bounds__(256, OCC) void gemm_short_kernel(const ShortArgs a)
                 for (int gq = 0; gq < 4; ++gq)
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        res[t][gq][e] = a.epi.res[(int64_t)m * a.epi.ldres + min(nb + 8 * gq + e, a.N - 1)];
+                        res[t][gq][e] = G.epi.res[(int64_t)m * G.epi.ldres + min(nb + 8 * gq + e, G.N - 1)];
             }
         }
 #pragma unroll
         for (int t = 0; t < TM; ++t) {
             const int m = m0 + 32 * (TM * wm + t) + l32;
             if (m >= a.M) continue;
-            uint16_t* yr = a.y + (int64_t)m * a.ldy;
+            uint16_t* yr = G.y + (int64_t)m * G.ldy;
 #pragma unroll
             for (int gq = 0; gq < 4; ++gq) {
                 const int n = nb + 8 * gq;
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (n + e < a.N)
-                        yr[n + e] = epilogue(acc[u][t][4 * gq + e], sc[gq][e], a.epi.kind,
-                                             a.epi.kind == kEpiResidual ? res[t][gq][e] : (uint16_t)0);
+                    if (n + e < G.N)
+                        yr[n + e] = epilogue(acc[u][t][4 * gq + e], sc[gq][e], G.epi.kind,
+                                             G.epi.kind == kEpiResidual ? res[t][gq][e] : (uint16_t)0);
             }
         }
     }
@@ -257,20 +272,21 @@ __global__ __launch_bounds__(256, OCC) void gemm_short_kernel(const ShortArgs a)
 // of up to 8 splits are loaded before any is added (one memory round trip for them, not one per
 // split), the scales and residuals before the partials.
 __global__ __launch_bounds__(256) void gemm_short_reduce_kernel(const ShortArgs a) {
+    const ShortGroup& G = a.g[blockIdx.y];
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int q_n = (a.N + 3) / 4;
+    const int q_n = (G.N + 3) / 4;
     if (i >= (int64_t)a.M * q_n) return;
     const int m = (int)(i / q_n), n = 4 * (int)(i % q_n);
-    const size_t stride = (size_t)a.M * a.N;
-    const float* p = a.part + (size_t)m * a.N + n;
-    const int cnt = min(4, a.N - n);
+    const size_t stride = (size_t)a.M * G.N;
+    const float* p = G.part + (size_t)m * G.N + n;
+    const int cnt = min(4, G.N - n);
     float sc[4], v[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int e = 0; e < 4; ++e) sc[e] = a.s[min(n + e, a.N - 1)];
+    for (int e = 0; e < 4; ++e) sc[e] = G.s[min(n + e, G.N - 1)];
     uint16_t r[4] = {0, 0, 0, 0};
-    if (a.epi.kind == kEpiResidual)
-        for (int e = 0; e < cnt; ++e) r[e] = a.epi.res[(int64_t)m * a.epi.ldres + n + e];
-    if (a.part_vec) {
+    if (G.epi.kind == kEpiResidual)
+        for (int e = 0; e < cnt; ++e) r[e] = G.epi.res[(int64_t)m * G.epi.ldres + n + e];
+    if (G.part_vec) {
         for (int s0 = 0; s0 < a.splits; s0 += 8) {
             float4 f[8];
 #pragma unroll
@@ -286,10 +302,10 @@ __global__ __launch_bounds__(256) void gemm_short_reduce_kernel(const ShortArgs 
         for (int sp = 0; sp < a.splits; ++sp)
             for (int e = 0; e < cnt; ++e) v[e] += p[sp * stride + e];
     }
-    uint16_t* yr = a.y + (int64_t)m * a.ldy + n;
+    uint16_t* yr = G.y + (int64_t)m * G.ldy + n;
     uint16_t o[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = epilogue(v[e], sc[e], a.epi.kind, r[e]);
+    for (int e = 0; e < 4; ++e) o[e] = epilogue(v[e], sc[e], G.epi.kind, r[e]);
     if (cnt == 4 && (reinterpret_cast<uintptr_t>(yr) & 7) == 0) {
         *reinterpret_cast<uint2*>(yr) = uint2{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
     } else {
@@ -297,15 +313,15 @@ __global__ __launch_bounds__(256) void gemm_short_reduce_kernel(const ShortArgs 
     }
 }
 
-template <int TN, int TM, int WN, int NS, int OCC>
-hipError_t launch_short_t(ShortArgs a, int tiles_m, hipStream_t stream) {
+template <int TN, int TM, int WN, int NS, int OCC, bool GROUPED>
+hipError_t launch_short_t(const ShortArgs& a, int tiles_m, hipStream_t stream) {
     constexpr int lds = NS * (32 * TN * WN * kBK + 32 * TM * (kWaves / WN) * kBK * 2);
     static_assert(lds * OCC <= 160 * 1024, "LDS of OCC workgroups per CU");
     static const hipError_t attr = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&gemm_short_kernel<TN, TM, WN, NS, OCC>), hipFuncAttributeMaxDynamicSharedMemorySize,
+        reinterpret_cast<const void*>(&gemm_short_kernel<TN, TM, WN, NS, OCC, GROUPED>), hipFuncAttributeMaxDynamicSharedMemorySize,
         lds);
     if (attr != hipSuccess) return attr;
-    hipLaunchKernelGGL((gemm_short_kernel<TN, TM, WN, NS, OCC>), dim3(a.tiles_n * a.splits, tiles_m), dim3(256), lds,
+    hipLaunchKernelGGL((gemm_short_kernel<TN, TM, WN, NS, OCC, GROUPED>), dim3(a.tiles_n * a.splits, tiles_m), dim3(256), lds,
                        stream, a);
     return hipGetLastError();
 }
@@ -367,10 +383,10 @@ int short_form(int M, int N) {
 
 }  // namespace
 
-int gemm_short_splits(int M, int N, int K) {
-    const ShortCfg& c = kForms[short_form(M, N)];
-    const int bn = c.bn(), bm = c.bm();
-    const int tiles = ((N + bn - 1) / bn) * ((M + bm - 1) / bm);
+// The K splits of `tiles_n` weight tiles of form c.
+static int short_splits(const ShortCfg& c, int tiles_n, int M, int K) {
+    const int bm = c.bm();
+    const int tiles = tiles_n * ((M + bm - 1) / bm);
     const int KT = K / kBK;
     if (tuning().gemm_splits > 0) return std::min(tuning().gemm_splits, KT);
     // one round of the form's target workgroups per CU, at least 4 k tiles each, and the partials
@@ -379,6 +395,11 @@ int gemm_short_splits(int M, int N, int K) {
     const int by_k = std::max(1, KT / 4);
     const int by_bytes = std::max(1, (int)((int64_t)K / (4 * (int64_t)M)));
     return std::max(1, std::min(want, std::min(by_k, by_bytes)));
+}
+
+int gemm_short_splits(int M, int N, int K) {
+    const ShortCfg& c = kForms[short_form(M, N)];
+    return short_splits(c, (N + c.bn() - 1) / c.bn(), M, K);
 }
 
 // Fitted to sweeps of M = 100 .. 511 on the model's projections and on N = 64 .. 2048 above M = 64
@@ -420,38 +441,87 @@ size_t gemm_short_workspace_bytes(int M, int N, int K) {
     return kFlagRegion + (size_t)rows * M * sizeof(float);
 }
 
+namespace {
+
+template <bool GROUPED>
+hipError_t launch_short_form(int form, const ShortArgs& a, int tiles_m, hipStream_t stream) {
+    switch (form) {
+        case 0: return launch_short_t<2, 1, 4, 7, 1, GROUPED>(a, tiles_m, stream);
+        case 1: return launch_short_t<1, 1, 4, 6, 2, GROUPED>(a, tiles_m, stream);
+        case 3: return launch_short_t<1, 2, 4, 4, 2, GROUPED>(a, tiles_m, stream);
+        case 6: return launch_short_t<2, 2, 2, 4, 1, GROUPED>(a, tiles_m, stream);
+        default: break;
+    }
+    if constexpr (!GROUPED) {                       // forms that only the tuning knob takes
+        switch (form) {
+            case 2: return launch_short_t<2, 2, 4, 6, 1, false>(a, tiles_m, stream);
+            case 4: return launch_short_t<1, 1, 2, 6, 2, false>(a, tiles_m, stream);
+            case 5: return launch_short_t<2, 4, 4, 4, 1, false>(a, tiles_m, stream);
+            case 7: return launch_short_t<1, 2, 2, 3, 2, false>(a, tiles_m, stream);
+            default: break;
+        }
+    }
+    return hipErrorInvalidValue;
+}
+
+// The launch behind both entries: the matrices in one grid, their partials one after the other.
+hipError_t launch_short_groups(const uint16_t* x, int64_t ldx, int M, int K, const GemvGroup* g, int ng, int form,
+                               int splits, void* ws, hipStream_t stream) {
+    const ShortCfg& c = kForms[form];
+    ShortArgs a{};
+    a.x = x; a.ldx = ldx; a.M = M; a.K = K; a.ngroups = ng;
+    const int KT = K / kBK;
+    a.kt_per = (KT + splits - 1) / splits;
+    a.splits = (KT + a.kt_per - 1) / a.kt_per;      // no empty split
+    float* part = a.splits > 1 ? reinterpret_cast<float*>(static_cast<char*>(ws) + kFlagRegion) : nullptr;
+    int64_t n4 = 0;
+    for (int i = 0; i < ng; ++i) {
+        const bool vec = g[i].N % 4 == 0 && (reinterpret_cast<uintptr_t>(part) & 15) == 0;
+        a.g[i] = ShortGroup{g[i].W, g[i].ldw, g[i].s, g[i].y, g[i].ldy, part, g[i].N, a.tiles_n, vec ? 1 : 0, g[i].epi};
+        a.tiles_n += (g[i].N + c.bn() - 1) / c.bn();
+        if (part) part += (size_t)a.splits * M * g[i].N;
+        n4 = std::max(n4, (int64_t)M * ((g[i].N + 3) / 4));
+    }
+    const int tiles_m = (M + c.bm() - 1) / c.bm();
+    const hipError_t e = ng > 1 ? launch_short_form<true>(form, a, tiles_m, stream)
+                                : launch_short_form<false>(form, a, tiles_m, stream);
+    if (e != hipSuccess || a.splits == 1) return e;
+    hipLaunchKernelGGL(gemm_short_reduce_kernel, dim3((unsigned)((n4 + 255) / 256), ng), dim3(256), 0, stream, a);
+    return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_gemm_short(const uint16_t* x, int64_t ldx, const uint8_t* W, int64_t ldw, const float* s,
                              uint16_t* y, int64_t ldy, int M, int N, int K, hipStream_t stream, const Epi& epi,
                              void* ws, size_t ws_bytes) {
-    const int form = short_form(M, N);
-    const ShortCfg& c = kForms[form];
-    ShortArgs a{};
-    a.x = x; a.ldx = ldx; a.W = W; a.ldw = ldw; a.s = s; a.y = y; a.ldy = ldy;
-    a.M = M; a.N = N; a.K = K; a.epi = epi;
-    a.tiles_n = (N + c.bn() - 1) / c.bn();
-    const int KT = K / kBK;
     int splits = gemm_short_splits(M, N, K);
     if (splits > 1 && (!ws || ws_bytes < kFlagRegion + (size_t)splits * M * N * sizeof(float))) splits = 1;
-    a.kt_per = (KT + splits - 1) / splits;
-    a.splits = (KT + a.kt_per - 1) / a.kt_per;      // no empty split
-    a.part = splits > 1 ? reinterpret_cast<float*>(static_cast<char*>(ws) + kFlagRegion) : nullptr;
-    a.part_vec = N % 4 == 0 ? 1 : 0;
-    const int tiles_m = (M + c.bm() - 1) / c.bm();
-    hipError_t e;
-    switch (form) {
-        case 0: e = launch_short_t<2, 1, 4, 7, 1>(a, tiles_m, stream); break;
-        case 1: e = launch_short_t<1, 1, 4, 6, 2>(a, tiles_m, stream); break;
-        case 2: e = launch_short_t<2, 2, 4, 6, 1>(a, tiles_m, stream); break;
-        case 3: e = launch_short_t<1, 2, 4, 4, 2>(a, tiles_m, stream); break;
-        case 4: e = launch_short_t<1, 1, 2, 6, 2>(a, tiles_m, stream); break;
-        case 5: e = launch_short_t<2, 4, 4, 4, 1>(a, tiles_m, stream); break;
-        case 6: e = launch_short_t<2, 2, 2, 4, 1>(a, tiles_m, stream); break;
-        default: e = launch_short_t<1, 2, 2, 3, 2>(a, tiles_m, stream); break;
-    }
-    if (e != hipSuccess || a.splits == 1) return e;
-    const int64_t n4 = (int64_t)M * ((N + 3) / 4);
-    hipLaunchKernelGGL(gemm_short_reduce_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, stream, a);
-    return hipGetLastError();
+    const GemvGroup g{W, ldw, s, y, ldy, N, 0, 0, epi};
+    return launch_short_groups(x, ldx, M, K, &g, 1, short_form(M, N), splits, ws, stream);
+}
+
+// A grouped call's matrices as one launch and one reduction, with one K split for all.
+bool gemm_short_grouped_fits(int M, const GemvGroup* g, int ng, int K, const void* ws, size_t ws_bytes) {
+    int64_t N = 0;
+    for (int i = 0; i < ng; ++i) N += g[i].N;
+    if (N > INT32_MAX) return false;
+    const ShortCfg& c = kForms[short_form(M, (int)N)];
+    int tiles = 0;
+    for (int i = 0; i < ng; ++i) tiles += (g[i].N + c.bn() - 1) / c.bn();
+    const int splits = short_splits(c, tiles, M, K);
+    return splits == 1 || (ws && ws_bytes >= kFlagRegion + (size_t)splits * M * N * sizeof(float));
+}
+
+hipError_t launch_gemm_short_grouped(const uint16_t* x, int64_t ldx, int M, int K, const GemvGroup* g, int ng,
+                                     hipStream_t stream, void* ws) {
+    int64_t N = 0;
+    for (int i = 0; i < ng; ++i) N += g[i].N;
+    const int form = short_form(M, (int)N);
+    const ShortCfg& c = kForms[form];
+    int tiles = 0;
+    for (int i = 0; i < ng; ++i) tiles += (g[i].N + c.bn() - 1) / c.bn();
+    return launch_short_groups(x, ldx, M, K, g, ng, form, short_splits(c, tiles, M, K), ws, stream);
 }
 
 }  // namespace nmi

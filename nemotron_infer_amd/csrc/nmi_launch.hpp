@@ -231,6 +231,11 @@ int mlp_forward_fp8(const void* input_bf16, const float* norm_w, const void* up_
 hipError_t launch_gemm_short(const uint16_t* x, int64_t ldx, const uint8_t* W, int64_t ldw, const float* s,
                              uint16_t* y, int64_t ldy, int M, int N, int K, hipStream_t stream, const Epi& epi,
                              void* ws, size_t ws_bytes);
+// The same kernel over up to kMaxGroups matrices that share x, as one launch (and one reduction)
+// with one K split: whether the workspace holds the split's partials, and the launch.
+bool gemm_short_grouped_fits(int M, const GemvGroup* g, int ng, int K, const void* ws, size_t ws_bytes);
+hipError_t launch_gemm_short_grouped(const uint16_t* x, int64_t ldx, int M, int K, const GemvGroup* g, int ng,
+                                     hipStream_t stream, void* ws);
 // Attention decode (sdpa_decode.hip): q [H, 128] against the caches [H_KV, cap, 128] over
 // positions [0, S), then K_new / V_new appended at position S; H / H_KV in 1..kSdpaMaxGroup.
 // The workspace (sdpa_decode_workspace_bytes) holds the fp32 partials of split launches.

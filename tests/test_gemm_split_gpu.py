@@ -146,6 +146,35 @@ def test_below_512_rows(M, Ns, K):
             assert_parity(bits(y), ref, f"M={M} group {i} ws={nbytes}", per_row_scales=True)
 
 
+# Matrices sharing x below 512 rows as one launch: every row-tile form of the short-prompt kernel, row
+# counts that are no multiple of 4 (the partials after them are unaligned), one k tile (no split), many.
+@pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 128, 129])
+@pytest.mark.parametrize("K", [64, 1088])
+def test_grouped_short(M, K):
+    Ns = (130, 77, 1, 260)
+    announce("gemm_grouped_short", M, Ns, K)
+    cases = [_case(M, N, K, 19 * i + M + N + K) for i, N in enumerate(Ns)]
+    xd = x_to_dev(cases[0][0])
+    wd = [(w_to_dev(w), s_to_dev(s)) for _, w, s in cases]
+    L = _lib.lib()
+    total = sum(Ns)
+    need = L.nmi_linear_workspace_bytes(M, total, K)
+    ws = torch.full((max(need, 256),), 255, dtype=torch.uint8, device=DEV)
+    ybig = torch.full((M, total + 3), 5.0, dtype=torch.bfloat16, device=DEV)
+    offs = np.cumsum((0,) + Ns)
+    arr = (_lib.LinearGroup * len(Ns))()
+    for i, (w, s) in enumerate(wd):
+        y = ybig[:, offs[i]:offs[i + 1]]
+        arr[i] = _lib.LinearGroup(w.data_ptr(), w.stride(0), s.data_ptr(), y.data_ptr(), y.stride(0), w.shape[0])
+    _lib.check(L.nmi_linear_fp8_w8a16_grouped(xd.data_ptr(), K, M, K, arr, len(Ns), ws.data_ptr(), need, None), "grouped")
+    torch.cuda.synchronize()
+    for i, (_, w, s) in enumerate(cases):
+        assert_parity(bits(ybig[:, offs[i]:offs[i + 1]]), oracle_bits(cases[0][0], w, s), f"M={M} K={K} group {i}",
+                      per_row_scales=True)
+    assert torch.all(ybig[:, total:] == 5.0)
+    assert torch.all(ws[:min(need, 65536)] == 255), "flag region written"
+
+
 # Groups of ragged column bands with K split in every tile height.
 @pytest.mark.parametrize("bm", [128, 192, 256])
 def test_grouped_split_tile_rows(bm):

@@ -100,6 +100,18 @@ def test_rmsnorm_matches_oracle(M, K):
     assert r["ok"] and r["n_diff"] <= max(1, 0.001 * y.size), r
 
 
+# the edges of one, two and four register pieces per thread, and the first K past them
+@pytest.mark.parametrize("M,K", [(3, 2048), (3, 2056), (2, 4096), (2, 8192), (2, 8200)])
+def test_rmsnorm_pieces_per_thread(M, K):
+    announce("rmsnorm", M, K)
+    x = _act(M, K, 40 + M)
+    w = (1.0 + 0.1 * np.random.default_rng(K).standard_normal(K)).astype(np.float32)
+    y = bits(ops.rmsnorm_bf16(x_to_dev(x), torch.from_numpy(w).to(DEV), EPS))
+    ref = block.rmsnorm_bf16(x, w, EPS)
+    r = linear.parity(y, ref)
+    assert r["ok"] and r["n_diff"] <= max(1, 0.001 * y.size), r
+
+
 def test_rmsnorm_zero_rows_and_binding():
     from nemotron_infer_amd.csrc import binding as B
 

@@ -86,17 +86,18 @@ __device__ __forceinline__ float silu_fast(float v) {
 // Vector form (row strides and the xBC column offset 16-byte aligned): one thread per (8
 // channels, 16-token run), 16-byte loads and stores of 8 channels; the run's 19 input rows are
 // all loaded before the first output is formed.
+template <int T>
 __global__ __launch_bounds__(256) void mamba_conv_prefill_vec_kernel(const MambaPrefillArgs a) {
     const int c0 = 8 * (int)(blockIdx.x * 256 + threadIdx.x);
-    const int t0 = blockIdx.y * kConvT;
+    const int t0 = blockIdx.y * T;
     const int b = blockIdx.z;
     if (c0 >= a.conv_dim || t0 >= a.S) return;
-    const int n = min(kConvT, a.S - t0);
+    const int n = min(T, a.S - t0);
     const uint16_t* xin = a.proj + (size_t)b * a.S * a.proj_ld + a.inter + c0;
     uint16_t* out = a.xc + (size_t)b * a.S * a.xc_ld + c0;
-    uint4 v[kConvT + 3];                                        // tokens t0 - 3 .. t0 + kConvT - 1
+    uint4 v[T + 3];                                        // tokens t0 - 3 .. t0 + T - 1
 #pragma unroll
-    for (int k = 0; k < kConvT + 3; ++k) {
+    for (int k = 0; k < T + 3; ++k) {
         const int t = t0 - 3 + k;
         v[k] = (t >= 0 && k < n + 3) ? load16(xin + (size_t)t * a.proj_ld) : uint4{0u, 0u, 0u, 0u};
     }
@@ -112,7 +113,7 @@ __global__ __launch_bounds__(256) void mamba_conv_prefill_vec_kernel(const Mamba
         return e & 1 ? bf16hi_to_f32(d) : bf16lo_to_f32(d);
     };
 #pragma unroll
-    for (int k = 0; k < kConvT; ++k) {
+    for (int k = 0; k < T; ++k) {
         float o[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -333,7 +334,6 @@ __device__ __forceinline__ float wave_incl_sum(float v) {
     return v + add;
 }
 __device__ __forceinline__ int bc_off(int row, int c) { return row * 256 + ((c ^ (row & 15)) << 4); }
-__device__ __forceinline__ int t_off(int row, int c) { return row * 128 + ((c ^ ((row >> 1) & 7)) << 4); }
 __device__ __forceinline__ int s_off(int p, int c) { return p * 256 + ((c ^ (p & 15)) << 4); }
 
 constexpr int kSsdWaves = 8, kSsdThreads = 64 * kSsdWaves;
@@ -650,12 +650,22 @@ hipError_t launch_mamba_prefill_mixer(const MambaPrefillArgs& a, int batch, hipS
     const bool vec = a.conv_dim % 8 == 0 && a.inter % 8 == 0 && a.proj_ld % 8 == 0 && a.xc_ld % 8 == 0 &&
                      (reinterpret_cast<uintptr_t>(a.proj) & 15) == 0 && (reinterpret_cast<uintptr_t>(a.xc) & 15) == 0 &&
                      (reinterpret_cast<uintptr_t>(a.conv_w) & 15) == 0;
-    if (vec)
-        hipLaunchKernelGGL(mamba_conv_prefill_vec_kernel,
-                           dim3((a.conv_dim / 8 + 255) / 256, (a.S + kConvT - 1) / kConvT, batch), dim3(256), 0, stream, a);
-    else
+    if (vec) {
+        // Tokens per thread: a longer run reads fewer rows twice (T + 3 per T), a shorter one leaves
+        // more workgroups for the latency and the SiLUs to spread over.  Measured (us, T = 16 / 8 / 4;
+        // 9728 channels): 64 tokens 8.5 / 5.8 / 4.6, 256 10.9 / 7.9 / 9.1, 2 x 500 16.4 / 15.0 / 15.4,
+        // 2048 24.6 / 25.5 / 28.0: 16 from two workgroups per CU, 8 from half a one, else 4.
+        const int64_t bx = (a.conv_dim / 8 + 255) / 256, cu = device_info().num_cu;
+        auto groups = [&](int T) { return bx * ((a.S + T - 1) / T) * batch; };
+        const int T = groups(16) >= 2 * cu ? 16 : 2 * groups(8) >= cu ? 8 : 4;
+        const auto kernel = T == 16  ? mamba_conv_prefill_vec_kernel<16>
+                            : T == 8 ? mamba_conv_prefill_vec_kernel<8>
+                                     : mamba_conv_prefill_vec_kernel<4>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)bx, (a.S + T - 1) / T, batch), dim3(256), 0, stream, a);
+    } else {
         hipLaunchKernelGGL(mamba_conv_prefill_kernel, dim3((a.conv_dim + 255) / 256, (a.S + kConvT - 1) / kConvT, batch),
                            dim3(256), 0, stream, a);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (tuning().mamba_scan == 1) {

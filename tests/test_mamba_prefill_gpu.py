@@ -149,6 +149,35 @@ def test_mamba_forward_two_sequences_past_512_rows():
         assert r["nan_ok"] and r["rel_l2_all"] <= 4e-3, (f"sequence {b}", r)
 
 
+@pytest.mark.parametrize("batch", [30, 180])
+def test_mamba_forward_many_sequences(batch):
+    """30 and 180 sequences of 45 tokens: enough conv workgroups for its 8- and its 16-token runs
+    (45 tokens end both in a partial run; the other tests here have 4-token runs).  The first and the
+    last sequence against the oracle on the GPU's own in_proj output, with the bars of the
+    600-row test above."""
+    announce("mamba_forward_many_sequences", batch)
+    W = _weights()
+    dw = _dev(W)
+    S = 45
+    x = _bf16_np((batch * S, HIDDEN), 8950)
+    xd = x_to_dev(x)
+    cs = torch.zeros((batch, CONV_DIM, 3), device=DEV)
+    ss = torch.zeros((batch, H, P, N), device=DEV)
+    out = bits(ops.mamba_forward_fp8(xd, *dw, H, P, G, batch=batch, conv_state_out=cs, ssm_state_out=ss, eps=EPS))
+    h = ops.rmsnorm_bf16(xd, dw[0], EPS)
+    proj = bits(ops.linear_fp8_w8a16(h, dw[1], dw[2]))
+    torch.cuda.synchronize()
+    for b in (0, batch - 1):
+        rows = slice(b * S, (b + 1) * S)
+        yr, csr, ssr = _oracle_mixer_sequence(proj[rows], W["prm"])
+        assert np.array_equal(cs.cpu().numpy()[b:b + 1], csr), f"conv state {b}"
+        _check_state(ss.cpu().numpy()[b:b + 1], ssr, f"ssm state {b}")
+        g_ref = mamba.gated_rmsnorm(yr, proj[rows, :INTER], W["prm"]["gnorm_w"], G, EPS)
+        out_ref = block.add_bf16(x[rows], linear.linear_fp8_w8a16(g_ref, *W["out"]))
+        r = linear.parity(out[rows], out_ref)
+        assert r["nan_ok"] and r["rel_l2_all"] <= 4e-3, (f"sequence {b}", r)
+
+
 def test_mamba_forward_batch_and_decode_continuation():
     """Two sequences in one call equal two single-sequence calls (outputs and states); then
     decode steps continue from the prefill's states as they would from a token-by-token

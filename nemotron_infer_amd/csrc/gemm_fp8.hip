@@ -1562,13 +1562,16 @@ namespace {
 // 12544 x 3136 68.5 / 35.5, 400 x 3136 x 12544 57.0 / 46.7, 500 x 3136 x 7680 39.8 / 36.5; but 200 x 3136
 // x 12544 33.7 / 34.4, 256 x 7168 x 3136 24.8 / 24.9, 511 x 1024 x 12544 27.6 / 34.6; and fewer rows
 // than a column band stay with the short kernel (300 x 64 x 2048 23.6 / 26.0), as do its own knobs.
+// 10% for the DMA-fed kernel: on inputs that the launch before it wrote it loses some of its lead
+// (200 x 12544 x 3136 alone 37.6 / 34.8, but the MLP block at M = 196 71.4 with the short kernel and
+// 73.8 with this one).
 double dma_short_m_us(int M, int N, int K, size_t ws_bytes) {
     return dma_plan_ws(M, (N + 255) / 256, K, 1, ws_bytes).us;
 }
 bool dma_beats_short(int M, int N, int K, size_t ws_bytes) {
     const Tuning& t = tuning();
     if (M <= kShortOnlyM || N < 256 || t.gemm_short != 0 || t.gemm_splits > 1 || t.gemm_sk == 1 || t.gemm_bm == 256) return false;
-    return dma_short_m_us(M, N, K, ws_bytes) < gemm_short_us(M, N, K, ws_bytes);
+    return 1.1 * dma_short_m_us(M, N, K, ws_bytes) < gemm_short_us(M, N, K, ws_bytes);
 }
 }  // namespace
 

@@ -1393,7 +1393,8 @@ DmaPlan dma_plan(int M, int tiles_n, int K, int ng, bool may_split) {
             const bool forced = t.gemm_splits > 0 && sp == t.gemm_splits;
             if (sp > 1) {
                 if (!may_split || sp > KT || T * sp > (int64_t)4 * G) break;
-                if (t.gemm_splits > 0 ? !forced : ((ng == 1 && K < kMinSplitK) || T * sp > G)) continue;
+                if (t.gemm_splits > 0 && !forced) continue;
+                if (t.gemm_splits <= 0 && ((ng == 1 && K < kMinSplitK) || T * sp > G)) break;
             }
             DmaPlan p{c.bm, (int)T, sp, 0.0};
             const int64_t rounds = (T * sp + G - 1) / G;
@@ -1542,16 +1543,20 @@ size_t gemm_workspace_bytes(int M) {
 
 // The K split's partial tiles for N rows of one matrix, or of up to kMaxGroups below M = 512
 // (after the 64 KiB flag region, which it leaves alone); 0 where dma_plan does not split.  Groups
-// have up to kMaxGroups - 1 more column bands than one matrix of their rows.
+// have up to kMaxGroups - 1 more column bands than one matrix of their rows.  Up to kShortOnlyM rows the
+// short-prompt kernel, whose partials are smaller, takes both (the block entries ask for this on
+// every call: five plans took 1-2 us, four such questions 9 us of an attention block's call).
 size_t gemm_split_workspace_bytes(int M, int64_t N, int K) {
     if (M < 1 || K % kBK != 0 || N > (1 << 30) || tuning().gemm_sk == 1) return 0;
+    if (M <= kShortOnlyM && tuning().gemm_splits <= 1) return 0;
+    const int tn = (int)((N + 255) / 256);
     size_t bytes = 0;
-    for (int more = 0; more < (M < 512 ? kMaxGroups : 1); ++more) {
-        for (int ng = 1; ng <= (M < 512 ? 2 : 1); ++ng) {
-            const DmaPlan p = dma_plan(M, (int)((N + 255) / 256) + more, K, ng, true);
-            if (p.splits > 1) bytes = std::max(bytes, kSkFlagBytes + p.part_bytes());
-        }
-    }
+    auto plan = [&](int tiles_n, int ng) {
+        const DmaPlan p = dma_plan(M, tiles_n, K, ng, true);
+        if (p.splits > 1) bytes = std::max(bytes, kSkFlagBytes + p.part_bytes());
+    };
+    plan(tn, 1);
+    for (int more = 0; M < 512 && more < kMaxGroups; ++more) plan(tn + more, 2);
     return bytes;
 }
 

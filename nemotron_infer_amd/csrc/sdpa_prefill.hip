@@ -23,8 +23,10 @@
 //   accumulators are rescaled rarely); keys after the query masked on the diagonal blocks only.
 // * O^T += V^T . P^T: P is the B operand straight from the score registers -- a 16-key step's
 //   lane-half h holds keys {4h..4h+3, 8+4h..8+4h+3} -- in two bf16 parts (hi = bf16(p), lo =
-//   bf16(p - hi)), so the weights carry about 16 significant bits and the float32 row sums stay
-//   consistent with them.  The V^T operand, in the same key order, comes from two transposing
+//   bf16(p - hi)), so the weights carry about 16 significant bits.  The row sum is float32: a block's
+//   16 weights in a lane first, then one add per block, so that its error grows with the blocks and
+//   not with the keys (one running sum over all keys was off by 6e-5 in a flat row of 8192, this
+//   by 2e-6).  The V^T operand, in the same key order, comes from two transposing
 //   LDS reads (ds_read_b64_tr_b16) of the token-major V tile.
 // The three run as a pipeline over blocks: while the matrix cores do the products with V of block g
 // and the scores of block g + 2, the same wave's vector unit turns the scores of block g + 1 into
@@ -237,6 +239,7 @@ __global__ __launch_bounds__(256, 2) void sdpa_prefill_kernel(const PrefillArgs 
         uint32_t hi[8], lo[8];
     };
     float p0 = 0.f, p1 = 0.f;
+    float psum = 0.f;                   // the 16 weights' sum, added to l by their block (see below)
     // pin: keeps the computation of x in the slot it is written in (the compiler otherwise sinks it
     // to the block that uses it, past all the MFMAs meant to hide it)
     auto pin = [](auto& x) __attribute__((always_inline)) { asm volatile("" : "+v"(x)); };
@@ -248,10 +251,9 @@ __global__ __launch_bounds__(256, 2) void sdpa_prefill_kernel(const PrefillArgs 
             pin(p1);
         } else if (stage == 1) {
             w.hi[i] = pack_bf16(p0, p1);
-            l += p0;
-            l += p1;
+            psum = i == 0 ? p0 + p1 : psum + p0 + p1;
             pin(w.hi[i]);
-            pin(l);
+            pin(psum);
         } else {
             // (v_dot2 would save the unpacking of hi, but beside MFMAs each costs 16 cycles and more)
             w.lo[i] = pack_bf16(p0 - bf16lo_to_f32(w.hi[i]), p1 - bf16hi_to_f32(w.hi[i]));
@@ -321,6 +323,7 @@ __global__ __launch_bounds__(256, 2) void sdpa_prefill_kernel(const PrefillArgs 
             mask(nxt, kvb2);
             tmax = row_max(nxt);
         }
+        l += psum;                      // block g + 1's, still under the max its weights were formed with
         settle();
         raise_max(tmax);
     };
@@ -408,6 +411,7 @@ __global__ __launch_bounds__(256, 2) void sdpa_prefill_kernel(const PrefillArgs 
 #pragma unroll
             for (int st = 0; st < 3; ++st) weigh(sa, mc, i, st, wa);
     }
+    l += psum;
     raise_max(row_max(sb));
     // the rest landed; and slots 0 and 1 are refilled in tile 0: every wave's reads of them first
     publish();

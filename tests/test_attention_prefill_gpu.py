@@ -59,6 +59,40 @@ def test_sdpa_prefill_long_prompts(S):
     assert_parity(bits(o), attention.sdpa_prefill(q, k, v, n_kv), f"S={S}")
 
 
+# The largest error of the softmax row sum of a query with n keys, relative: each lane half adds 16
+# weights of a 32-key block, then the block's sum to its running sum, so no chain of float32 adds of
+# positive terms is longer than 16 + n / 32 (2^-24 each); 8 more for the weight (the argument's
+# rounding and v_exp_f32), the last exchange and the division.
+def _row_sum_bound(n):
+    return (24 + n / 32) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("step", [1.0, 8.0, 16.0])
+def test_sdpa_prefill_row_sum_of_flat_rows(step):
+    """Rows whose weights are all alike but the first: key 0 scores `step` above the others, and only
+    its value is not zero, so O = v / l exactly but for the row sum l = 1 + i c.  8192 rows x 128
+    values put quotients at every distance from a bf16 tie: one that rounds to the other side
+    than the float64 quotient does must lie within the row sum's bound of that tie."""
+    S = 8192
+    announce("sdpa_prefill_flat_rows", S, step)
+    q = torch.zeros((S, D), dtype=torch.bfloat16, device=DEV)
+    k, v = torch.zeros_like(q), torch.zeros_like(q)
+    q[:, 0], k[0, 0] = 1.0, step
+    v[0] = 1.0 + torch.arange(D, device=DEV) / D
+    o = ops.sdpa_prefill_bf16(q, k, v, 1, 1)
+    torch.cuda.synchronize()
+    c = 2.0 ** (-step * float(np.float32(np.log2(np.e) / np.sqrt(128.0))))
+    exact = (1.0 + np.arange(D) / D)[None, :] / (1.0 + c * np.arange(S))[:, None]
+    got = linear.bf16_to_f32(bits(o)).astype(np.float64)
+    ref = linear.bf16_to_f32(block.bf16_round_exact(exact)).astype(np.float64)
+    rows, cols = np.nonzero(got != ref)
+    tie = 0.5 * (got + ref)[rows, cols]
+    off = np.abs(tie - exact[rows, cols]) / exact[rows, cols]
+    beyond = off > _row_sum_bound(rows + 1)
+    assert not beyond.any(), (f"{beyond.sum()} of {rows.size} flipped quotients lie beyond the bound, the farthest "
+                              f"{off.max():.1e} from its tie")
+
+
 @pytest.mark.parametrize("H,n_kv", [(8, 8), (12, 4), (6, 1), (16, 2)])
 def test_sdpa_prefill_gqa_and_packed_rows(H, n_kv):
     """q, k and v as column slices of one packed [S, (H + 2 n_kv) * 128] buffer (the layout of a

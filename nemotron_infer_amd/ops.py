@@ -74,32 +74,21 @@ def _check_device(*ts: torch.Tensor) -> None:
             raise ValueError(f"all tensors must be on {dev}, got {t.device}")
 
 
-_WORKSPACE: dict[int, torch.Tensor] = {}
-
-
-def workspace(device: torch.device, nbytes: int) -> torch.Tensor | None:
-    """Per-device workspace of the short-prompt GEMM's K split: zero-filled when (re)allocated,
-    kept for the process; every launch leaves it ready for the next.  Calls on one device
-    share it, so they must be ordered on one stream (as torch's current stream orders them).
-    Grows on demand -- make one eager call of the largest shape before capturing a graph."""
-    if nbytes <= 0:
-        return None
-    idx = (device if isinstance(device, torch.device) else torch.device(device)).index or 0
-    ws = _WORKSPACE.get(idx)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-        _WORKSPACE[idx] = ws
-    return ws
+def _workspace(device: torch.device, need: int) -> torch.Tensor | None:
+    """The transient device memory of one call (None where it needs none), from torch's allocator
+    like any temporary of the current stream: calls on other streams and threads, and graphs
+    captured with torch.cuda.graph (whose pool it then comes from), never share it, and nothing
+    outlives the call.  The kernels write what they read of it."""
+    return torch.empty(need, dtype=torch.uint8, device=device) if need else None
 
 
 def _linear_ws(L, device: torch.device, M: int, N: int, K: int) -> torch.Tensor | None:
-    """The workspace of one linear call.  From M = 512 the K split's partials (up to 64 MiB) come
-    from torch's allocator for this call, ordered on the current stream like any temporary, so
-    calls on several streams share nothing; below, the per-device tensor of workspace()."""
-    need = L.nmi_linear_workspace_bytes(M, N, K)
-    if need and M >= 512 and not L.nmi_linear_workspace_needs_zero(M):
-        return torch.empty(need, dtype=torch.uint8, device=device)
-    return workspace(device, need)
+    """_workspace() of a linear.  Only the stream-K form (a tuning knob, from M = 512) reads what it
+    has not written: its flags, in the first 64 KiB."""
+    ws = _workspace(device, L.nmi_linear_workspace_bytes(M, N, K))
+    if ws is not None and M >= 512 and L.nmi_linear_workspace_needs_zero(M):
+        ws[:_lib.NMI_WS_ERROR_OFFSET + 4].zero_()
+    return ws
 
 
 def _as_2d(x: torch.Tensor):
@@ -256,15 +245,12 @@ def rmsnorm_bf16(x: torch.Tensor, w: torch.Tensor, eps: float = 1e-5,
     return out
 
 
-_BLOCK_WS: dict[int, torch.Tensor] = {}
-
-
 def mlp_forward_fp8(x: torch.Tensor, norm_w: torch.Tensor, up_w: torch.Tensor, up_s: torch.Tensor,
                     down_w: torch.Tensor, down_s: torch.Tensor, out: torch.Tensor | None = None,
                     eps: float = 1e-5, use_workspace: bool = True) -> torch.Tensor:
     """The fp8 MLP block (model/mlp_block.cuh:121-176): out = x + down(relu(up(rmsnorm(x)))^2).
     x, out: [M, hidden] bf16; up_w [inter, hidden], down_w [hidden, inter] e4m3 with per-row
-    float32 scales.  The transient buffers come from a per-device tensor kept for the process
+    float32 scales.  The transient buffers come from torch's allocator, for this call
     (or, with use_workspace=False, from the library's bump allocator)."""
     x2 = _as_2d(x)
     if not x2.is_contiguous():
@@ -284,22 +270,13 @@ def mlp_forward_fp8(x: torch.Tensor, norm_w: torch.Tensor, up_w: torch.Tensor, u
     _check_out(out, M, hidden) if x.dim() == 2 else _check_out(out, 1, hidden)
     _check_device(x2, norm_w, up_w, up_s, down_w, down_s, out)
     L = _lib.lib()
-    ws = _block_ws(x.device, L.nmi_mlp_workspace_bytes(M, hidden, inter)) if use_workspace else None
+    ws = _workspace(x.device, L.nmi_mlp_workspace_bytes(M, hidden, inter)) if use_workspace else None
     rc = L.nmi_mlp_forward_fp8(x2.data_ptr(), norm_w.data_ptr(), up_w.data_ptr(), up_s.data_ptr(),
                                down_w.data_ptr(), down_s.data_ptr(), out.data_ptr(), M, hidden, inter, eps,
                                None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
                                _stream())
     _lib.check(rc, "nmi_mlp_forward_fp8")
     return out
-
-
-def _block_ws(device: torch.device, need: int) -> torch.Tensor:
-    idx = device.index or 0
-    ws = _BLOCK_WS.get(idx)
-    if ws is None or ws.numel() < need:
-        ws = torch.empty(max(need, 1 << 20), dtype=torch.uint8, device=device)
-        _BLOCK_WS[idx] = ws
-    return ws
 
 
 def _check_bf16(t: torch.Tensor, shape, name: str) -> None:
@@ -337,7 +314,7 @@ def sdpa_decode_bf16(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     _check_device(q, k_cache, v_cache, k_new, v_new, out)
     L = _lib.lib()
     need = L.nmi_sdpa_decode_workspace_bytes(H, n_kv, S_cache)
-    ws = _block_ws(q.device, need) if need else None
+    ws = _workspace(q.device, need)
     rc = L.nmi_sdpa_decode_bf16(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
                                 k_new.data_ptr(), v_new.data_ptr(), S_cache, cap, H, n_kv,
                                 None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _stream())
@@ -382,7 +359,7 @@ def attn_decode_fp8(x: torch.Tensor, norm_w: torch.Tensor, q_w, q_s, k_w, k_s, v
     L = _lib.lib()
     ws = None
     if use_workspace:
-        ws = _block_ws(x.device, L.nmi_attn_decode_workspace_bytes(hidden, H, n_kv, S_cache))
+        ws = _workspace(x.device, L.nmi_attn_decode_workspace_bytes(hidden, H, n_kv, S_cache))
     rc = L.nmi_attn_decode_fp8(x2.data_ptr(), norm_w.data_ptr(), q_w.data_ptr(), q_s.data_ptr(), k_w.data_ptr(),
                                k_s.data_ptr(), v_w.data_ptr(), v_s.data_ptr(), o_w.data_ptr(), o_s.data_ptr(),
                                k_cache.data_ptr(), v_cache.data_ptr(), S_cache, cap, out.data_ptr(), hidden, H, n_kv,
@@ -413,7 +390,7 @@ def sdpa_prefill_bf16(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, n_heads
     _check_device(q, k, v, out)
     L = _lib.lib()
     need = L.nmi_sdpa_prefill_workspace_bytes(n_kv_heads, S)     # 0: the kernel reads q, k, v in place
-    ws = _block_ws(q.device, need) if need else None
+    ws = _workspace(q.device, need)
     rc = L.nmi_sdpa_prefill_bf16(q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
                                  out.data_ptr(), out.stride(0), S, n_heads, n_kv_heads,
                                  ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0,
@@ -459,7 +436,7 @@ def attn_forward_fp8(x: torch.Tensor, norm_w: torch.Tensor, q_w, q_s, k_w, k_s, 
     _check_out(out, S, hidden) if x.dim() == 2 else _check_out(out, 1, hidden)
     _check_device(x2, norm_w, q_w, q_s, k_w, k_s, v_w, v_s, o_w, o_s, out)
     L = _lib.lib()
-    ws = _block_ws(x.device, L.nmi_attn_forward_workspace_bytes(S, hidden, H, n_kv)) if use_workspace else None
+    ws = _workspace(x.device, L.nmi_attn_forward_workspace_bytes(S, hidden, H, n_kv)) if use_workspace else None
     rc = L.nmi_attn_forward_fp8(x2.data_ptr(), norm_w.data_ptr(), q_w.data_ptr(), q_s.data_ptr(), k_w.data_ptr(),
                                 k_s.data_ptr(), v_w.data_ptr(), v_s.data_ptr(), o_w.data_ptr(), o_s.data_ptr(),
                                 out.data_ptr(), S, None if k_cache is None else k_cache.data_ptr(),
@@ -542,7 +519,7 @@ def mamba_decode_fp8(x: torch.Tensor, norm_w: torch.Tensor, in_w, in_s, conv_w, 
     L = _lib.lib()
     ws = None
     if use_workspace:
-        ws = _block_ws(x.device, L.nmi_mamba_decode_workspace_bytes(batch, hidden, n_heads, head_dim, n_groups, 128))
+        ws = _workspace(x.device, L.nmi_mamba_decode_workspace_bytes(batch, hidden, n_heads, head_dim, n_groups, 128))
     rc = L.nmi_mamba_decode_fp8(x2.data_ptr(), norm_w.data_ptr(), in_w.data_ptr(), in_s.data_ptr(), conv_w.data_ptr(),
                                 conv_b.data_ptr(), A_log.data_ptr(), D.data_ptr(), dt_bias.data_ptr(),
                                 gnorm_w.data_ptr(), out_w.data_ptr(), out_s.data_ptr(), conv_state.data_ptr(),
@@ -594,7 +571,7 @@ def mamba_forward_fp8(x: torch.Tensor, norm_w: torch.Tensor, in_w, in_s, conv_w,
     L = _lib.lib()
     ws = None
     if use_workspace:
-        ws = _block_ws(x.device, L.nmi_mamba_forward_workspace_bytes(batch, S, hidden, n_heads, head_dim, n_groups,
+        ws = _workspace(x.device, L.nmi_mamba_forward_workspace_bytes(batch, S, hidden, n_heads, head_dim, n_groups,
                                                                      128))
     rc = L.nmi_mamba_forward_fp8(x2.data_ptr(), norm_w.data_ptr(), in_w.data_ptr(), in_s.data_ptr(), conv_w.data_ptr(),
                                  conv_b.data_ptr(), A_log.data_ptr(), D.data_ptr(), dt_bias.data_ptr(),

@@ -2,11 +2,13 @@
 //
 // Behaviour of nemotron::BumpAllocator (nemotron_infer/csrc/include/tensor/allocator.cuh:58-175):
 // 64 MiB slabs (larger when one request needs more), 128-byte aligned blocks, rewind() moves
-// the cursor back to slab 0 and keeps every slab so that replaying the same (or a smaller)
-// sequence of requests after a rewind touches no hipMalloc, reset() frees all slabs.
-// Differences: failures are returned as status codes instead of abort()
-// (allocator.cuh:158-163), and the allocator object is never destroyed at process exit (a
-// static destructor calling hipFree after the HIP runtime has shut down is unsafe).
+// the cursor back to slab 0 and keeps every slab so that replaying any sequence of requests that ran
+// before after a rewind touches no hipMalloc, reset() frees all slabs.
+// Here a request tries every slab after the current one before a new slab is made (with the next
+// one only, two sequences replayed in turn added a slab on each round), failures are returned as
+// status codes instead of abort() (allocator.cuh:158-163), and the allocator object is never
+// destroyed at process exit (a static destructor calling hipFree after the HIP runtime has shut
+// down is unsafe).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -29,8 +31,12 @@ public:
         std::lock_guard<std::mutex> lock(mu_);
         const size_t need = (std::max<size_t>(bytes, 1) + kAlign - 1) & ~(kAlign - 1);
         if (slabs_.empty() || offset_ + need > slabs_[cur_].size) {
-            if (!slabs_.empty() && cur_ + 1 < slabs_.size() && need <= slabs_[cur_ + 1].size) {
-                ++cur_;                       // replay after rewind(): reuse the next slab
+            // the first later slab that holds it (a replay after rewind() finds the one it took before:
+            // the slabs between were too small then too)
+            size_t next = slabs_.empty() ? 0 : cur_ + 1;
+            while (next < slabs_.size() && need > slabs_[next].size) ++next;
+            if (next < slabs_.size()) {
+                cur_ = next;
                 offset_ = 0;
             } else {
                 void* p = nullptr;

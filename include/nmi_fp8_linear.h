@@ -259,7 +259,11 @@ int nmi_rmsnorm_bf16(const void* x_bf16, const float* w, void* y_bf16, int M, in
  * from M = 512 the GEMMs' stream-K region, whose flags each call zeroes with one small kernel);
  * calls that may overlap in time need distinct workspaces.  NULL
  * takes it from the bump allocator (nmi_alloc, so a slab may be hipMalloc'd), valid until
- * nmi_alloc_rewind(), as the reference's blocks do (binding.cu:7-9).
+ * nmi_alloc_rewind(), as the reference's blocks do (binding.cu:7-9).  The size is not largest at the
+ * most rows (the K split's partials: hidden 3136, inter 12544 64 MB at M = 2048, 110 MB at 1536); a
+ * smaller workspace that holds everything but those partials is accepted, and taken where the
+ * allocator cannot give the whole (out of memory; under stream capture, no slab with the room), the
+ * projections then running without that split.  The same holds for the other blocks below.
  * Requires M >= 1, hidden and inter positive multiples of 16, input, norm_w and both weights
  * 16-byte aligned, scales 4-byte aligned, out 2-byte aligned.
  */

@@ -27,7 +27,8 @@ public:
     static constexpr size_t kSlabBytes = 64ull << 20;
     static constexpr size_t kAlign = 128;
 
-    int allocate(size_t bytes, void** out) {
+    // grow = false: from the slabs there are, or NMI_ERR_ALLOC without a HIP call
+    int allocate(size_t bytes, void** out, bool grow = true) {
         std::lock_guard<std::mutex> lock(mu_);
         const size_t need = (std::max<size_t>(bytes, 1) + kAlign - 1) & ~(kAlign - 1);
         if (slabs_.empty() || offset_ + need > slabs_[cur_].size) {
@@ -38,6 +39,8 @@ public:
             if (next < slabs_.size()) {
                 cur_ = next;
                 offset_ = 0;
+            } else if (!grow) {
+                return NMI_ERR_ALLOC;
             } else {
                 void* p = nullptr;
                 const size_t sz = std::max(kSlabBytes, need);
@@ -45,6 +48,7 @@ public:
                 if (e != hipSuccess) {
                     set_last_error("nmi_alloc: hipMalloc of a %zu-byte slab failed: %s",
                                    sz, hipGetErrorString(e));
+                    (void)hipGetLastError();     // reported here: the next launch must not find it
                     return (int)e;
                 }
                 slabs_.push_back(Slab{p, sz});   // as allocator.cuh:164-166
@@ -99,6 +103,20 @@ BumpAllocator& global_allocator() {
 }
 
 }  // namespace
+
+int alloc_workspace(size_t full, size_t least, hipStream_t stream, void** ws, size_t* bytes) {
+    BumpAllocator& a = global_allocator();
+    if (least < full) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (stream && hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
+        *bytes = full;
+        const int rc = a.allocate(full, ws, capture == hipStreamCaptureStatusNone);
+        if (rc == NMI_OK) return rc;
+    }
+    *bytes = least;
+    return a.allocate(least, ws);
+}
+
 }  // namespace nmi
 
 extern "C" {

@@ -133,8 +133,11 @@ int mlp_forward_fp8(const void* input_bf16, const float* norm_w, const void* up_
             return NMI_ERR_WORKSPACE;
         }
     } else {
-        const int rc = nmi_alloc(need, &workspace);   // as the reference's allocate_tensor calls
+        // as the reference's allocate_tensor calls
+        const size_t least = split ? mlp_bytes(M, hidden, inter, Region::kLeast) : need;
+        const int rc = alloc_workspace(need, least, static_cast<hipStream_t>(stream), &workspace, &workspace_bytes);
         if (rc != NMI_OK) return rc;
+        if (workspace_bytes < need) region = Region::kLeast;
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
     const uint16_t* in = static_cast<const uint16_t*>(input_bf16);

@@ -155,8 +155,12 @@ int nmi_mamba_forward_fp8(const void* input_bf16, const float* norm_w, const voi
             return NMI_ERR_WORKSPACE;
         }
     } else {
-        const int rc = nmi_alloc(lay.total, &workspace);   // as the reference's allocate_tensor calls
+        // as the reference's allocate_tensor calls
+        const FwdLayout least = fwd_layout(M, hidden, d, false);
+        const int rc = alloc_workspace(lay.total, least.total, static_cast<hipStream_t>(stream), &workspace,
+                                       &workspace_bytes);
         if (rc != NMI_OK) return rc;
+        if (workspace_bytes < lay.total) lay = least;
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
     char* base = static_cast<char*>(workspace);
@@ -326,9 +330,10 @@ int nmi_mamba_decode_fp8(const void* input_bf16, const float* norm_w, const void
             return NMI_ERR_WORKSPACE;
         }
     } else {
-        const int rc = nmi_alloc(lay.total, &workspace);   // as the reference's allocate_tensor calls
+        // as the reference's allocate_tensor calls
+        const int rc = alloc_workspace(lay.total, lay.least, static_cast<hipStream_t>(stream), &workspace,
+                                       &workspace_bytes);
         if (rc != NMI_OK) return rc;
-        workspace_bytes = lay.total;
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
     char* base = static_cast<char*>(workspace);

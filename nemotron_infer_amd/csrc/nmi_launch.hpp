@@ -221,6 +221,10 @@ size_t linear_workspace_bytes(int M, int64_t total_n, int K);
 bool gemm_workspace_has_flags(int M);
 // The same without the DMA-fed kernel's K split, whose region a caller may leave out.
 size_t linear_workspace_bytes_least(int M, int64_t total_n, int K);
+// A block call's workspace where the caller gives none: `full` bytes from the bump allocator, or
+// `least` where they cannot be had -- out of memory, or `stream` is being captured and no slab has
+// the room (a hipMalloc would end the capture).  *bytes: which it was.
+int alloc_workspace(size_t full, size_t least, hipStream_t stream, void** ws, size_t* bytes);
 // The fp8 MLP block (block.cpp) behind nmi_mlp_forward_fp8 (split = true) and its allocation-free
 // form (split = false: the short-prompt GEMMs run unsplit, so the workspace has no partial
 // region); fn names the entry point in error messages.

@@ -18,7 +18,7 @@ struct Config {
     size_t shmem;
     void* stream;
 };
-constexpr int kSuccess = 0, kOutOfMemory = 2;
+constexpr int kSuccess = 0, kOutOfMemory = 2, kCaptureUnsupported = 900;
 
 std::map<const void*, std::string>& names() {
     static std::map<const void*, std::string> m;
@@ -29,7 +29,7 @@ Config g_config{};
 int g_last = kSuccess;
 uintptr_t g_next = uintptr_t{1} << 40;
 size_t g_limit = SIZE_MAX;
-int g_mallocs = 0;
+int g_mallocs = 0, g_capturing = 0;
 
 }  // namespace
 
@@ -44,6 +44,7 @@ const char* stub_take_log() {                  // launches since the last call: 
 }
 void stub_malloc_limit(size_t bytes) { g_limit = bytes; }   // hipMalloc of more fails
 int stub_mallocs() { return g_mallocs; }
+void stub_capturing(int on) { g_capturing = on; }           // every stream; hipMalloc then fails
 
 // --- the runtime's side
 void** __hipRegisterFatBinary(const void*) {
@@ -73,10 +74,9 @@ int hipLaunchKernel(const void* host, dim3 grid, dim3 block, void**, size_t, voi
     return kSuccess;
 }
 int hipMalloc(void** p, size_t bytes) {
-    if (bytes > g_limit) {
-        *p = nullptr;
-        return g_last = kOutOfMemory;
-    }
+    *p = nullptr;
+    if (g_capturing) return g_last = kCaptureUnsupported;
+    if (bytes > g_limit) return g_last = kOutOfMemory;
     ++g_mallocs;
     *p = reinterpret_cast<void*>(g_next);
     g_next += (bytes + 0xffff) & ~size_t{0xffff};
@@ -99,6 +99,10 @@ int hipGetDevice(int* dev) {
 }
 int hipDeviceGetAttribute(int* value, int, int) {
     *value = 256;                              // the only attribute asked for: compute units
+    return kSuccess;
+}
+int hipStreamIsCapturing(void*, int* status) {
+    *status = g_capturing;                     // 0: none, 1: active
     return kSuccess;
 }
 int hipDeviceSynchronize() { return kSuccess; }

@@ -67,3 +67,75 @@ for _ in range(4):
 """)
     assert rounds[0][1] == 3
     assert all(r == rounds[0] for r in rounds), rounds
+
+
+# The four blocks without a workspace, at sizes whose K-split region is more than half of the whole.
+BLOCKS = """
+W = 1 << 38                                      # a 256-byte aligned address, never touched
+ST = 1 << 12                                     # a stream
+def mlp(ws, n):
+    return L.nmi_mlp_forward_fp8(W, W, W, W, W, W, W, 1536, 3136, 12544, 1e-5, ws, n, ST)
+def attn(ws, n):
+    return L.nmi_attn_forward_fp8(W, W, W, W, W, W, W, W, W, W, W, 520, W, W, 520, 3136, 40, 8, 1e-5, ws, n, ST)
+def mamba_forward(ws, n):
+    return L.nmi_mamba_forward_fp8(*[W] * 13, 1, 520, W, W, 3136, 96, 80, 8, 128, 4, 1e-5, ws, n, ST)
+def mamba_decode(ws, n):
+    return L.nmi_mamba_decode_fp8(*[W] * 15, 24, 3136, 96, 80, 8, 128, 4, 1e-5, ws, n, ST)
+full = {"mlp": L.nmi_mlp_workspace_bytes(1536, 3136, 12544), "attn": L.nmi_attn_forward_workspace_bytes(520, 3136, 40, 8),
+        "mamba_forward": L.nmi_mamba_forward_workspace_bytes(1, 520, 3136, 96, 80, 8, 128),
+        "mamba_decode": L.nmi_mamba_decode_workspace_bytes(24, 3136, 96, 80, 8, 128)}[BLOCK]
+call = globals()[BLOCK]
+lo, hi = 1, full                                 # the least a caller's workspace may be
+while lo < hi:
+    mid = (lo + hi) // 2
+    lo, hi = (lo, mid) if call(W, mid) == 0 else (mid + 1, hi)
+least = lo
+hip.stub_take_log()
+def kernels():
+    return [l[0] for l in launches()]
+assert call(W, least) == 0
+unsplit = kernels()
+assert call(W, full) == 0
+split = kernels()
+"""
+
+
+@pytest.mark.parametrize("block", ["mlp", "attn", "mamba_forward", "mamba_decode"])
+def test_blocks_without_a_workspace_fall_back_to_the_unsplit_form(host, block):
+    """The K split's partials are no reason to fail: where the allocator cannot give the whole
+    workspace -- the device is out of memory, or the stream is being captured and no slab has the
+    room, when asking for one would end the capture -- the block runs with the smaller one."""
+    r = host(f"BLOCK = {block!r}" + BLOCKS + """
+slab = lambda n: max(64 * MB, (n + 127) // 128 * 128)
+result = {"full": full, "least": least, "split": split, "unsplit": unsplit}
+def without(setup):
+    L.nmi_alloc_reset()
+    setup()
+    rc, before = call(None, 0), hip.stub_mallocs()
+    k = kernels()
+    hip.stub_capturing(0)
+    hip.stub_malloc_limit(1 << 60)
+    return [rc, k]
+result["room"] = without(lambda: None)
+# a little less than the whole, of a slab that already holds something
+taken = max(0, 64 * MB - full + 4096) if full < 64 * MB else 0
+def fill():
+    if taken:
+        alloc(taken)
+def small_device():
+    fill()
+    hip.stub_malloc_limit(max(least, full - 4096) if not taken else 0)
+def capture():
+    if taken:
+        fill()
+    else:
+        alloc(least)
+        L.nmi_alloc_rewind()
+    hip.stub_capturing(1)
+result["small_device"] = without(small_device)
+result["capture"] = without(capture)
+""")
+    assert r["least"] < r["full"] and r["unsplit"] != r["split"]
+    assert r["room"] == [0, r["split"]]
+    assert r["small_device"] == [0, r["unsplit"]], r["small_device"]
+    assert r["capture"] == [0, r["unsplit"]], r["capture"]

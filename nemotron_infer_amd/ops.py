@@ -18,7 +18,10 @@ from . import _lib
 def _stream() -> int:
     """torch's current stream as a hipStream_t, without building a torch.cuda.Stream (a call's
     tensors are on a GPU, so torch's device state is set up)."""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    try:
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    except AttributeError:                     # private to torch: another version may lack them
+        return torch.cuda.current_stream().cuda_stream
 
 
 def _check_w(w: torch.Tensor, K: int | None = None) -> torch.Tensor:

@@ -133,3 +133,11 @@ def test_mlp_block_checks():
         ops.mlp_forward_fp8(x, nw, uw, us, dw, ds, out=torch.empty(4, hid, dtype=torch.bfloat16)[::2])
     with pytest.raises(ValueError, match="norm_w"):
         ops.mlp_forward_fp8(x, nw[:hid - 8], uw, us, dw, ds)
+
+
+def test_stream_without_torch_private_entries(monkeypatch):
+    class Stream:
+        cuda_stream = 4096
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", Stream)
+    assert ops._stream() == 4096

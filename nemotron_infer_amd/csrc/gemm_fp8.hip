@@ -1562,8 +1562,8 @@ size_t gemm_split_workspace_bytes(int M, int64_t N, int K) {
 
 namespace {
 // The DMA-fed kernel for one matrix at M < 512, by its modelled time against the short-prompt
-// kernel's: their crossing lies between M = 100 (N = 17504) and about 400 (N = 3136).  Measured
-// (us, short-prompt / DMA-fed): 100 x 17504 x 3136 35.6 / 34.6, 200 x 17504 x 3136 66.8 / 36.1, 300 x
+// kernel's: their crossing lies between M = 129 (N = 17504) and about 400 (N = 3136).  Measured
+// (us, short-prompt / DMA-fed): 100 x 17504 x 3136 33.9 / 33.8, 200 x 17504 x 3136 66.8 / 36.1, 300 x
 // 12544 x 3136 68.5 / 35.5, 400 x 3136 x 12544 57.0 / 46.7, 500 x 3136 x 7680 39.8 / 36.5; but 200 x 3136
 // x 12544 33.7 / 34.4, 256 x 7168 x 3136 24.8 / 24.9, 511 x 1024 x 12544 27.6 / 34.6; and fewer rows
 // than a column band stay with the short kernel (300 x 64 x 2048 23.6 / 26.0), as do its own knobs.
@@ -1573,10 +1573,20 @@ namespace {
 double dma_short_m_us(int M, int N, int K, size_t ws_bytes) {
     return dma_plan_ws(M, (N + 255) / 256, K, 1, ws_bytes).us;
 }
-bool dma_beats_short(int M, int N, int K, size_t ws_bytes) {
+// 30% where the plan is unsplit and its last column band (or, where y's rows are not 16-byte aligned, every
+// band) loads its scales or stores value by value, 3-9 us that the model does not have:
+// 300 x 300 x 2048 23.2 / 28.6, 511 x 900 x 3136 31.8 / 37.6, 200 x 9001 x 3136 33.9 / 38.9, 511 x
+// 1000 x 3136 32.7 / 34.6, 511 x 384 x 3136 33.4 / 34.3, but 511 x 9001 x 2048 52.1 / 31.1 and 200 x
+// 17504 x 3136 64.1 / 34.9.  A band short by whole 64-row parts costs no more than the lead from N =
+// 1024 (511 x 1600 x 3136 34.9 / 34.3).
+bool dma_beats_short(int M, int N, int K, const uint16_t* y, int64_t ldy, size_t ws_bytes) {
     const Tuning& t = tuning();
     if (M <= kShortOnlyM || N < 256 || t.gemm_short != 0 || t.gemm_splits > 1 || t.gemm_sk == 1 || t.gemm_bm == 256) return false;
-    return 1.1 * dma_short_m_us(M, N, K, ws_bytes) < gemm_short_us(M, N, K, ws_bytes);
+    const DmaPlan p = dma_plan_ws(M, (N + 255) / 256, K, 1, ws_bytes);
+    const bool aligned = ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+    const bool whole = N % 256 == 0 || (N % 64 == 0 && N >= 1024);
+    const double margin = p.splits > 1 || (aligned && whole) ? 1.1 : 1.3;
+    return margin * p.us < gemm_short_us(M, N, K, ws_bytes);
 }
 }  // namespace
 
@@ -1641,7 +1651,7 @@ hipError_t launch_gemm(const uint16_t* x, int64_t ldx, const uint8_t* W, int64_t
         // 4-wave forms, raised issue priority -- were slower.)
         const DeviceInfo& dev = device_info();
         const int64_t big = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
-        if (M < 512 && !(dma_supported(x, ldx, W, ldw, M, N, K) && dma_beats_short(M, N, K, ws ? ws_bytes : 0)))
+        if (M < 512 && !(dma_supported(x, ldx, W, ldw, M, N, K) && dma_beats_short(M, N, K, y, ldy, ws ? ws_bytes : 0)))
             tile = gemm_short_supported(x, ldx, W, ldw, M, N, K) ? 2 : 1;
         else if (dma_supported(x, ldx, W, ldw, M, N, K)) tile = 24;
         else tile = (4 * big >= 3 * (int64_t)dev.num_cu) ? 20 : 21;

@@ -139,3 +139,26 @@ result["capture"] = without(capture)
     assert r["room"] == [0, r["split"]]
     assert r["small_device"] == [0, r["unsplit"]], r["small_device"]
     assert r["capture"] == [0, r["unsplit"]], r["capture"]
+
+
+# Which kernel takes one matrix of N x K below 512 rows (y with row stride N + pad): at the crossings of
+# the two models, and where the DMA-fed kernel's tiles end in a ragged band or y's rows are not
+# 16-byte aligned.
+@pytest.mark.parametrize("M,N,K,pad,kernel", [
+    (64, 12544, 3136, 0, "short"), (300, 12544, 3136, 0, "dma"), (200, 3136, 12544, 0, "short"),
+    (511, 3136, 12544, 0, "dma"), (511, 3137, 12544, 0, "dma"), (128, 17504, 3136, 0, "short"),
+    (129, 17504, 3136, 0, "dma"), (511, 255, 3136, 0, "short"), (511, 256, 3136, 0, "dma"),
+    (300, 300, 2048, 0, "short"), (511, 257, 3136, 0, "short"), (511, 384, 3136, 0, "short"),
+    (511, 900, 3136, 0, "short"), (511, 1000, 3136, 0, "short"), (511, 1600, 3136, 0, "dma"),
+    (200, 9001, 3136, 0, "short"), (511, 9001, 2048, 0, "dma"), (511, 1536, 3136, 0, "dma"),
+    (511, 1536, 3136, 3, "short"), (511, 1536, 3136, 8, "dma"),
+])
+def test_kernel_below_512_rows(host, M, N, K, pad, kernel):
+    got = host(f"""
+M, N, K, ldy = {M}, {N}, {K}, {N + pad}
+W = 1 << 38
+n = L.nmi_linear_workspace_bytes(M, N, K)
+assert L.nmi_linear_fp8_w8a16_ws(W, K, W, K, W, W, ldy, M, N, K, W if n else None, n, 1 << 12) == 0
+result = [l[0] for l in launches()]
+""")
+    assert ("gemm_short_kernel" if kernel == "short" else "gemm_fp8_w8a16_dma_kernel") in got[0], got

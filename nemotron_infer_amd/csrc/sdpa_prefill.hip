@@ -39,6 +39,10 @@
 // At S = 4096 the cycles fell by 16% and the clock with them (2.1 -> 1.76 GHz): with the matrix
 // cores busy 62% of the time at 1.5 times the plain flops (P in two parts) the power budget is the
 // next bound.
+// The last tile has a body of its own without the scores that nothing follows (40 / 8 heads, S = 1 /
+// 33 / 64 / 192: 4.7 / 5.6 / 6.0 / 8.8 -> 4.2 / 4.7 / 5.4 / 8.3 us): with them the short prompts were
+// slower than in the form above (4.9 / 5.3 / 5.9 / 9.1).  65 to 128 tokens still are, by 0.1 to 0.4 us
+// (S = 128 7.7 / 8.1): two tiles are too few to pay for filling the pipeline.
 // The KV caches of the attention block are filled by the same launch (it was one of its own, 5-7 us).
 // Query tiles are scheduled longest first over all heads (the last tiles see the most keys).
 #include "nmi_device.hpp"
@@ -327,6 +331,29 @@ __global__ __launch_bounds__(256, 2) void sdpa_prefill_kernel(const PrefillArgs 
         settle();
         raise_max(tmax);
     };
+    // The same for the last tile, after which no scores are needed: the products with V of block g
+    // (weights wc) and, with weighs, the weights of block g + 1.
+    auto finish = [&](auto weighs, const f32x16& sc, const Weights& wc, Weights& wn, const uint8_t* vst,
+                      int j0) __attribute__((always_inline)) {
+        const float mc = m * a.scale2;
+        bf16x8 vf[3];
+        vf[0] = read_v(vst, j0, 0);
+        vf[1] = read_v(vst, j0, 1);
+#pragma unroll
+        for (int p = 0; p < 16; ++p) {
+            const int u = p >> 1, b = u & 3;
+            const bf16x8 w = frag((p & 1) ? wc.lo : wc.hi, u >> 2);
+            oacc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[u % 3], w, oacc[b], 0, 0, 0);
+            if (!(p & 1) && u + 2 < 8) vf[(u + 2) % 3] = read_v(vst, j0 + ((u + 2) >> 2), (u + 2) & 3);
+            if constexpr (decltype(weighs)::value) {
+#pragma unroll
+                for (int s = 24 * p / 16; s < 24 * (p + 1) / 16; ++s) weigh(sc, mc, s / 3, s % 3, wn);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (decltype(weighs)::value) l += psum;
+        settle();
+    };
     auto kslot = [&](int g) { return lds + (g & 3) * kKBlk; };
     auto vstage = [&](int t) { return lds + 4 * kKBlk + (t & 1) * kVBytes; };
     // Tile t = blocks 2 t, 2 t + 1.  On entry wa holds block 2 t's weights, sb block 2 t + 1's scores;
@@ -422,18 +449,25 @@ __global__ __launch_bounds__(256, 2) void sdpa_prefill_kernel(const PrefillArgs 
         step(std::integral_constant<int, 0>{}, t);
         step(std::integral_constant<int, 1>{}, t + 1);
     }
-    // the last tiles (up to four), one body for all: a short prompt runs no other.  Each wave takes
-    // the blocks with a key <= some query of its own.  The scores past those come from slots that
-    // may hold other blocks; they are masked (their keys lie past every query).
-    for (; t < ntiles; ++t) {
-        const bool more = t + 1 < ntiles;
-        if (more) issue(t);
+    // the last tiles (up to four) but the very last, one body for all.  Each wave takes the blocks
+    // with a key <= some query of its own; the scores past those are masked.
+    for (; t + 1 < ntiles; ++t) {
+        issue(t);
         if (qw < S && t * kBK <= qw + 31) {
             constexpr std::true_type masked{};
             block(masked, sb, sa, wa, wb, kslot(2 * t + 2), vstage(t), 0, t * kBK + 64);
             if (t * kBK + 32 <= qw + 31) block(masked, sa, sb, wb, wa, kslot(2 * t + 3), vstage(t), 2, t * kBK + 96);
         }
-        if (more) publish();
+        publish();
+    }
+    if (qw < S && t * kBK <= qw + 31) {
+        int j0 = 0;
+        if (t * kBK + 32 <= qw + 31) {
+            finish(std::true_type{}, sb, wa, wb, vstage(t), 0);
+            wa = wb;                    // (one body for the second half)
+            j0 = 2;
+        }
+        finish(std::false_type{}, sb, wa, wb, vstage(t) + 4096 * j0, 0);
     }
     l += __shfl_xor(l, 32);
 

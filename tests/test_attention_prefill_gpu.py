@@ -109,6 +109,54 @@ def test_sdpa_prefill_gqa_and_packed_rows(H, n_kv):
     assert_parity(bits(o), ref, f"H={H} n_kv={n_kv}")
 
 
+@pytest.mark.parametrize("S", [33, 64, 65, 96, 128, 161, 321])
+@pytest.mark.parametrize("kind", ["rising", "spikes"])
+def test_sdpa_prefill_late_maxima(S, kind):
+    """Rows whose running maximum is raised in every block of 32 keys (a step of 8 in raw score per
+    key: e^-0.7 in weight) or at single keys beside the edges of blocks and tiles, up to the last
+    one: the rescales of the sums, also the ones left pending when the last tile begins."""
+    H, n_kv = 3, 1
+    announce("sdpa_prefill_late_maxima", S, kind)
+    g = torch.Generator().manual_seed(S)
+    q = torch.randn((S, H, D), generator=g)
+    k = torch.randn((S, D), generator=g)
+    v = torch.randn((S, D), generator=g)
+    q[:, :, 0] = 16.0
+    if kind == "rising":
+        k[:, 0] = 0.5 * torch.arange(S)
+    else:
+        at = [j for j in (0, 1, 30, 31, 32, 63, 64, 95, 96, 127, 128, 160, 256, 287, 320) if j < S]
+        k[:, 0] = 0.0
+        k[at, 0] = 8.0 * torch.arange(1, len(at) + 1)
+    qb, kb, vb = (t.reshape(S, -1).to(torch.bfloat16).view(torch.int16).numpy().view(np.uint16) for t in (q, k, v))
+    o = ops.sdpa_prefill_bf16(x_to_dev(qb), x_to_dev(kb), x_to_dev(vb), H, n_kv)
+    torch.cuda.synchronize()
+    assert_parity(bits(o), attention.sdpa_prefill(qb, kb, vb, n_kv), f"S={S} {kind}")
+
+
+@pytest.mark.parametrize("H,n_kv", [(4, 4), (4, 2), (9, 3), (6, 1)])
+@pytest.mark.parametrize("S", [31, 129, 520])
+def test_attn_forward_fills_the_caches_for_every_head_ratio(H, n_kv, S):
+    """The attention launch fills the caches, each (KV head, query tile) by one query head of its
+    group: every position once, for groups of 1, 2, 3 and 6 and one to five query tiles."""
+    hidden = 256
+    announce("attn_forward_caches", H, n_kv, S)
+    mats = [synth.make_weight(n, kk, 8100 + i, DEV) for i, (n, kk) in
+            enumerate([(H * D, hidden), (n_kv * D, hidden), (n_kv * D, hidden), (hidden, H * D)])]
+    nw = torch.ones(hidden, device=DEV)
+    x = synth.make_act(S, hidden, 8200 + S, DEV)
+    kc = torch.full((n_kv, S + 2, D), 7.0, dtype=torch.bfloat16, device=DEV)
+    vc = torch.full_like(kc, 7.0)
+    got = ops.attn_forward_fp8(x, nw, *[t for m in mats for t in m], k_cache=kc, v_cache=vc, eps=EPS)
+    q, k, v = ops.linear_fp8_w8a16_grouped(ops.rmsnorm_bf16(x, nw, EPS), mats[:3])
+    ref = x + ops.linear_fp8_w8a16(ops.sdpa_prefill_bf16(q, k, v, H, n_kv), *mats[3])
+    torch.cuda.synchronize()
+    for cache, t in ((kc, k), (vc, v)):
+        assert torch.equal(cache[:, :S].view(torch.int16), t.view(S, n_kv, D).transpose(0, 1).view(torch.int16))
+        assert torch.all(cache[:, S:] == 7.0)
+    assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+
+
 # --------------------------------------------------------------------------------------
 # the block at the model's dimensions
 # --------------------------------------------------------------------------------------

@@ -420,8 +420,8 @@ double gemm_short_us(int M, int N, int K, size_t ws_bytes) {
 }
 
 // Enough for any N' <= N (grouped launches share one workspace): splits x N' is at most
-// min(splits by k and bytes) x N, and the one-round limit keeps it below the rows one round of
-// workgroups covers.
+// min(splits by k and bytes) x N, and the one-round limit keeps it below the rows that one round of
+// the form's workgroups covers.
 size_t gemm_short_workspace_bytes(int M, int N, int K) {
     if (M < 1 || N < 1 || K < kBK) return 0;
     const int KT = K / kBK;
@@ -433,10 +433,15 @@ size_t gemm_short_workspace_bytes(int M, int N, int K) {
     } else {
         const int64_t cap = std::max(1, std::min(KT / 4, (int)((int64_t)K / (4 * (int64_t)M))));
         if (cap <= 1) return 0;
-        // over the forms M can take: at most the rows one round of workgroups covers
+        // splits <= round x CUs / (weight tiles x row tiles), over the forms that a matrix of up to N
+        // rows may take (short_form's answers for few rows and for N)
         int64_t round_rows = 0;
-        for (const ShortCfg& c : kForms) round_rows = std::max<int64_t>(round_rows, (int64_t)c.per_cu * c.bn());
-        rows = std::min<int64_t>(cap * N, round_rows * device_info().num_cu);
+        for (const int f : {short_form(M, 1), short_form(M, N)}) {
+            const ShortCfg& c = kForms[f];
+            const int tiles_m = (M + c.bm() - 1) / c.bm();
+            round_rows = std::max<int64_t>(round_rows, (int64_t)(c.round * device_info().num_cu / tiles_m) * c.bn());
+        }
+        rows = std::min<int64_t>(cap * N, round_rows);
     }
     return kFlagRegion + (size_t)rows * M * sizeof(float);
 }

@@ -162,3 +162,32 @@ assert L.nmi_linear_fp8_w8a16_ws(W, K, W, K, W, W, ldy, M, N, K, W if n else Non
 result = [l[0] for l in launches()]
 """)
     assert ("gemm_short_kernel" if kernel == "short" else "gemm_fp8_w8a16_dma_kernel") in got[0], got
+
+
+def test_linear_workspace_is_enough(host):
+    """The bytes the library asks for give the launches that unlimited ones do: one matrix, and up to
+    64 rows matrices sharing x, at and between the row tiles of the kernels."""
+    bad, asked = host("""
+import random
+rng = random.Random(5)
+W, ST, HUGE = 1 << 38, 1 << 12, 1 << 33
+bad, asked = [], {}
+def linear(Ns, M, K, n):
+    arr = (_lib.LinearGroup * len(Ns))(*[_lib.LinearGroup(W, K, W, W, N, N) for N in Ns])
+    assert L.nmi_linear_fp8_w8a16_grouped(W, K, M, K, arr, len(Ns), W, n, ST) == 0
+    return launches()
+for M in (17, 31, 32, 33, 64, 65, 100, 128, 129, 256, 300, 511):
+    for i in range(60):
+        K = 64 * rng.choice((1, 5, 16, 32, 49, 80, 120, 196))
+        Ns = [rng.choice((1, 130, 300, 1024, 2048, 3136, 5120, 12544, 17504, rng.randint(1, 50000)))]
+        if M <= 64 and i % 3 == 0:
+            Ns += [rng.randint(1, 9000) for _ in range(rng.randint(1, 3))]
+        n = L.nmi_linear_workspace_bytes(M, sum(Ns), K)
+        if linear(Ns, M, K, n) != linear(Ns, M, K, HUGE):
+            bad.append((M, Ns, K, n))
+        asked[M] = max(asked.get(M, 0), n)
+result = [bad, asked]
+""")
+    assert not bad, bad[:5]
+    # the short-prompt kernel's one round of 128-row tiles, or one 256 x 256 tile per CU
+    assert all(n <= 65536 + (64 << 20) for m, n in asked.items() if int(m) > 64), asked

@@ -120,7 +120,8 @@ def test_automatic_split_in_the_mlp_block_and_a_graph():
 
 
 # The choice between the short-prompt and the DMA-fed kernel at M < 512 (one matrix, and matrices
-# sharing x), on both sides of it: with a workspace, without one, and with one too small.
+# sharing x), on both sides of it: with a workspace, without one, and with one too small.  (Which
+# kernel takes which of these: test_host_runtime_cpu.py.)
 @pytest.mark.parametrize("M", [17, 64, 65, 130, 300, 511])
 @pytest.mark.parametrize("Ns,K", [((17500,), 320), ((1000, 260, 130), 1024), ((300,), 5120)])
 def test_below_512_rows(M, Ns, K):
@@ -146,8 +147,8 @@ def test_below_512_rows(M, Ns, K):
             assert_parity(bits(y), ref, f"M={M} group {i} ws={nbytes}", per_row_scales=True)
 
 
-# Matrices sharing x below 512 rows as one launch: every row-tile form of the short-prompt kernel, row
-# counts that are no multiple of 4 (the partials after them are unaligned), one k tile (no split), many.
+# Matrices sharing x below 512 rows as one launch: every row-tile form of the short-prompt kernel but
+# the widest (the next test), row counts that are no multiple of 4 (the partials after them are unaligned), one k tile (no split), many.
 @pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 128, 129])
 @pytest.mark.parametrize("K", [64, 1088])
 def test_grouped_short(M, K):
@@ -173,6 +174,26 @@ def test_grouped_short(M, K):
                       per_row_scales=True)
     assert torch.all(ybig[:, total:] == 5.0)
     assert torch.all(ws[:min(need, 65536)] == 255), "flag region written"
+
+
+# The 256 x 32 tiles, which only few rows of x against some 49000 weight rows and more take: ragged
+# matrices, a matrix within one tile, two and five k tiles (too few to split).
+@pytest.mark.parametrize("M", [17, 32])
+@pytest.mark.parametrize("K", [128, 320])
+def test_grouped_short_wide_tiles(M, K):
+    Ns = (30001, 12544, 77, 6800)
+    announce("gemm_grouped_short_wide", M, Ns, K)
+    cases = [_case(M, N, K, 23 * i + M + K) for i, N in enumerate(Ns)]
+    xd = x_to_dev(cases[0][0])
+    wd = [(w_to_dev(w), s_to_dev(s)) for _, w, s in cases]
+    ys = [torch.full((M, N + 3), 5.0, dtype=torch.bfloat16, device=DEV) for N in Ns]
+    arr = (_lib.LinearGroup * len(Ns))(*[_lib.LinearGroup(w.data_ptr(), K, s.data_ptr(), y.data_ptr(), y.stride(0), N)
+                                         for (w, s), y, N in zip(wd, ys, Ns)])
+    _lib.check(_lib.lib().nmi_linear_fp8_w8a16_grouped(xd.data_ptr(), K, M, K, arr, len(Ns), None, 0, None), "grouped")
+    torch.cuda.synchronize()
+    for i, ((_, w, s), y) in enumerate(zip(cases, ys)):
+        assert_parity(bits(y[:, :-3]), oracle_bits(cases[0][0], w, s), f"M={M} K={K} group {i}", per_row_scales=True)
+        assert torch.all(y[:, -3:] == 5.0)
 
 
 # Groups of ragged column bands with K split in every tile height.

@@ -164,6 +164,27 @@ result = [l[0] for l in launches()]
     assert ("gemm_short_kernel" if kernel == "short" else "gemm_fp8_w8a16_dma_kernel") in got[0], got
 
 
+def test_both_kernels_take_some_of_the_gpu_parity_cases(host):
+    """tests/test_gemm_split_gpu.py runs these sizes against the oracle as cases on both sides of the
+    choice, and the grouped ones as every form of the short-prompt kernel's tiles."""
+    one, many, forms = host("""
+W, ST = 1 << 38, 1 << 12
+def grouped(Ns, M, K):
+    arr = (_lib.LinearGroup * len(Ns))(*[_lib.LinearGroup(W, K, W, W, N, N) for N in Ns])
+    n = L.nmi_linear_workspace_bytes(M, sum(Ns), K)
+    assert L.nmi_linear_fp8_w8a16_grouped(W, K, M, K, arr, len(Ns), W if n else None, n, ST) == 0
+    return launches()[0][0]
+Ms = (17, 64, 65, 130, 300, 511)
+result = [[grouped(Ns, M, K) for Ns, K in (((17500,), 320), ((300,), 5120)) for M in Ms],
+          [grouped((1000, 260, 130), M, 1024) for M in Ms],
+          [grouped((130, 77, 1, 260), M, K) for M in (17, 32, 33, 64, 65, 128, 129) for K in (64, 1088)]
+          + [grouped((30001, 12544, 77, 6800), M, K) for M in (17, 32) for K in (128, 320)]]
+""")
+    for names in (one, many):
+        assert any("gemm_short_kernel" in k for k in names) and any("gemm_fp8_w8a16_dma_kernel" in k for k in names), names
+    assert len({k for k in forms if "gemm_short_kernel" in k and "Lb1E" in k}) == 4, set(forms)
+
+
 def test_linear_workspace_is_enough(host):
     """The bytes the library asks for give the launches that unlimited ones do: one matrix, and up to
     64 rows matrices sharing x, at and between the row tiles of the kernels."""

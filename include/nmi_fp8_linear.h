@@ -93,7 +93,11 @@ int nmi_linear_fp8_w8a16(const void* x_bf16, int64_t ldx, const void* w_e4m3, in
  * workspace for it only then.
  * workspace: 256-byte aligned, at least nmi_linear_workspace_bytes(M, N, K) bytes, zero-filled
  * before its first use; every launch leaves it ready for the next one.  NULL / too small ->
- * the kernels run without the split (same results up to float32 summation order).  Two
+ * the kernels run without the split (same results up to float32 summation order).  So for M >= 17 a
+ * row's last bits may depend on how many rows are in the call (below M = 512 for any K, from M =
+ * 512 where one matrix has K >= 4096) and on whether the workspace has the room: a prompt run
+ * whole and the same prompt run in chunks agree up to that order.  Equal calls with equal
+ * workspace sizes give the same bytes.  Two
  * launches that may run concurrently must not share a workspace.  The reference's blocks
  * likewise hand a workspace to their prefill GEMMs (model/mlp_block.cuh:133,156,160-161).
  * Stream-K ordering: a contributor stores its partial tile, then releases its flag at device
@@ -192,17 +196,17 @@ int nmi_gemv_chain_launch(const nmi_gemv_chain* chain, void* workspace, size_t w
 int nmi_gemv_chain_destroy(nmi_gemv_chain* chain);
 
 /* Workspace bytes the kernels can use for M rows, total_n output rows (the sum over groups)
- * and K on the current device; 0 when the selected kernel needs none (the GEMV, the skinny
- * kernels by default, which split K inside the workgroup only).  With the 4x4x4 kernel's K
- * split (s4.kg > 1): 64 KiB of arrival counters and the fp32 partials, s4.kg x M x total_n x 4
- * bytes (fewer K groups when K has fewer windows).  For M >= 17 (the GEMMs) a 64 KiB region they
- * leave alone, then the fp32 partials of the K split (at most about one 256 x 256 tile per CU,
- * 64 MiB; 0 when no kernel the call may take splits K).  Every
+ * and K on the current device; 0 when the selected kernel needs none (the GEMV and the skinny
+ * kernels, M <= 16, split K inside the workgroup only).  For M >= 17 (the GEMMs) a 64 KiB region
+ * they leave alone, then the fp32 partials of the K split (0 when no kernel the call may take splits
+ * K): at most one 256 x 256 tile per CU (64 MiB on 256 CUs), four where gemm.splits forces a split.
+ * The size is not largest at the most rows.  Every
  * kernel leaves the first 64 KiB as it found it (zero at rest), so one zero-filled workspace
  * serves every M in turn. */
 size_t nmi_linear_workspace_bytes(int M, int64_t total_n, int K);
-/* 0 where a workspace for M rows may hold anything (the K split from M = 512 writes its partials
- * before it reads them), 1 where it must start zero-filled. */
+/* 0 where a workspace for M rows may hold anything (the K split writes its partials before it reads
+ * them), 1 where it must start zero-filled: the stream-K form, and, for callers that keep one
+ * workspace for every M, every M < 512 (whose kernels leave the region that must be zero alone). */
 int nmi_linear_workspace_needs_zero(int M);
 
 /*
@@ -211,7 +215,7 @@ int nmi_linear_workspace_needs_zero(int M);
  * ws_size, stream) (nemotron_infer/csrc/include/ops/gemm.cuh:325-403) including its
  * per-row scale epilogue (gemm.cuh:227-238, 398-402), which here is fused and rounds once.
  * x is bf16 (no activation scale); `workspace`/`workspace_bytes` as for
- * nmi_linear_fp8_w8a16_ws (NULL/0: every tile in one workgroup, no stream-K).
+ * nmi_linear_fp8_w8a16_ws (NULL/0: every tile in one workgroup, K whole).
  */
 int nmi_gemm_fp8_w8a16(const void* x_bf16, int64_t ldx, const void* w_e4m3, int64_t ldw,
                        const float* w_scale, void* y_bf16, int64_t ldy, int M, int N, int K,
@@ -255,9 +259,8 @@ int nmi_rmsnorm_bf16(const void* x_bf16, const float* w, void* y_bf16, int M, in
  * RMSNorm applied while the up projection stages its activations, relu^2 and the residual add
  * in the projections' stores), larger M three (a separate RMSNorm).
  * workspace: nmi_mlp_workspace_bytes(M, hidden, inter) bytes, 16-byte aligned, no
- * initialisation needed (for 17 <= M < 512 it includes the short-prompt GEMMs' K-split partials;
- * from M = 512 the GEMMs' stream-K region, whose flags each call zeroes with one small kernel);
- * calls that may overlap in time need distinct workspaces.  NULL
+ * initialisation needed (from M = 17 it includes the GEMMs' K-split partials; under the knobs of the
+ * stream-K form also its flags, which each call zeroes with one small kernel); calls that may overlap in time need distinct workspaces.  NULL
  * takes it from the bump allocator (nmi_alloc, so a slab may be hipMalloc'd), valid until
  * nmi_alloc_rewind(), as the reference's blocks do (binding.cu:7-9).  The size is not largest at the
  * most rows (the K split's partials: hidden 3136, inter 12544 64 MB at M = 2048, 110 MB at 1536); a
@@ -450,11 +453,8 @@ int nmi_mamba_forward_fp8(const void* input_bf16, const float* norm_w, const voi
  * (1: none), "gemm.bm": tile rows from M = 512 (128, 192, 256), "gemm.short": f + 1 forces its tile form f (0..7),
  * "gemm.sk_cap": workgroups per tile of the stream-K form at most (0: 2, -1: one workgroup per
  * CU), "skinny.path" (2: the skinny kernels take M = 2 too, 3: the GEMV kernel takes M <= 4),
- * "m1.path" (3: M = 1 on the 4x4x4 skinny kernel), "s4.ks", "s4.t", "s4.u",
- * "s4.dma": 2 selects the windowed form of the 4x4x4 skinny kernel instead of the pipelined one,
- * "s4.kg": K groups split between workgroups by the pipelined form (> 1; needs the workspace
- * nmi_linear_workspace_bytes then reports), "s16": the 16x16x32 skinny kernel (0: automatic, from
- * M = 3, 1: for 2 <= M <= 16, 2: never), "s16.r": its row tiles of 16 (1) or 32 (2), "s16.w": its
+ * "m1.path" (3: M = 1 on the 4x4x4 skinny kernel), "s4.ks", "s4.t", "s4.u", "s16": the 16x16x32
+ * skinny kernel (0: automatic, from M = 3, 1: for 2 <= M <= 16, 2: never), "s16.r": its row tiles of 16 (1) or 32 (2), "s16.w": its
  * waves per workgroup (2, 4), "s16.t": 1 its row-run form instead of the DMA form, "chain.wgs":
  * workgroups per CU of a GEMV chain created afterwards); 0 restores the automatic choice.
  * Process-wide, not thread-safe against concurrent launches; results do not depend on them

@@ -77,8 +77,9 @@ struct FwdLayout {
 };
 
 // The GEMMs' region (the K splits' partials, or the stream-K flags and partials where that form
-// is forced by tuning knob): the largest of the q, k, v (launched one by one below M = 512) and o
-// needs.  split = false: without the DMA-fed kernel's K split.
+// is forced by tuning knob): the largest of what q | k | v as one launch, each of the three alone (where
+// the models prefer that below M = 512) and o need.  split = false: without the DMA-fed kernel's K
+// split.
 size_t gemm_region(int M, int hidden, int QD, int KD, bool split) {
     if (choose_path(M) != Path::Gemm) return 0;
     const auto need = split ? linear_workspace_bytes : linear_workspace_bytes_least;

@@ -45,8 +45,8 @@ bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) %
 
 size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// Workspace layout: the GEMMs' region (M >= 17: flags, then the K split's partials), act [M, inter] bf16, then normed [M, hidden] bf16 when the RMSNorm is not fused into the up
-// projection.
+// Workspace layout: the GEMMs' region (M >= 17: flags, then the K split's partials), act [M, inter]
+// bf16, then normed [M, hidden] bf16 when the RMSNorm is not fused into the up projection.
 bool norm_fused(int M, int hidden) { return gemv_fuses_norm(M, hidden); }
 
 // The GEMMs' region: kFull, kLeast without the DMA-fed kernel's K split (a caller's workspace

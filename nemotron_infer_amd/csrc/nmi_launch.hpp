@@ -197,15 +197,16 @@ hipError_t launch_gemv_stream_chain(const StreamPhase* tab, const int* wave_step
 
 // Prefill GEMM.  Given a workspace of at least gemm_workspace_bytes(M) bytes whose first 64 KiB
 // (the flag region) are zero -- every launch leaves them zero again -- the DMA-fed kernel splits
-// the k tiles of all tiles evenly between the CUs (stream-K) when the tiles cover at most half
-// of them (tuning knob gemm.sk = 1: always, also for the 8-wave kernels; 2: never); otherwise
-// one tile per workgroup.  launch_sk_flags_clear zeroes the flag region (one small kernel, safe
+// the k tiles of all tiles evenly between the CUs (stream-K) under tuning knob gemm.sk = 1 (also the
+// 8-wave kernels), or under gemm.bm = 256 where the tiles cover at most half of the CUs; otherwise it
+// is 0 and tiles go one per workgroup, K whole or split as dma_plan says.  launch_sk_flags_clear zeroes the flag region (one small kernel, safe
 // under graph capture).
 size_t gemm_workspace_bytes(int M);
 // Workspace of the DMA-fed kernel's K split (N rows in all; 0: not split): float32 partial tiles
-// after the flag region, no initialisation needed.
+// after the flag region, no initialisation needed.  At most one 256 x 256 tile per CU (four under a
+// forced gemm.splits).
 size_t gemm_split_workspace_bytes(int M, int64_t N, int K);
-// Short prompts (17 <= M < 512; gemm_short.hip): the pipelined 128-row-tile kernel, with K split
+// Short prompts (17 <= M < 512; gemm_short.hip): the pipelined kernel of small tiles, with K split
 // between workgroups when a workspace of gemm_short_workspace_bytes(M, N, K) bytes is given
 // (float32 partials, no initialisation needed; 0: the schedule does not split).
 bool gemm_short_supported(const uint16_t* x, int64_t ldx, const uint8_t* W, int64_t ldw, int M, int N, int K);
@@ -309,8 +310,9 @@ hipError_t launch_sdpa_prefill(const uint16_t* q, int64_t ldq, const uint16_t* k
                                uint16_t* v_cache, int cap, hipStream_t stream);
 
 hipError_t launch_sk_flags_clear(void* ws, hipStream_t stream);
-// Several matrices sharing x: one launch of the DMA-fed kernel where it takes them all (M >= 512),
-// else launch_gemm per matrix.
+// Several matrices sharing x: one launch of the DMA-fed kernel (from M = 512 where it takes them all,
+// below by modelled time) or of the short-prompt kernel (M < 512: always up to kShortOnlyM rows where
+// the workspace holds its K split, above by modelled time), else launch_gemm per matrix.
 hipError_t launch_gemm_grouped(const uint16_t* x, int64_t ldx, int M, int K, const GemvGroup* g, int ng,
                                hipStream_t stream, void* ws, size_t ws_bytes);
 hipError_t launch_gemm(const uint16_t* x, int64_t ldx, const uint8_t* W, int64_t ldw,

@@ -1371,7 +1371,7 @@ struct DmaPlan {
 // K >= 4096 (below, from M = 512, no split of any projection was faster than its best unsplit
 // tiles, and a row's sums stay the same in a larger batch or a group), matrices sharing x where
 // M < 512 (dma_plan_ws); and only for a modelled gain of 8%: with most CUs busy either way the power budget decides (2048 x 3136 x
-// 12544, 256-row tiles split in two against whole 128-row tiles: 143 against 148 us on one box, the
+// 12544, 256-row tiles split in two against whole 128-row tiles: 143 against 148 us in one run, the
 // MLP block 329 against 318 us on another).
 // Examples (us): 777 x 12544 x 3136 256 / 192 / 128-row tiles 67.5 / 59.6 / 75.9; 2048 x 17504 x
 // 3136 209 / 180 / 209; 512 x 3136 x 12544 in 128-row tiles, splits of 1 / 2 / 3 / 4: 113 / 70 /

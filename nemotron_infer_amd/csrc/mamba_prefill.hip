@@ -296,7 +296,7 @@ __global__ __launch_bounds__(256, 4) void mamba_scan_kernel(const MambaPrefillAr
 // the same staged chunk and the same S0, so the two run beside each other instead of one after the
 // other in four waves: a chunk is a chain of dependent LDS reads, MFMAs and vector work (at S =
 // 2048 the four-wave form had its vector units busy 43% of the cycles, its matrix cores 14%, and
-// waited 35%).  Same box, 96 heads of 80: one sequence of 2048 tokens 87.9 -> 82.7 us, two of 500 equal.  (Two,
+// waited 35%).  Measured side by side, 96 heads of 80: one sequence of 2048 tokens 87.9 -> 82.7 us, two of 500 equal.  (Two,
 // three or five blocks of 16 rows of P per workgroup, sharing G: slower, the chain grows by each.)
 // Each SIMD issues a wave64 VALU instruction over 4 cycles, so the per-element work is kept on
 // MFMA: what remains on VALU per chunk is the decay weights, the G mask and the two-part splits.

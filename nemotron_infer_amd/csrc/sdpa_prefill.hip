@@ -33,7 +33,7 @@
 // weights.  A 32-cycle MFMA hides up to six vector instructions or two exponentials of its own
 // wave (measured), so the 24 MFMAs of a block are laid out in 24 slots with the block's 106 vector
 // instructions and 24 LDS reads spread over them; the compiler's own order ran the vector work
-// between the MFMAs' blocks.  Same-box times against that form (scores one block ahead, weights in
+// between the MFMAs' blocks.  Times beside that form (scores one block ahead, weights in
 // the block that uses them), 40 / 8 heads, S = 512 / 1000 / 2048 / 4096 / 8192: 17.5 / 31.4 / 69.8
 // / 235.9 / 877.5 -> 16.2 / 27.9 / 65.5 / 223.6 / 826.9 us; 16 / 4 heads, S = 2048: 52.4 -> 43.7.
 // At S = 4096 the cycles fell by 16% and the clock with them (2.1 -> 1.76 GHz): with the matrix

@@ -77,21 +77,40 @@ def _check_device(*ts: torch.Tensor) -> None:
             raise ValueError(f"all tensors must be on {dev}, got {t.device}")
 
 
-def _workspace(device: torch.device, need: int) -> torch.Tensor | None:
-    """The transient device memory of one call (None where it needs none), from torch's allocator
-    like any temporary of the current stream: calls on other streams and threads, and graphs
-    captured with torch.cuda.graph (whose pool it then comes from), never share it, and nothing
-    outlives the call.  The kernels write what they read of it."""
-    return torch.empty(need, dtype=torch.uint8, device=device) if need else None
+# Transient device memory of up to _KEEP_BYTES is kept between calls, one tensor for each (device,
+# stream): torch.empty and the release cost a call 2 us of host time, 5-10% of an eager decode call
+# that the host bounds (attention decode over 30 / 65 positions 19.1 / 22.6 us with the memory at hand,
+# 21.2 / 24.0 without; kept 0.3-0.5 us more than at hand).  A call takes the tensor out for its
+# duration, so that a second thread on the stream gets memory of its own.
+_KEEP_BYTES = 32 << 20
+_kept: dict[tuple[int, int], torch.Tensor] = {}
 
 
-def _linear_ws(L, device: torch.device, M: int, N: int, K: int) -> torch.Tensor | None:
+def _workspace(device: torch.device, need: int, stream: int):
+    """The transient device memory of one call on `stream`: (tensor, key), the tensor None where it
+    needs none; after the launch the caller puts it back, _kept[key] = tensor, where key is not None.
+    Large memory, and all of it under stream capture (from the graph's pool, which a replay may
+    write to at any time), comes from torch's allocator for this call alone.  The kernels write what
+    they read of it."""
+    if not need:
+        return None, None
+    key = None
+    if need <= _KEEP_BYTES and not torch.cuda.is_current_stream_capturing():
+        key = (device.index, stream)
+        ws = _kept.pop(key, None)
+        if ws is not None and ws.numel() >= need:
+            return ws, key
+        need = max(need, 1 << 20)
+    return torch.empty(need, dtype=torch.uint8, device=device), key
+
+
+def _linear_ws(L, device: torch.device, M: int, need: int, stream: int):
     """_workspace() of a linear.  Only the stream-K form (a tuning knob, from M = 512) reads what it
     has not written: its flags, in the first 64 KiB."""
-    ws = _workspace(device, L.nmi_linear_workspace_bytes(M, N, K))
-    if ws is not None and M >= 512 and L.nmi_linear_workspace_needs_zero(M):
+    ws, key = _workspace(device, need, stream)
+    if need and M >= 512 and L.nmi_linear_workspace_needs_zero(M):
         ws[:_lib.NMI_WS_ERROR_OFFSET + 4].zero_()
-    return ws
+    return ws, key
 
 
 def _as_2d(x: torch.Tensor):
@@ -117,11 +136,14 @@ def linear_fp8_w8a16(x: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
     _check_out(out, M, N)
     _check_device(x2, w, w_scale, out)
     L = _lib.lib()
-    ws = _linear_ws(L, x.device, M, N, K) if use_workspace else None
+    st = _stream()
+    need = L.nmi_linear_workspace_bytes(M, N, K) if use_workspace else 0
+    ws, key = _linear_ws(L, x.device, M, need, st)
     rc = L.nmi_linear_fp8_w8a16_ws(
         x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0), w_scale.data_ptr(),
-        out.data_ptr(), N, M, N, K,
-        None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _stream())
+        out.data_ptr(), N, M, N, K, None if ws is None else ws.data_ptr(), need, st)
+    if key is not None:
+        _kept[key] = ws
     _lib.check(rc, "nmi_linear_fp8_w8a16_ws")
     return out
 
@@ -148,10 +170,13 @@ def linear_fp8_w8a16_grouped(x: torch.Tensor, weights, outs=None, use_workspace:
         arr[i] = _lib.LinearGroup(w.data_ptr(), w.stride(0), s.data_ptr(), y.data_ptr(), N, N)
     L = _lib.lib()
     total = sum(w.shape[0] for w, _ in weights)
-    ws = _linear_ws(L, x.device, M, total, K) if use_workspace else None
+    st = _stream()
+    need = L.nmi_linear_workspace_bytes(M, total, K) if use_workspace else 0
+    ws, key = _linear_ws(L, x.device, M, need, st)
     rc = L.nmi_linear_fp8_w8a16_grouped(x2.data_ptr(), x2.stride(0), M, K, arr, n,
-                                        None if ws is None else ws.data_ptr(),
-                                        0 if ws is None else ws.numel(), _stream())
+                                        None if ws is None else ws.data_ptr(), need, st)
+    if key is not None:
+        _kept[key] = ws
     _lib.check(rc, "nmi_linear_fp8_w8a16_grouped")
     return outs
 
@@ -221,11 +246,14 @@ def gemm_fp8_w8a16(x: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
     _check_out(out, M, N)
     _check_device(x2, w, w_scale, out)
     L = _lib.lib()
-    ws = _linear_ws(L, x.device, M, N, K) if use_workspace else None
+    st = _stream()
+    need = L.nmi_linear_workspace_bytes(M, N, K) if use_workspace else 0
+    ws, key = _linear_ws(L, x.device, M, need, st)
     rc = L.nmi_gemm_fp8_w8a16(x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0),
                               w_scale.data_ptr(), out.data_ptr(), N, M, N, K,
-                              None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
-                              _stream())
+                              None if ws is None else ws.data_ptr(), need, st)
+    if key is not None:
+        _kept[key] = ws
     _lib.check(rc, "nmi_gemm_fp8_w8a16")
     return out
 
@@ -253,8 +281,8 @@ def mlp_forward_fp8(x: torch.Tensor, norm_w: torch.Tensor, up_w: torch.Tensor, u
                     eps: float = 1e-5, use_workspace: bool = True) -> torch.Tensor:
     """The fp8 MLP block (model/mlp_block.cuh:121-176): out = x + down(relu(up(rmsnorm(x)))^2).
     x, out: [M, hidden] bf16; up_w [inter, hidden], down_w [hidden, inter] e4m3 with per-row
-    float32 scales.  The transient buffers come from torch's allocator, for this call
-    (or, with use_workspace=False, from the library's bump allocator)."""
+    float32 scales.  The transient buffers come from torch's allocator (_workspace; or, with
+    use_workspace=False, from the library's bump allocator)."""
     x2 = _as_2d(x)
     if not x2.is_contiguous():
         raise ValueError("x must be contiguous")
@@ -273,11 +301,14 @@ def mlp_forward_fp8(x: torch.Tensor, norm_w: torch.Tensor, up_w: torch.Tensor, u
     _check_out(out, M, hidden) if x.dim() == 2 else _check_out(out, 1, hidden)
     _check_device(x2, norm_w, up_w, up_s, down_w, down_s, out)
     L = _lib.lib()
-    ws = _workspace(x.device, L.nmi_mlp_workspace_bytes(M, hidden, inter)) if use_workspace else None
+    st = _stream()
+    need = L.nmi_mlp_workspace_bytes(M, hidden, inter) if use_workspace else 0
+    ws, key = _workspace(x.device, need, st)
     rc = L.nmi_mlp_forward_fp8(x2.data_ptr(), norm_w.data_ptr(), up_w.data_ptr(), up_s.data_ptr(),
                                down_w.data_ptr(), down_s.data_ptr(), out.data_ptr(), M, hidden, inter, eps,
-                               None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
-                               _stream())
+                               None if ws is None else ws.data_ptr(), need, st)
+    if key is not None:
+        _kept[key] = ws
     _lib.check(rc, "nmi_mlp_forward_fp8")
     return out
 
@@ -317,10 +348,13 @@ def sdpa_decode_bf16(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     _check_device(q, k_cache, v_cache, k_new, v_new, out)
     L = _lib.lib()
     need = L.nmi_sdpa_decode_workspace_bytes(H, n_kv, S_cache)
-    ws = _workspace(q.device, need)
+    st = _stream()
+    ws, key = _workspace(q.device, need, st)
     rc = L.nmi_sdpa_decode_bf16(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
                                 k_new.data_ptr(), v_new.data_ptr(), S_cache, cap, H, n_kv,
-                                None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _stream())
+                                None if ws is None else ws.data_ptr(), need, st)
+    if key is not None:
+        _kept[key] = ws
     _lib.check(rc, "nmi_sdpa_decode_bf16")
     return out
 
@@ -360,14 +394,15 @@ def attn_decode_fp8(x: torch.Tensor, norm_w: torch.Tensor, q_w, q_s, k_w, k_s, v
     _check_out(out, 1, hidden)
     _check_device(x2, norm_w, q_w, q_s, k_w, k_s, v_w, v_s, o_w, o_s, k_cache, v_cache, out)
     L = _lib.lib()
-    ws = None
-    if use_workspace:
-        ws = _workspace(x.device, L.nmi_attn_decode_workspace_bytes(hidden, H, n_kv, S_cache))
+    st = _stream()
+    need = L.nmi_attn_decode_workspace_bytes(hidden, H, n_kv, S_cache) if use_workspace else 0
+    ws, key = _workspace(x.device, need, st)
     rc = L.nmi_attn_decode_fp8(x2.data_ptr(), norm_w.data_ptr(), q_w.data_ptr(), q_s.data_ptr(), k_w.data_ptr(),
                                k_s.data_ptr(), v_w.data_ptr(), v_s.data_ptr(), o_w.data_ptr(), o_s.data_ptr(),
                                k_cache.data_ptr(), v_cache.data_ptr(), S_cache, cap, out.data_ptr(), hidden, H, n_kv,
-                               eps, None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
-                               _stream())
+                               eps, None if ws is None else ws.data_ptr(), need, st)
+    if key is not None:
+        _kept[key] = ws
     _lib.check(rc, "nmi_attn_decode_fp8")
     return out
 
@@ -393,11 +428,13 @@ def sdpa_prefill_bf16(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, n_heads
     _check_device(q, k, v, out)
     L = _lib.lib()
     need = L.nmi_sdpa_prefill_workspace_bytes(n_kv_heads, S)     # 0: the kernel reads q, k, v in place
-    ws = _workspace(q.device, need)
+    st = _stream()
+    ws, key = _workspace(q.device, need, st)
     rc = L.nmi_sdpa_prefill_bf16(q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
                                  out.data_ptr(), out.stride(0), S, n_heads, n_kv_heads,
-                                 ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0,
-                                 _stream())
+                                 None if ws is None else ws.data_ptr(), need, st)
+    if key is not None:
+        _kept[key] = ws
     _lib.check(rc, "nmi_sdpa_prefill_bf16")
     return out
 
@@ -439,12 +476,16 @@ def attn_forward_fp8(x: torch.Tensor, norm_w: torch.Tensor, q_w, q_s, k_w, k_s, 
     _check_out(out, S, hidden) if x.dim() == 2 else _check_out(out, 1, hidden)
     _check_device(x2, norm_w, q_w, q_s, k_w, k_s, v_w, v_s, o_w, o_s, out)
     L = _lib.lib()
-    ws = _workspace(x.device, L.nmi_attn_forward_workspace_bytes(S, hidden, H, n_kv)) if use_workspace else None
+    st = _stream()
+    need = L.nmi_attn_forward_workspace_bytes(S, hidden, H, n_kv) if use_workspace else 0
+    ws, key = _workspace(x.device, need, st)
     rc = L.nmi_attn_forward_fp8(x2.data_ptr(), norm_w.data_ptr(), q_w.data_ptr(), q_s.data_ptr(), k_w.data_ptr(),
                                 k_s.data_ptr(), v_w.data_ptr(), v_s.data_ptr(), o_w.data_ptr(), o_s.data_ptr(),
                                 out.data_ptr(), S, None if k_cache is None else k_cache.data_ptr(),
                                 None if v_cache is None else v_cache.data_ptr(), cap, hidden, H, n_kv, eps,
-                                None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _stream())
+                                None if ws is None else ws.data_ptr(), need, st)
+    if key is not None:
+        _kept[key] = ws
     _lib.check(rc, "nmi_attn_forward_fp8")
     return out
 
@@ -520,14 +561,18 @@ def mamba_decode_fp8(x: torch.Tensor, norm_w: torch.Tensor, in_w, in_s, conv_w, 
     _check_device(x2, norm_w, in_w, in_s, conv_w, conv_b, A_log, D, dt_bias, gnorm_w, out_w, out_s, conv_state,
                   ssm_state, out)
     L = _lib.lib()
-    ws = None
+    st = _stream()
+    need = 0
     if use_workspace:
-        ws = _workspace(x.device, L.nmi_mamba_decode_workspace_bytes(batch, hidden, n_heads, head_dim, n_groups, 128))
+        need = L.nmi_mamba_decode_workspace_bytes(batch, hidden, n_heads, head_dim, n_groups, 128)
+    ws, key = _workspace(x.device, need, st)
     rc = L.nmi_mamba_decode_fp8(x2.data_ptr(), norm_w.data_ptr(), in_w.data_ptr(), in_s.data_ptr(), conv_w.data_ptr(),
                                 conv_b.data_ptr(), A_log.data_ptr(), D.data_ptr(), dt_bias.data_ptr(),
                                 gnorm_w.data_ptr(), out_w.data_ptr(), out_s.data_ptr(), conv_state.data_ptr(),
                                 ssm_state.data_ptr(), out.data_ptr(), batch, hidden, n_heads, head_dim, n_groups, 128, 4,
-                                eps, None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _stream())
+                                eps, None if ws is None else ws.data_ptr(), need, st)
+    if key is not None:
+        _kept[key] = ws
     _lib.check(rc, "nmi_mamba_decode_fp8")
     return out
 
@@ -572,17 +617,19 @@ def mamba_forward_fp8(x: torch.Tensor, norm_w: torch.Tensor, in_w, in_s, conv_w,
     _check_out(out, M, hidden) if x.dim() == 2 else _check_out(out, 1, hidden)
     _check_device(x2, norm_w, in_w, in_s, conv_w, conv_b, A_log, D, dt_bias, gnorm_w, out_w, out_s, out)
     L = _lib.lib()
-    ws = None
+    st = _stream()
+    need = 0
     if use_workspace:
-        ws = _workspace(x.device, L.nmi_mamba_forward_workspace_bytes(batch, S, hidden, n_heads, head_dim, n_groups,
-                                                                     128))
+        need = L.nmi_mamba_forward_workspace_bytes(batch, S, hidden, n_heads, head_dim, n_groups, 128)
+    ws, key = _workspace(x.device, need, st)
     rc = L.nmi_mamba_forward_fp8(x2.data_ptr(), norm_w.data_ptr(), in_w.data_ptr(), in_s.data_ptr(), conv_w.data_ptr(),
                                  conv_b.data_ptr(), A_log.data_ptr(), D.data_ptr(), dt_bias.data_ptr(),
                                  gnorm_w.data_ptr(), out_w.data_ptr(), out_s.data_ptr(), out.data_ptr(), batch, S,
                                  None if conv_state_out is None else conv_state_out.data_ptr(),
                                  None if ssm_state_out is None else ssm_state_out.data_ptr(), hidden, n_heads, head_dim,
-                                 n_groups, 128, 4, eps, None if ws is None else ws.data_ptr(),
-                                 0 if ws is None else ws.numel(), _stream())
+                                 n_groups, 128, 4, eps, None if ws is None else ws.data_ptr(), need, st)
+    if key is not None:
+        _kept[key] = ws
     _lib.check(rc, "nmi_mamba_forward_fp8")
     return out
 

@@ -1,7 +1,8 @@
 """Where the torch front end's transient device memory comes from (nemotron_infer_amd/ops.py), no GPU
-needed: each call takes its own from torch's allocator and keeps none of it.  Memory kept between
-calls would be shared by every stream and thread, and a HIP graph captured with it would go on
-writing into it after a larger call had replaced it.  The library is replaced by a recorder."""
+needed.  Memory shared by streams or threads would be overwritten by the other's call, and a HIP
+graph captured with memory that a larger call replaces would go on writing into it: so what is kept
+between calls is kept per stream, out of reach while a call has it, and never under capture.  The
+library is replaced by a recorder."""
 import ctypes
 import weakref
 
@@ -10,45 +11,55 @@ import torch
 
 from nemotron_infer_amd import _lib, ops
 
-NEED = 1_200_000
+SMALL, LARGE = 1_200_000, ops._KEEP_BYTES + 512
 FLAGS = _lib.NMI_WS_ERROR_OFFSET + 4
 
 
 class Recorder:
-    """Stands in for libnmi.so: every workspace is NEED bytes; launches note their arguments and the
-    first bytes of the workspace they were given."""
+    """Stands in for libnmi.so: every workspace is `need` bytes; launches note the workspace they were
+    given and its first bytes, and call `during`."""
 
-    def __init__(self, needs_zero=0):
-        self.needs_zero, self.launches = needs_zero, []
+    def __init__(self, need=SMALL, needs_zero=0):
+        self.need, self.needs_zero, self.launches, self.during = need, needs_zero, [], None
 
     def __getattr__(self, name):
         if name.endswith("workspace_bytes"):
-            return lambda *a: NEED
+            return lambda *a: self.need
         if name == "nmi_linear_workspace_needs_zero":
             return lambda M: self.needs_zero
 
         def launch(*args):
-            at = next(i for i in range(len(args) - 1) if args[i + 1] == NEED)
+            at = next(i for i in range(len(args) - 1) if args[i + 1] == self.need)
             self.launches.append((name, args[at], ctypes.string_at(args[at], FLAGS + 16)))
+            during, self.during = self.during, None
+            if during:
+                during()
             return _lib.NMI_OK
         return launch
 
 
 @pytest.fixture
-def made(monkeypatch):
-    """The uint8 tensors torch.empty makes (weak), filled with 255."""
-    refs, empty = [], torch.empty
+def env(monkeypatch):
+    """The uint8 tensors torch.empty makes (weak, filled with 255), and the stream and capture state
+    that the front end sees."""
+    class Env:
+        made, stream, capturing, lib = [], 0, False, Recorder()
+    e, empty = Env(), torch.empty
+    e.made = []
 
     def spy(*a, **kw):
         t = empty(*a, **kw)
         if t.dtype == torch.uint8:
             t.fill_(255)
-            refs.append((weakref.ref(t), t.data_ptr()))
+            e.made.append((weakref.ref(t), t.data_ptr()))
         return t
     monkeypatch.setattr(torch, "empty", spy)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: e.capturing)
     monkeypatch.setattr(ops, "_check_device", lambda *ts: None)
-    monkeypatch.setattr(ops, "_stream", lambda: 0)
-    return refs
+    monkeypatch.setattr(ops, "_stream", lambda: e.stream)
+    monkeypatch.setattr(ops, "_kept", {})
+    monkeypatch.setattr(_lib, "lib", lambda: e.lib)
+    return e
 
 
 def _bf(*shape):
@@ -81,24 +92,53 @@ CALLS = {
 
 
 @pytest.mark.parametrize("call", CALLS)
-def test_workspaces_belong_to_one_call(call, made, monkeypatch):
-    lib = Recorder()
-    monkeypatch.setattr(_lib, "lib", lambda: lib)
+@pytest.mark.parametrize("need,capturing", [(LARGE, False), (SMALL, True)])
+def test_large_and_captured_memory_belongs_to_one_call(call, need, capturing, env):
+    env.lib, env.capturing = Recorder(need), capturing
     for n in (1, 2):
-        before = len(made)
-        out = CALLS[call]()
-        assert out is not None and len(lib.launches) == n
-        mine = {ptr: ref for ref, ptr in made[before:]}
-        assert lib.launches[-1][1] in mine, "not from torch's allocator in this call"
-        assert mine[lib.launches[-1][1]]() is None, "kept after the call"
+        before = len(env.made)
+        CALLS[call]()
+        assert len(env.lib.launches) == n
+        mine = {ptr: ref for ref, ptr in env.made[before:]}
+        assert env.lib.launches[-1][1] in mine, "not from torch's allocator in this call"
+        assert mine[env.lib.launches[-1][1]]() is None and not ops._kept, "kept after the call"
+
+
+@pytest.mark.parametrize("call", CALLS)
+def test_small_memory_is_kept_for_its_stream_only(call, env):
+    """The same memory for the next call on the stream, other memory on another stream, for a call
+    that begins while one is under way on the same stream (a second thread), and under capture;
+    a larger call replaces what its own stream keeps; every call is told what it asked for."""
+    lib = env.lib
+
+    def run(stream=0):
+        env.stream = stream
+        CALLS[call]()
+        return lib.launches[-1][1]
+
+    first = run()
+    assert run() == first
+    other = run(stream=64)
+    assert other != first and run() == first and run(stream=64) == other
+    lib.during = run                                  # begins before the outer call's launch returns
+    outer = len(lib.launches)
+    run()
+    assert lib.launches[outer][1] == first and lib.launches[outer + 1][1] != first
+    env.capturing = True
+    kept = dict(ops._kept)
+    assert run() not in [t.data_ptr() for t in kept.values()] and ops._kept == kept
+    env.capturing = False
+    lib.need = 3 * SMALL
+    run()
+    assert sorted(ops._kept) == [(None, 0), (None, 64)] and ops._kept[None, 0].numel() == 3 * SMALL
+    assert ops._kept[None, 64].data_ptr() == other
 
 
 @pytest.mark.parametrize("M,needs_zero,zeroed", [(600, 1, True), (600, 0, False), (24, 1, False)])
-def test_only_stream_k_flags_are_cleared(M, needs_zero, zeroed, made, monkeypatch):
+def test_only_stream_k_flags_are_cleared(M, needs_zero, zeroed, env):
     """From M = 512 the flag region starts at zero where the library says so (the stream-K form);
     below, the kernels leave it alone, so it is not cleared on every call."""
-    lib = Recorder(needs_zero)
-    monkeypatch.setattr(_lib, "lib", lambda: lib)
+    env.lib = Recorder(SMALL, needs_zero)
     ops.linear_fp8_w8a16(_bf(M, 64), *_mat(32, 64))
-    head = lib.launches[0][2]
+    head = env.lib.launches[0][2]
     assert head == (b"\0" * FLAGS if zeroed else b"\xff" * FLAGS) + b"\xff" * 16

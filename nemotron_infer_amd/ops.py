@@ -81,8 +81,9 @@ def _check_device(*ts: torch.Tensor) -> None:
 # stream): torch.empty and the release cost a call 2 us of host time, 5-10% of an eager decode call
 # that the host bounds (attention decode over 30 / 65 positions 19.1 / 22.6 us with the memory at hand,
 # 21.2 / 24.0 without; kept 0.3-0.5 us more than at hand).  A call takes the tensor out for its
-# duration, so that a second thread on the stream gets memory of its own.
-_KEEP_BYTES = 32 << 20
+# duration, so that a second thread on the stream gets memory of its own.  (torch has 32 streams a
+# device to give out; a program that makes its own without end keeps memory for the first ones only.)
+_KEEP_BYTES, _KEEP_STREAMS = 32 << 20, 64
 _kept: dict[tuple[int, int], torch.Tensor] = {}
 
 
@@ -100,6 +101,8 @@ def _workspace(device: torch.device, need: int, stream: int):
         ws = _kept.pop(key, None)
         if ws is not None and ws.numel() >= need:
             return ws, key
+        if ws is None and len(_kept) >= _KEEP_STREAMS:
+            key = None
         need = max(need, 1 << 20)
     return torch.empty(need, dtype=torch.uint8, device=device), key
 

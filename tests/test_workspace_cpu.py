@@ -134,6 +134,16 @@ def test_small_memory_is_kept_for_its_stream_only(call, env):
     assert ops._kept[None, 64].data_ptr() == other
 
 
+def test_kept_memory_is_bounded(env):
+    for stream in range(2 * ops._KEEP_STREAMS):
+        env.stream = 64 * stream
+        for need in (SMALL, LARGE, 2 * SMALL):
+            env.lib.need = need
+            ops.linear_fp8_w8a16(_bf(24, 64), *_mat(32, 64))
+    assert len(ops._kept) == ops._KEEP_STREAMS
+    assert all(t.numel() == 2 * SMALL for t in ops._kept.values())
+
+
 @pytest.mark.parametrize("M,needs_zero,zeroed", [(600, 1, True), (600, 0, False), (24, 1, False)])
 def test_only_stream_k_flags_are_cleared(M, needs_zero, zeroed, env):
     """From M = 512 the flag region starts at zero where the library says so (the stream-K form);

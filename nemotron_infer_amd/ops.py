@@ -111,7 +111,7 @@ def _linear_ws(L, device: torch.device, M: int, need: int, stream: int):
     """_workspace() of a linear.  Only the stream-K form (a tuning knob, from M = 512) reads what it
     has not written: its flags, in the first 64 KiB."""
     ws, key = _workspace(device, need, stream)
-    if need and M >= 512 and L.nmi_linear_workspace_needs_zero(M):
+    if M >= 512 and L.nmi_linear_workspace_needs_zero(M):
         ws[:_lib.NMI_WS_ERROR_OFFSET + 4].zero_()
     return ws, key
 
@@ -141,7 +141,7 @@ def linear_fp8_w8a16(x: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
     L = _lib.lib()
     st = _stream()
     need = L.nmi_linear_workspace_bytes(M, N, K) if use_workspace else 0
-    ws, key = _linear_ws(L, x.device, M, need, st)
+    ws, key = _linear_ws(L, x.device, M, need, st) if need else (None, None)
     rc = L.nmi_linear_fp8_w8a16_ws(
         x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0), w_scale.data_ptr(),
         out.data_ptr(), N, M, N, K, None if ws is None else ws.data_ptr(), need, st)
@@ -175,7 +175,7 @@ def linear_fp8_w8a16_grouped(x: torch.Tensor, weights, outs=None, use_workspace:
     total = sum(w.shape[0] for w, _ in weights)
     st = _stream()
     need = L.nmi_linear_workspace_bytes(M, total, K) if use_workspace else 0
-    ws, key = _linear_ws(L, x.device, M, need, st)
+    ws, key = _linear_ws(L, x.device, M, need, st) if need else (None, None)
     rc = L.nmi_linear_fp8_w8a16_grouped(x2.data_ptr(), x2.stride(0), M, K, arr, n,
                                         None if ws is None else ws.data_ptr(), need, st)
     if key is not None:
@@ -251,7 +251,7 @@ def gemm_fp8_w8a16(x: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
     L = _lib.lib()
     st = _stream()
     need = L.nmi_linear_workspace_bytes(M, N, K) if use_workspace else 0
-    ws, key = _linear_ws(L, x.device, M, need, st)
+    ws, key = _linear_ws(L, x.device, M, need, st) if need else (None, None)
     rc = L.nmi_gemm_fp8_w8a16(x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0),
                               w_scale.data_ptr(), out.data_ptr(), N, M, N, K,
                               None if ws is None else ws.data_ptr(), need, st)
